@@ -1437,11 +1437,11 @@ int launch_vsp(hipStream_t s, double *const F[3], int ncomp, const Grid &g, doub
  * k_diag_ring. */
 /* Row of the diagnostics ring of the current step (device step counter
  * *step): the two energy sums of k_energy_part's nparts partials (fixed
- * order) and the three kinetic sums wk[0..2] of the push. */
+ * order) and the three kinetic sums of the push (its slots). */
 struct DiagRingArgs {
     const double *part;
     int           nparts;
-    const double *wk;
+    const double *kin;
     double       *ring;
     int          *step;
     int           cap;
@@ -1450,33 +1450,29 @@ struct DiagRingArgs {
 
 #define RING_TPB 1024
 
-__device__ static inline void diag_ring(const double *part, int nparts, const double *wk,
+__device__ static inline void diag_ring(const double *part, int nparts, const double *kin,
                                         double *ring, int *step, int cap, int tick)
 {
-    __shared__ double se[RING_TPB], sb[RING_TPB];
-    double a = 0, c = 0;
+    __shared__ double sw[5][RING_TPB / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    double v[5] = {0, 0, 0, 0, 0};
+    if (threadIdx.x < KIN_SLOTS)
+        for (int a = 0; a < 3; ++a) v[2 + a] = kin[KIN_STRIDE * threadIdx.x + a];
     for (int q = threadIdx.x; q < nparts; q += RING_TPB) {
-        a += part[2 * q];
-        c += part[2 * q + 1];
+        v[0] += part[2 * q];
+        v[1] += part[2 * q + 1];
     }
-    se[threadIdx.x] = a;
-    sb[threadIdx.x] = c;
+    for (int a = 0; a < 5; ++a) {
+        for (int d = 32; d > 0; d >>= 1) v[a] += __shfl_down(v[a], d, 64);
+        if (lane == 0) sw[a][w] = v[a];
+    }
     __syncthreads();
-    for (int w = RING_TPB / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            se[threadIdx.x] += se[threadIdx.x + w];
-            sb[threadIdx.x] += sb[threadIdx.x + w];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        double *row = ring + 5 * (long)(*step % cap);
-        row[0] = se[0];
-        row[1] = sb[0];
-        row[2] = wk[0];
-        row[3] = wk[1];
-        row[4] = wk[2];
-        if (tick) *step += 1;
+    if (threadIdx.x < 5) {
+        double s = 0;
+        for (int q = 0; q < RING_TPB / 64; ++q) s += sw[threadIdx.x][q];
+        const int st = *step;
+        ring[5 * (long)(st % cap) + threadIdx.x] = s;
+        if (tick && threadIdx.x == 0) *step = st + 1;   /* one wavefront: read before written */
     }
 }
 
@@ -1484,14 +1480,14 @@ template <> struct KernelDef<DiagRingArgs> {
     static constexpr int kBlock = RING_TPB;
     __device__ __forceinline__ static void body(const DiagRingArgs &a, VBlock, VBlock)
     {
-        diag_ring(a.part, a.nparts, a.wk, a.ring, a.step, a.cap, a.tick);
+        diag_ring(a.part, a.nparts, a.kin, a.ring, a.step, a.cap, a.tick);
     }
 };
 
-int launch_diag_ring(hipStream_t s, const double *part, int nparts, const double *wk,
+int launch_diag_ring(hipStream_t s, const double *part, int nparts, const double *kin,
                      double *ring, int *step, int cap, int tick)
 {
-    DiagRingArgs a = {part, nparts, wk, ring, step, cap, tick};
+    DiagRingArgs a = {part, nparts, kin, ring, step, cap, tick};
     return launch_def(s, a, 1);
 }
 
@@ -1511,7 +1507,7 @@ int launch_zero(hipStream_t s, double *p, long n)
 }
 
 /* J cleared before the push, only on the x planes the previous step's
- * deposit can have written, and the three temperature sums.
+ * deposit can have written, and the push's kinetic sums.
  *
  * A tiled push deposits the markers of the active tiles only (the list is
  * in tile order, tiles i-major), each into nodes [4u-1, 4u+5] along x of
@@ -1529,7 +1525,7 @@ struct JClearArgs {
     double       *J;          /* 3 components, ncell apart */
     long          ncell, plane;
     int           n0, tpp;    /* cells along x, tiles per x layer of tiles */
-    double       *acc;        /* 3 sums */
+    double       *kin;        /* the push's kinetic sums */
     int          *range;      /* [2][2] plane ranges by step parity, [2] this step's */
     const int    *step, *active, *nactive;
     int           full;
@@ -1543,10 +1539,9 @@ __device__ static inline void jclear(const JClearArgs &a, const VBlock &b, const
         lo = a.range[2 * (s & 1)];
         hi = a.range[2 * (s & 1) + 1];
     }
+    if (b.x == 0)
+        for (int q = threadIdx.x; q < KIN_SLOTS * KIN_STRIDE; q += TPB) a.kin[q] = 0.0;
     if (b.x == 0 && threadIdx.x == 0) {
-        a.acc[0] = 0.0;
-        a.acc[1] = 0.0;
-        a.acc[2] = 0.0;
         int nlo = -2, nhi = a.n0 + 2;
         if (!a.full) {
             const int na = *a.nactive;
@@ -1587,10 +1582,10 @@ template <> struct KernelDef<JClearArgs> {
     }
 };
 
-static JClearArgs jclear_args(double *J, const Grid &g, double *acc, int *range, const int *step,
+static JClearArgs jclear_args(double *J, const Grid &g, double *kin, int *range, const int *step,
                               const int *active, const int *nactive, int tpp, int full)
 {
-    JClearArgs a = {J, g.ncell, (long)g.GY * g.GZ, g.n[0], tpp, acc, range, step, active,
+    JClearArgs a = {J, g.ncell, (long)g.GY * g.GZ, g.n[0], tpp, kin, range, step, active,
                     nactive, full};
     return a;
 }
@@ -1606,10 +1601,10 @@ static unsigned jclear_blocks(const Grid &g)
     return (unsigned)nb;
 }
 
-int launch_jclear(hipStream_t s, double *J, const Grid &g, double *acc, int *range,
+int launch_jclear(hipStream_t s, double *J, const Grid &g, double *kin, int *range,
                   const int *step, const int *active, const int *nactive, int tpp, int full)
 {
-    return launch_def(s, jclear_args(J, g, acc, range, step, active, nactive, tpp, full),
+    return launch_def(s, jclear_args(J, g, kin, range, step, active, nactive, tpp, full),
                       jclear_blocks(g));
 }
 
@@ -1777,13 +1772,13 @@ int launch_probes(hipStream_t s, T *const E[3], T *const H[3], const Grid &g, co
  * x folds have run before). */
 template <class T>
 int launch_h_update_jclear(hipStream_t s, const FieldsT<T> &f, const Grid &g, const BoxSet &flush,
-                           int full, double *part, double *J, double *acc, int *range,
+                           int full, double *part, double *J, double *kin, int *range,
                            const int *step, const int *active, const int *nactive, int tpp,
                            int jfull)
 {
     const HUpdateArgs<T> a = h_args(f, g, flush, full, part, LaserPlane());
     return launch_pair(s, a, dim3(grid_span(a.sp, g.n[0] + 2)),
-                       jclear_args(J, g, acc, range, step, active, nactive, tpp, jfull),
+                       jclear_args(J, g, kin, range, step, active, nactive, tpp, jfull),
                        dim3(jclear_blocks(g)));
 }
 

@@ -100,6 +100,21 @@ struct JPtrs {
     double *J[3];
 };
 
+/* The push's kinetic sums (W p_a^2, a = x, y, z) are kept as KIN_SLOTS
+ * partial sums, three doubles each, KIN_STRIDE apart: every wavefront (or
+ * workgroup) of the push adds its own with three FP64 atomics, and atomics to
+ * one address are served one after the other (about 11 ns each across the
+ * XCDs), so the wavefronts are spread over the slots by block index.  The
+ * J clear zeroes them; the ring kernel and mpic_temperature add them up in
+ * slot order. */
+#define KIN_SLOTS 256
+#define KIN_STRIDE 4
+
+__device__ static inline double *kin_slot(double *kin, unsigned block)
+{
+    return kin + KIN_STRIDE * (block % KIN_SLOTS);
+}
+
 struct Markers64 {
     double  *x, *y, *z, *ux, *uy, *uz;
     float   *w, *qm;
@@ -163,7 +178,7 @@ int launch_face_pair(hipStream_t s, const Grid &g, const FaceOp &a, const FaceOp
 int launch_face_planes(hipStream_t s, const Grid &g, const FaceOp *ops, int nop);
 template <class T>
 int launch_h_update_jclear(hipStream_t s, const FieldsT<T> &f, const Grid &g, const BoxSet &flush,
-                           int full, double *part, double *J, double *acc, int *range,
+                           int full, double *part, double *J, double *kin, int *range,
                            const int *step, const int *active, const int *nactive, int tpp,
                            int jfull);
 template <class T>
@@ -212,14 +227,14 @@ template <class T> int launch_energy(hipStream_t s, const FieldsT<T> &f, const G
  * 'part'; the ring row {W_E sum, W_M sum, WTx, WTy, WTz} of the device step
  * counter's step sums them, and with 'tick' advances the counter. */
 int h_update_blocks(const Grid &g, int fp32);
-int launch_diag_ring(hipStream_t s, const double *part, int nparts, const double *wk,
+int launch_diag_ring(hipStream_t s, const double *part, int nparts, const double *kin,
                      double *ring, int *step, int cap, int tick);
 int launch_zero(hipStream_t s, double *p, long n);
-int launch_jclear(hipStream_t s, double *J, const Grid &g, double *acc, int *range,
+int launch_jclear(hipStream_t s, double *J, const Grid &g, double *kin, int *range,
                   const int *step, const int *active, const int *nactive, int tpp, int full);
 
 int launch_push64(hipStream_t s, const Markers64 &m, long n, const Fields64 &f,
-                  const Grid &g, const PushConsts &c, double *Wacc, int mode, unsigned *err);
+                  const Grid &g, const PushConsts &c, double *kin, int mode, unsigned *err);
 int launch_rho64(hipStream_t s, const Markers64 &m, long n, double *rho,
                  const Grid &g, const int *perm, const int *nmark, int parity);
 int launch_rho_fold(hipStream_t s, double *rho, const Grid &g, int b, int bc);

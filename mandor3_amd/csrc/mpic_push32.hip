@@ -494,13 +494,13 @@ struct Push32Args {
     Push32Consts c;
     TileView     tv;
     float       *tj;
-    double      *Wacc;
+    double      *kin;
 };
 
 template <int W>
 __device__ __forceinline__ static void push32_tiles(const Markers32 &m, const Markers32 &d,
                                            const F32View &v, const Push32Consts &c,
-                                           const TileView &tv, float *tj, double *Wacc,
+                                           const TileView &tv, float *tj, double *kin,
                                            const VBlock &bk, const VBlock &gd)
 {
     constexpr int BS = TW * W;                       /* threads of the workgroup */
@@ -628,9 +628,10 @@ __device__ __forceinline__ static void push32_tiles(const Markers32 &m, const Ma
         d2 += __shfl_down(d2, d, 64);
     }
     if (lane == 0 && (d0 != 0.0 || d1 != 0.0 || d2 != 0.0)) {
-        atomicAdd(Wacc + 0, d0 * c.vol);
-        atomicAdd(Wacc + 1, d1 * c.vol);
-        atomicAdd(Wacc + 2, d2 * c.vol);
+        double *ks = kin_slot(kin, bk.x);
+        atomicAdd(ks + 0, d0 * c.vol);
+        atomicAdd(ks + 1, d1 * c.vol);
+        atomicAdd(ks + 2, d2 * c.vol);
     }
 }
 
@@ -645,7 +646,7 @@ template <int W> struct KernelDef<Push32ArgsW<W>> {
     static constexpr int kWaves = 4;
     __device__ __forceinline__ static void body(const Push32ArgsW<W> &a, VBlock b, VBlock gd)
     {
-        push32_tiles<W>(a.m, a.d, a.v, a.c, a.tv, a.tj, a.Wacc, b, gd);
+        push32_tiles<W>(a.m, a.d, a.v, a.c, a.tv, a.tj, a.kin, b, gd);
     }
 };
 
@@ -768,7 +769,7 @@ template <> struct KernelDef<JGatherArgs> {
 
 int launch_push32(hipStream_t s, const Markers32 &m, const Markers32 &dst, const Fields32 &f,
                   const Grid &g, const PushConsts &pc, const float *qm, const TileView &tv,
-                  float *tj, double *Wacc, int nblocks, int waves)
+                  float *tj, double *kin, int nblocks, int waves)
 {
     F32View v;
     for (int a = 0; a < 3; ++a) {
@@ -786,7 +787,7 @@ int launch_push32(hipStream_t s, const Markers32 &m, const Markers32 &dst, const
     c.vol = g.h[0] * g.h[1] * g.h[2];
     for (int q = 0; q < 4; ++q) c.qm[q] = qm[q];
     for (int b = 0; b < 6; ++b) c.bc[b] = pc.bc[b];
-    const Push32Args a = {m, dst, v, c, tv, tj, Wacc};
+    const Push32Args a = {m, dst, v, c, tv, tj, kin};
     switch (waves) {
     case 1: return launch_def(s, Push32ArgsW<1>{a}, (unsigned)nblocks);
     case 2: return launch_def(s, Push32ArgsW<2>{a}, (unsigned)nblocks);

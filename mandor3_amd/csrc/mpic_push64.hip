@@ -335,7 +335,7 @@ __device__ static int push_marker(const S &sink, const F64View &v, const PushCon
     return walls(c, r, u);
 }
 
-__device__ static void block_sum3(double w3[3], double *Wacc)
+__device__ static void block_sum3(double w3[3], double *ks)
 {
     __shared__ double sw[3][TPB];
     sw[0][threadIdx.x] = w3[0];
@@ -351,9 +351,9 @@ __device__ static void block_sum3(double w3[3], double *Wacc)
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        atomicAdd(Wacc + 0, sw[0][0]);
-        atomicAdd(Wacc + 1, sw[1][0]);
-        atomicAdd(Wacc + 2, sw[2][0]);
+        atomicAdd(ks + 0, sw[0][0]);
+        atomicAdd(ks + 1, sw[1][0]);
+        atomicAdd(ks + 2, sw[2][0]);
     }
 }
 
@@ -366,13 +366,13 @@ struct Push64Args {
     long       n;
     F64View    v;
     PushConsts c;
-    double    *Wacc;
+    double    *kin;
     int        mode;
     unsigned  *err;
 };
 
 __device__ __forceinline__ static void push64(const Markers64 &m, long n, const F64View &v,
-                                     const PushConsts &c, double *Wacc, int mode, unsigned *err,
+                                     const PushConsts &c, double *kin, int mode, unsigned *err,
                                      long p)
 {
     double w3[3] = {0, 0, 0};
@@ -397,19 +397,19 @@ __device__ __forceinline__ static void push64(const Markers64 &m, long n, const 
         }
     }
     if (mode != 0) return;
-    block_sum3(w3, Wacc);
+    block_sum3(w3, kin_slot(kin, (unsigned)(p / TPB)));
 }
 
 template <> struct KernelDef<Push64Args> {
     static constexpr int kBlock = TPB;
     __device__ __forceinline__ static void body(const Push64Args &a, VBlock b, VBlock)
     {
-        push64(a.m, a.n, a.v, a.c, a.Wacc, a.mode, a.err, (long)b.x * TPB + threadIdx.x);
+        push64(a.m, a.n, a.v, a.c, a.kin, a.mode, a.err, (long)b.x * TPB + threadIdx.x);
     }
 };
 
 int launch_push64(hipStream_t s, const Markers64 &m, long n, const Fields64 &f, const Grid &g,
-                  const PushConsts &c, double *Wacc, int mode, unsigned *err)
+                  const PushConsts &c, double *kin, int mode, unsigned *err)
 {
     if (n <= 0) return MPIC_OK;
     F64View v;
@@ -419,7 +419,7 @@ int launch_push64(hipStream_t s, const Markers64 &m, long n, const Fields64 &f, 
         v.J[a] = f.J[a];
     }
     v.g = g;
-    Push64Args a = {m, n, v, c, Wacc, mode, err};
+    Push64Args a = {m, n, v, c, kin, mode, err};
     return launch_def(s, a, (unsigned)((n + TPB - 1) / TPB));
 }
 
@@ -488,13 +488,13 @@ struct Push64TArgs {
     F64View    v;
     PushConsts c;
     TileView   tv;
-    double    *Wacc;
+    double    *kin;
     unsigned  *err;
 };
 
 __device__ __forceinline__ static void push64_tiled(const Markers64 &m, const Markers64 &d,
                                            const F64View &v, const PushConsts &c,
-                                           const TileView &tv, double *Wacc, unsigned *err,
+                                           const TileView &tv, double *kin, unsigned *err,
                                            const VBlock &bk)
 {
     __shared__ double lj[TJN * TJN * TJN * 3];
@@ -569,7 +569,7 @@ __device__ __forceinline__ static void push64_tiled(const Markers64 &m, const Ma
         }
         __syncthreads();
     }
-    block_sum3(w3, Wacc);
+    block_sum3(w3, kin_slot(kin, bk.x));
 }
 
 template <> struct KernelDef<Push64TArgs> {
@@ -577,7 +577,7 @@ template <> struct KernelDef<Push64TArgs> {
     static constexpr int kWaves = 3;   /* register budget for 3 wavefronts per SIMD */
     __device__ __forceinline__ static void body(const Push64TArgs &a, VBlock b, VBlock)
     {
-        push64_tiled(a.m, a.d, a.v, a.c, a.tv, a.Wacc, a.err, b);
+        push64_tiled(a.m, a.d, a.v, a.c, a.tv, a.kin, a.err, b);
     }
 };
 
@@ -594,7 +594,7 @@ int push64_blocks_per_cu(void)
 
 int launch_push64_tiled(hipStream_t s, const Markers64 &m, const Markers64 &dst,
                         const Fields64 &f, const Grid &g, const PushConsts &c,
-                        const TileView &tv, double *Wacc, unsigned *err, int nblocks)
+                        const TileView &tv, double *kin, unsigned *err, int nblocks)
 {
     F64View v;
     for (int a = 0; a < 3; ++a) {
@@ -603,7 +603,7 @@ int launch_push64_tiled(hipStream_t s, const Markers64 &m, const Markers64 &dst,
         v.J[a] = f.J[a];
     }
     v.g = g;
-    Push64TArgs a = {m, dst, v, c, tv, Wacc, err};
+    Push64TArgs a = {m, dst, v, c, tv, kin, err};
     return launch_def(s, a, (unsigned)nblocks);
 }
 

@@ -140,8 +140,10 @@ struct mpic_run {
     std::vector<double *> murbuf;
     std::vector<Laser> lasers;
     PushConsts    pc;
-    double       *dacc;       /* device scratch: [0..1] energy, [2..4] W, [5..6] gauss */
+    double       *dacc;       /* device scratch: [0..1] energy, [5..6] gauss */
     double       *hacc;       /* pinned host mirror */
+    double       *dkin;       /* the push's kinetic sums: KIN_SLOTS partial sums */
+    double       *hkin;       /* pinned host mirror */
     unsigned     *derr;       /* device error flags (bit 0: marker off the grid, bit 1: a
                                  tile scan's wait for an earlier workgroup ran out) */
     int           stage;
@@ -565,6 +567,10 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     r->n = 0;
     MPIC_CHECK(hipMalloc(&r->dacc, sizeof(double) * 8));
     MPIC_CHECK(hipHostMalloc(&r->hacc, sizeof(double) * 8, hipHostMallocDefault));
+    MPIC_CHECK(hipMalloc(&r->dkin, sizeof(double) * KIN_SLOTS * KIN_STRIDE));
+    MPIC_CHECK(hipHostMalloc(&r->hkin, sizeof(double) * KIN_SLOTS * KIN_STRIDE,
+                             hipHostMallocDefault));
+    MPIC_CHECK(hipMemsetAsync(r->dkin, 0, sizeof(double) * KIN_SLOTS * KIN_STRIDE, r->stream));
     MPIC_CHECK(hipMalloc(&r->derr, sizeof(unsigned)));
     MPIC_CHECK(hipMemsetAsync(r->derr, 0, sizeof(unsigned), r->stream));
     r->timed = -1;
@@ -637,6 +643,8 @@ extern "C" int mpic_destroy(mpic_run_t *r)
     hipFree(r->tv.item); hipFree(r->tv.istart);
     hipFree(r->tj);
     hipFree(r->dacc);
+    hipFree(r->dkin);
+    if (r->hkin) hipHostFree(r->hkin);
     hipFree(r->derr);
     if (r->hacc) hipHostFree(r->hacc);
     for (double *b : r->murbuf) hipFree(b);
@@ -1562,7 +1570,7 @@ extern "C" int mpic_init(mpic_run_t *r)
         TRY(init_ghosts(r, r->f.E, r->f.H));
     /* plasma_init: walls applied once to every loaded marker
      * (source/core/plasma.c:409-414). */
-    if (!r->fp32) TRY(launch_push64(r->stream, r->m, r->n, r->f, g, r->pc, r->dacc, 1, r->derr));
+    if (!r->fp32) TRY(launch_push64(r->stream, r->m, r->n, r->f, g, r->pc, r->dkin, 1, r->derr));
     if (r->tiled) {
         /* first sort of the loaded markers by tile-major cell key */
         const int nn = (int)r->n;
@@ -1807,7 +1815,7 @@ static int h_half(mpic_run *r, double *part, bool with_clear)
     TRY(walls_on(r, r->bcE));
     /* em_HSmallStep + cap_flushHalfH */
     if (with_clear) {
-        FCALL(launch_h_update_jclear, r->g, r->flH, 0, part, r->jp.J[0], r->dacc + 2, r->djr,
+        FCALL(launch_h_update_jclear, r->g, r->flH, 0, part, r->jp.J[0], r->dkin, r->djr,
               r->dstep, r->tiled ? r->tv.active : nullptr, r->tiled ? r->tv.nactive : nullptr,
               r->tiled ? r->tv.nt[1] * r->tv.nt[2] : 1, r->tiled ? 0 : 1);
         r->jclear_done = 1;
@@ -1848,23 +1856,23 @@ extern "C" int mpic_push_deposit(mpic_run_t *r)
      * kernel, not a memset (the step may be replayed from a graph), unless
      * the H half step's launch cleared them */
     if (!r->jclear_done)
-        TRY(launch_jclear(r->stream, r->jp.J[0], r->g, r->dacc + 2, r->djr, r->dstep,
+        TRY(launch_jclear(r->stream, r->jp.J[0], r->g, r->dkin, r->djr, r->dstep,
                           r->tiled ? r->tv.active : nullptr, r->tiled ? r->tv.nactive : nullptr,
                           r->tiled ? r->tv.nt[1] * r->tv.nt[2] : 1, r->tiled ? 0 : 1));
     r->jclear_done = 0;
     if (r->timed >= 0) TRY(record(r, 1));
     if (r->fp32) {
         TRY(launch_push32(r->stream, r->m32, r->m32buf[r->cur ^ 1], r->f32, r->g, r->pc, r->qm,
-                          r->tv, r->tj, r->dacc + 2,
+                          r->tv, r->tj, r->dkin,
                           r->tile_blocks, r->tile_waves));
         if (r->timed >= 0) TRY(record(r, 2));
         TRY(launch_jgather32(r->stream, r->f32, r->g, r->tv, r->tj, r->gather_blocks));
     } else if (r->tiled) {
         TRY(launch_push64_tiled(r->stream, r->m, r->mbuf[r->cur ^ 1], r->f, r->g, r->pc, r->tv,
-                                r->dacc + 2, r->derr,
+                                r->dkin, r->derr,
                                 r->push_blocks));
     } else {
-        TRY(launch_push64(r->stream, r->m, r->n, r->f, r->g, r->pc, r->dacc + 2, 0, r->derr));
+        TRY(launch_push64(r->stream, r->m, r->n, r->f, r->g, r->pc, r->dkin, 0, r->derr));
     }
     if (r->timed >= 0) {
         if (!r->fp32) TRY(record(r, 2));
@@ -1879,12 +1887,15 @@ extern "C" int mpic_temperature(mpic_run_t *r, double *WTx, double *WTy, double 
 {
     if (!r) return MPIC_ERR_ARG;
     MPIC_CHECK(hipSetDevice(r->dev));
-    MPIC_CHECK(hipMemcpyAsync(r->hacc + 2, r->dacc + 2, 3 * sizeof(double), hipMemcpyDeviceToHost,
-                              r->stream));
+    MPIC_CHECK(hipMemcpyAsync(r->hkin, r->dkin, sizeof(double) * KIN_SLOTS * KIN_STRIDE,
+                              hipMemcpyDeviceToHost, r->stream));
     MPIC_CHECK(hipStreamSynchronize(r->stream));
-    if (WTx) *WTx = r->hacc[2];
-    if (WTy) *WTy = r->hacc[3];
-    if (WTz) *WTz = r->hacc[4];
+    double w[3] = {0, 0, 0};
+    for (int q = 0; q < KIN_SLOTS; ++q)
+        for (int a = 0; a < 3; ++a) w[a] += r->hkin[KIN_STRIDE * q + a];
+    if (WTx) *WTx = w[0];
+    if (WTy) *WTy = w[1];
+    if (WTz) *WTz = w[2];
     return MPIC_OK;
 }
 
@@ -2082,7 +2093,7 @@ static int step_body(mpic_run *r)
     }
     TRY(e_spot(r));
     /* the ring row of this step, then the device step counter advances */
-    TRY(launch_diag_ring(r->stream, r->dpart, r->nparts, r->dacc + 2, r->dring, r->dstep,
+    TRY(launch_diag_ring(r->stream, r->dpart, r->nparts, r->dkin, r->dring, r->dstep,
                          DIAG_RING, 1));
     step_done(r);
     return MPIC_OK;

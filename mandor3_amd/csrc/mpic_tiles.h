@@ -128,7 +128,7 @@ int launch_scatter64(hipStream_t s, const Markers64 &src, const Markers64 &dst, 
                      const TileView &tv, int parity);
 int launch_push64_tiled(hipStream_t s, const Markers64 &m, const Markers64 &dst,
                         const Fields64 &f, const Grid &g, const PushConsts &c,
-                        const TileView &tv, double *Wacc, unsigned *err, int nblocks);
+                        const TileView &tv, double *kin, unsigned *err, int nblocks);
 int push64_blocks_per_cu(void);
 int launch_counts_natural(hipStream_t s, const TileView &tv, const Grid &g, int32_t *out);
 
@@ -139,7 +139,7 @@ int launch_counts_natural(hipStream_t s, const TileView &tv, const Grid &g, int3
 /* nblocks workgroups of 'waves' (1, 2 or 4) wavefronts each. */
 int launch_push32(hipStream_t s, const Markers32 &m, const Markers32 &dst, const Fields32 &f,
                   const Grid &g, const PushConsts &pc, const float *qm, const TileView &tv,
-                  float *tj, double *Wacc, int nblocks, int waves);
+                  float *tj, double *kin, int nblocks, int waves);
 int launch_jgather32(hipStream_t s, const Fields32 &f, const Grid &g, const TileView &tv,
                      const float *tj, int nblocks);
 int launch_keys32(hipStream_t s, const Markers32 &m, long n, const TileView &tv, int parity);
