@@ -484,10 +484,13 @@ __device__ static inline void write_back(const Markers32 &d, const TileView &tv,
  * counter).  The tile's E/H nodes are staged in LDS once for the W
  * wavefronts, which push interleaved batches of 64 markers each and add to
  * one FP32 LDS J block; the block is stored, without atomics, as the item's
- * block in 'tj'.  More wavefronts per tile keep every SIMD busy when tiles
- * are few (a 32^3 box has 512) and let the hardware balance tiles of very
- * different occupancy (workgroups finish at different times and new ones
- * start); each wavefront loads its next batch before pushing the current. */
+ * block in 'tj'.  Several wavefronts per tile (4 by default, see
+ * mpic_create) share the staging and the block, shorten a tile's serial chain
+ * of batches and let the hardware balance tiles of very different occupancy;
+ * each wavefront loads its next batch before pushing the current.  Laser-foil
+ * push (8.57 M markers) 202 us with one wavefront per tile, 165 us with
+ * four; it is bound by VALU issue (about 530 instructions per batch of 64
+ * at 4 cycles each, 65 % of the time on a full box). */
 struct Push32Args {
     Markers32    m, d;         /* current buffer (read through tv.perm), output buffer */
     F32View      v;
@@ -514,9 +517,15 @@ __device__ __forceinline__ static void push32_tiles(const Markers32 &m, const Ma
     const int nitems = *tv.nitems;
     float w0 = 0, w1 = 0, w2 = 0;         /* per-thread kinetic energy partials */
     for (int it = (int)bk.x; it < nitems; it += (int)gd.x) {
-        const int sl = tv.item[it];
-        const int t = tv.active[sl];
-        const int u = it - tv.istart[sl], nu = tv.istart[sl + 1] - tv.istart[sl];
+        const int4 work = tv.item[it];
+        const int t = work.x;
+        const unsigned beg = work.y, end = work.z;
+        /* the order's indices are loaded two batches ahead and the records
+         * one batch ahead, so no load waits for an index just loaded; the
+         * first ones are under way while the fields are staged */
+        const unsigned s0 = perm_at(tv.perm, beg + threadIdx.x, end - 1);
+        unsigned snx = perm_at(tv.perm, beg + BS + threadIdx.x, end - 1);
+        MarkerRegs cur;
         int t0, t1, t2;
         tile_coords(tv, t, t0, t1, t2);
         const int c0 = TILE * t0, c1 = TILE * t1, c2 = TILE * t2;
@@ -552,6 +561,7 @@ __device__ __forceinline__ static void push32_tiles(const Markers32 &m, const Ma
 #pragma unroll
                 for (int r = 0; r < NSTG; ++r) st[comp][r] = at(F, offs[r]);
             }
+            load_marker(m, s0, cur);
 #pragma unroll
             for (int comp = 0; comp < 6; ++comp)
 #pragma unroll
@@ -560,15 +570,6 @@ __device__ __forceinline__ static void push32_tiles(const Markers32 &m, const Ma
                     if (rr < TFN3) lf[comp * TFN3 + rr] = ok[r] ? st[comp][r] : 0.0f;
                 }
         }
-        /* item u of nu: an even share of the tile's markers */
-        const unsigned tb = tv.toff[t], cnt = tv.toff[t + 1] - tb;
-        const unsigned beg = tb + (unsigned)((unsigned long long)u * cnt / nu),
-                       end = tb + (unsigned)((unsigned long long)(u + 1) * cnt / nu);
-        /* the order's indices are loaded two batches ahead and the records
-         * one batch ahead, so no load waits for an index just loaded */
-        MarkerRegs cur;
-        load_marker(m, perm_at(tv.perm, beg + threadIdx.x, end - 1), cur);
-        unsigned snx = perm_at(tv.perm, beg + BS + threadIdx.x, end - 1);
         /* everything outstanding completes here, so that the loop's waits
          * only ever concern the prefetch of the batch in flight */
         __builtin_amdgcn_s_waitcnt(0);
@@ -692,9 +693,9 @@ __device__ __forceinline__ static void jgather32(const F32View &v, const TileVie
                       uz = t2 - 1 + threadIdx.x % 3;
             const bool in = ux >= 0 && uy >= 0 && uz >= 0 && ux < tv.nt[0] && uy < tv.nt[1] &&
                             uz < tv.nt[2];
-            const int su = in ? tv.slot[(ux * tv.nt[1] + uy) * tv.nt[2] + uz] : -1;
-            nfirst[threadIdx.x] = su >= 0 ? tv.istart[su] : 0;
-            nitem[threadIdx.x] = su >= 0 ? tv.istart[su + 1] - tv.istart[su] : 0;
+            const int2 ti = in ? tv.titem[(ux * tv.nt[1] + uy) * tv.nt[2] + uz] : make_int2(0, 0);
+            nfirst[threadIdx.x] = ti.x;
+            nitem[threadIdx.x] = ti.y;
         }
         __syncthreads();
         /* nodes in reverse order: the nodes an interior tile owns (block
@@ -792,8 +793,9 @@ int launch_push32(hipStream_t s, const Markers32 &m, const Markers32 &dst, const
     case 1: return launch_def(s, Push32ArgsW<1>{a}, (unsigned)nblocks);
     case 2: return launch_def(s, Push32ArgsW<2>{a}, (unsigned)nblocks);
     case 4: return launch_def(s, Push32ArgsW<4>{a}, (unsigned)nblocks);
+    case 8: return launch_def(s, Push32ArgsW<8>{a}, (unsigned)nblocks);
     default:
-        mpic_set_error("launch_push32: %d wavefronts per tile (1, 2 or 4)", waves);
+        mpic_set_error("launch_push32: %d wavefronts per tile (1, 2, 4 or 8)", waves);
         return MPIC_ERR_ARG;
     }
 }

@@ -399,7 +399,7 @@ extern "C" int mpic_footprint(const mpic_config_t *cfg, size_t *bytes)
     const size_t items = (size_t)items_capacity((int)tiles, cap, fp32 ? push32_item_markers() : 0);
     *bytes = field_bytes(cfg->n, fp32) + 2 * sizeof(double) * cells +
              2 * (size_t)cap * mk + tiles * 64 * 3 * sizeof(int) + tiles * 6 * sizeof(int) +
-             items * sizeof(int) + (fp32 ? items * TJB * sizeof(float) : 0);
+             items * sizeof(int4) + (fp32 ? items * TJB * sizeof(float) : 0);
     return MPIC_OK;
 }
 
@@ -528,11 +528,11 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     tv.perm = nullptr;
     if (r->tiled) MPIC_CHECK(hipMalloc(&tv.perm, sizeof(int) * r->cap));
     MPIC_CHECK(hipMalloc(&tv.active, sizeof(int) * tv.ntiles));
-    MPIC_CHECK(hipMalloc(&tv.slot, sizeof(int) * tv.ntiles));
     tv.chm = r->fp32 ? push32_item_markers() : 0;
     r->items_cap = items_capacity(tv.ntiles, r->cap, tv.chm);
-    MPIC_CHECK(hipMalloc(&tv.item, sizeof(int) * r->items_cap));
-    MPIC_CHECK(hipMalloc(&tv.istart, sizeof(int) * ((size_t)tv.ntiles + 1)));
+    MPIC_CHECK(hipMalloc(&tv.item, sizeof(int4) * r->items_cap));
+    MPIC_CHECK(hipMalloc(&tv.titem, sizeof(int2) * tv.ntiles));
+    MPIC_CHECK(hipMemsetAsync(tv.titem, 0, sizeof(int2) * tv.ntiles, r->stream));
     if (r->fp32) MPIC_CHECK(hipMalloc(&r->tj, sizeof(float) * TJB * (size_t)r->items_cap));
     MPIC_CHECK(hipMalloc(&tv.nactive, sizeof(int) * (4 + MPIC_XCDS)));
     tv.queue = tv.nactive + 1;
@@ -553,16 +553,23 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
          * the tiles: a workgroup pushes whole tiles */
         r->push_blocks = ncu * push64_blocks_per_cu();
         if (r->push_blocks > tv.ntiles) r->push_blocks = tv.ntiles;
-        /* the resident wavefronts of the tile push (16 per CU), one per
-         * workgroup; a workgroup takes work items with stride = grid size */
+        /* The tile push: a workgroup per work item up to 16 per CU (it takes
+         * items with stride = grid size), 4 wavefronts each; 8 on a box of
+         * at most two tiles per CU, where every wavefront is resident
+         * at once and the time is that of one wavefront's serial batches.
+         * Push in us with 1 / 2 / 4 / 8 wavefronts: 32^3 box, 512 tiles
+         * 59 / 39 / 26 / 24; 12^3 box 55 / 35 / 22 / 17; 64^3 foil
+         * 45 / 34 / 26 / 28; 64^3 full box 161 / 141 / 127 / 138; laser-foil
+         * 202 / 191 / 165 / 170. */
         r->tile_blocks = 16 * ncu < r->items_cap ? 16 * ncu : (int)r->items_cap;
-        r->tile_waves = 1;
+        r->tile_waves = tv.ntiles <= 2 * ncu ? 8 : 4;
         r->gather_blocks = 16 * ncu;
         r->ncu = ncu;
         const char *e = getenv("MPIC_PUSH_BLOCKS");
         if (e && atoi(e) > 0) r->push_blocks = r->tile_blocks = atoi(e);
         const char *w = getenv("MPIC_TILE_WAVES");
-        if (w && (atoi(w) == 2 || atoi(w) == 4)) r->tile_waves = atoi(w);
+        if (w && (atoi(w) == 1 || atoi(w) == 2 || atoi(w) == 4 || atoi(w) == 8))
+            r->tile_waves = atoi(w);
     }
     r->n = 0;
     MPIC_CHECK(hipMalloc(&r->dacc, sizeof(double) * 8));
@@ -639,8 +646,8 @@ extern "C" int mpic_destroy(mpic_run_t *r)
     }
     hipFree(r->tv.off); hipFree(r->tv.toff); hipFree(r->tv.cursor); hipFree(r->tv.count); hipFree(r->tv.key);
     hipFree(r->tv.perm);
-    hipFree(r->tv.active); hipFree(r->tv.slot); hipFree(r->tv.nactive); hipFree(r->scanw);
-    hipFree(r->tv.item); hipFree(r->tv.istart);
+    hipFree(r->tv.active); hipFree(r->tv.nactive); hipFree(r->scanw);
+    hipFree(r->tv.item); hipFree(r->tv.titem);
     hipFree(r->tj);
     hipFree(r->dacc);
     hipFree(r->dkin);
@@ -2577,9 +2584,9 @@ static int ensure_items(mpic_run *r, int chm)
     const long need = items_capacity(r->tv.ntiles, r->cap, chm);
     if (need <= r->items_cap) return MPIC_OK;
     MPIC_CHECK(hipStreamSynchronize(r->stream));
-    int *item = nullptr;
+    int4 *item = nullptr;
     float *tj = nullptr;
-    if (hipMalloc(&item, sizeof(int) * need) != hipSuccess ||
+    if (hipMalloc(&item, sizeof(int4) * need) != hipSuccess ||
         hipMalloc(&tj, sizeof(float) * TJB * (size_t)need) != hipSuccess) {
         hipFree(item);
         mpic_set_error("work items of %d markers: %ld items do not fit on the device", chm, need);
@@ -2617,7 +2624,7 @@ extern "C" int mpic_autotune(mpic_run_t *r, int steps, int *chosen)
         return MPIC_OK;
     }
     const int chms[3] = {0, 2048, 1024};
-    const int wavess[3] = {1, 2, 4};
+    const int wavess[4] = {1, 2, 4, 8};
     const char *verbose = getenv("MPIC_AUTOTUNE_VERBOSE");
     int best_nb = r->tile_blocks, best_w = r->tile_waves, best_chm = r->tv.chm;
     double best_ms = 1e300;
@@ -2629,7 +2636,7 @@ extern "C" int mpic_autotune(mpic_run_t *r, int steps, int *chosen)
         r->tv.chm = chm;
         TRY(sort_pass(r, 1));
         TRY(advance_timed(r, 1));          /* untimed: first launches of the new lists */
-        for (int wi = 0; wi < 3; ++wi) {
+        for (int wi = 0; wi < 4; ++wi) {
             const int w = wavess[wi];
             for (int per_cu = 4; per_cu <= 64; per_cu *= 2) {
                 int nb = per_cu * r->ncu / w;

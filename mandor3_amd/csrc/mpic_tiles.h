@@ -28,7 +28,6 @@ struct TileView {
     int *perm;               /* [capacity] the current order as indices into the
                               * current buffer (nmark[parity] of them; tiled runs) */
     int *active;             /* [ntiles] tiles holding markers, in tile order */
-    int *slot;               /* [ntiles] position of a tile in 'active', -1 if empty */
     int *nactive;            /* [1] */
     int *queue;              /* [MPIC_XCDS] work counters */
     int *nmark;              /* [2] markers in the current / next order */
@@ -36,8 +35,10 @@ struct TileView {
      * into ceil(count / chm) items of at most chm markers (chm = 0: one
      * item per active tile). */
     int  chm;
-    int *item;               /* [item capacity] active slot of each work item */
-    int *istart;             /* [ntiles + 1] first item of each active slot, [nactive] = items */
+    int4 *item;              /* [item capacity] work items in tile order: tile, first and last + 1
+                              * position in the order (one load tells a workgroup its work: a
+                              * chain of lookups costs a memory latency per link) */
+    int2 *titem;             /* [ntiles] first item and item count of every tile (count 0: empty) */
     int *nitems;             /* [1] */
 };
 

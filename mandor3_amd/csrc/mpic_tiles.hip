@@ -197,7 +197,6 @@ __device__ static inline void scan_pass(const ScanArgs &A, const VBlock &bk)
             tv.off[tv.ncellp] = tot;
             tv.toff[tv.ntiles] = tot;
             *tv.nactive = na;
-            tv.istart[na] = ni;
             *tv.nitems = ni;
             tv.nmark[A.parity_next] = tot;
             for (int q = 0; q < MPIC_XCDS; ++q) tv.queue[q] = 0;
@@ -210,14 +209,15 @@ __device__ static inline void scan_pass(const ScanArgs &A, const VBlock &bk)
     const int t = wt0 + lane;
     if (t < tv.ntiles) {
         tv.toff[t] = base;
-        const int a = spre[1] + inc[1] - own[1];
+        const int is = spre[2] + inc[2] - own[2], nu = own[2];
         if (c > 0) {
-            const int is = spre[2] + inc[2] - own[2];
-            tv.active[a] = t;
-            tv.istart[a] = is;
-            for (int u = 0; u < own[2]; ++u) tv.item[is + u] = a;
+            tv.active[spre[1] + inc[1] - own[1]] = t;
+            /* item u of nu: an even share of the tile's markers */
+            for (int u = 0; u < nu; ++u)
+                tv.item[is + u] = make_int4(t, base + (int)((long)u * c / nu),
+                                            base + (int)((long)(u + 1) * c / nu), 0);
         }
-        tv.slot[t] = c > 0 ? a : -1;
+        tv.titem[t] = make_int2(is, nu);
     }
     /* per-key offsets and cursors of the non-empty tiles, counters reset
      * (entries of empty tiles are not maintained) */

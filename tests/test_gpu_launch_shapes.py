@@ -1,0 +1,49 @@
+"""Launch shapes of the FP32 push beside those of test_gpu_modes.py: 1 and 8
+wavefronts per workgroup (8 is the rule's choice on small boxes), and the
+kinetic sums, which every wavefront adds to one of 256 slots.  Bars: the split
+form's own."""
+import numpy as np
+import pytest
+
+import mandor3_amd as ma
+from mandor3_amd import workloads
+from test_gpu_modes import _split_twenty_steps
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("items", [None, "64"])
+@pytest.mark.parametrize("waves", ["1", "8"])
+@pytest.mark.parametrize("case", ["periodic", "mixed"])
+def test_one_and_eight_wavefronts_per_tile(case, waves, items, monkeypatch):
+    monkeypatch.setenv("MPIC_TILE_WAVES", waves)
+    if items:
+        monkeypatch.setenv("MPIC_ITEM_MARKERS", items)
+    _split_twenty_steps(case, "%s wavefronts, items %s" % (waves, items))
+
+
+@pytest.mark.parametrize("prec", [ma.FP64, ma.FP32_SPLIT])
+@pytest.mark.parametrize("n", [8, 33])
+def test_kinetic_sums(n, prec):
+    """The first push of the two-stream box starts from E = H = 0, so its sums
+    are sum (gamma - 1) w u_a^2 / u^2 h^3 m/q over the loaded momenta: 8^3 has
+    fewer wavefronts than slots, 33^3 several per slot."""
+    st = workloads.two_stream_box(n)
+    M = st["markers"]
+    r = ma.Run(st["n"], st["h"], st["L"], st["tau"], st["bc"], 0.0, precision=prec,
+               max_markers=M.size)
+    z = np.zeros(3 * r.nodes)
+    r.set_fields(z, z)
+    r.load_markers(M)
+    r.init()
+    u = np.stack([M["vx"], M["vy"], M["vz"]])
+    u2 = (u * u).sum(0)
+    # (gamma - 1) / u^2 = 1 / (gamma + 1): no cancellation for slow markers
+    w = M["rho"].astype(float) / M["qDivM"] / (np.sqrt(1 + u2) + 1) * 0.05 ** 3
+    want = (w * u * u).sum(1)
+    r.stage("em_h_half")
+    r.stage("push_deposit")
+    got = r.temperature()
+    # FP32: momenta and each term rounded to 2^-24, all terms of one sign
+    np.testing.assert_allclose(got, want, rtol=1e-11 if prec == ma.FP64 else 1e-6)
+    r.close()
