@@ -185,7 +185,7 @@ int  mpic_set_graphs(mpic_run_t *run, int on);
 int  mpic_batch_advance(mpic_run_t *const *runs, int nruns, int nsteps);
 /* Picks the launch shape of the FP32 push -- markers per work item (a
  * tile's markers split into even items of at most 2048 or 1024, or one item
- * per tile), wavefronts per workgroup (1, 2, 4 or 8 sharing one tile's staged
+ * per tile), wavefronts per workgroup (1, 2 or 4 sharing one tile's staged
  * fields and J block) and workgroup count -- by timing 'steps' real steps
  * per candidate (the steps advance the run; the choice changes results only
  * by the summation order of J).  chosen (may be NULL) receives {workgroups,

@@ -1,7 +1,7 @@
 /*
  * mpic_push64.hip -- FP64 plain-form marker push and current deposit.
  *
- * One thread per marker: trilinear gather of E and H on the staggered Yee
+ * Per marker: trilinear gather of E and H on the staggered Yee
  * grid (source/misc_PIC.h:18-126), relativistic Boris rotation
  * (source/core/plasma.c:115-171), charge-conserving deposit of the straight
  * trajectory split at cell faces (source/core/plasma_currentKernel.c:20-279)
@@ -10,8 +10,13 @@
  * bit; J is accumulated with FP64 atomics, so only the summation order of J
  * differs from the CPU path.
  *
- * Roofline: HBM-bound.  Algorithmic bytes per marker-step: read 56 B +
- * write 52 B of SoA marker data (x y z ux uy uz, w qm, id read once), plus
+ * Two kernels: the tiled push (the default; one workgroup per tile of
+ * sorted markers, fields and J staged in LDS) and the untiled one (one thread
+ * per marker, everything straight from and to HBM), whose general marker
+ * push also takes the markers the tiled one leaves.
+ *
+ * Roofline: HBM-bound.  Algorithmic bytes per marker-step: 128 B (read the
+ * order's index, 56 B of state and the id; write state, id and new key), plus
  * per cell 48 B of E/H reads and 48 B of J read-modify-write divided by the
  * markers per cell.
  */
@@ -42,10 +47,7 @@ __device__ static inline double gather(const double *F, const Grid &g, int i, do
            F[gidx(g, i + 1, j + 1, k + 1)] * sx * (sy * sz);
 }
 
-/* Deposit targets.  GlobalSink adds straight to J in HBM with FP64
- * atomics; TileSink (tiled kernel) adds to a 7x7x7-node J block in LDS that
- * covers a 4x4x4-cell tile and its one-cell rim, and falls back to HBM for a
- * segment outside it. */
+/* Deposit target of the untiled push: J in HBM, by FP64 atomics. */
 struct GlobalSink {
     double *J[3];
     Grid g;
@@ -64,44 +66,6 @@ struct GlobalSink {
         unsafeAtomicAdd(J[2] + gidx(g, i + 1, j, k + 1), vz[1]);
         unsafeAtomicAdd(J[2] + gidx(g, i, j + 1, k + 1), vz[2]);
         unsafeAtomicAdd(J[2] + gidx(g, i + 1, j + 1, k + 1), vz[3]);
-    }
-};
-
-#define TILE 4
-/* TJN (mpic_tiles.h): LDS J nodes per axis, the tile plus its rim */
-
-struct TileSink {
-    GlobalSink gs;
-    double *lj;                    /* LDS: [TJN^3][3] */
-    int o0, o1, o2;                /* node of lj[0] */
-    __device__ void seg(int i, int j, int k, const double vx[4], const double vy[4],
-                        const double vz[4]) const
-    {
-        const int a = i - o0, b = j - o1, c = k - o2;
-        if (a < 0 || b < 0 || c < 0 || a > TJN - 2 || b > TJN - 2 || c > TJN - 2) {
-            gs.seg(i, j, k, vx, vy, vz);
-            return;
-        }
-        lds_add(a, b, c, vx, vy, vz);
-    }
-    /* the 12 values of a segment in the block's cell (a, b, c) */
-    __device__ void lds_add(int a, int b, int c, const double vx[4], const double vy[4],
-                            const double vz[4]) const
-    {
-#define L(aa, bb, cc, comp) (lj + 3 * (((aa) * TJN + (bb)) * TJN + (cc)) + (comp))
-        atomicAdd(L(a + 1, b, c, 0), vx[0]);
-        atomicAdd(L(a + 1, b + 1, c, 0), vx[1]);
-        atomicAdd(L(a + 1, b, c + 1, 0), vx[2]);
-        atomicAdd(L(a + 1, b + 1, c + 1, 0), vx[3]);
-        atomicAdd(L(a, b + 1, c, 1), vy[0]);
-        atomicAdd(L(a + 1, b + 1, c, 1), vy[1]);
-        atomicAdd(L(a, b + 1, c + 1, 1), vy[2]);
-        atomicAdd(L(a + 1, b + 1, c + 1, 1), vy[3]);
-        atomicAdd(L(a, b, c + 1, 2), vz[0]);
-        atomicAdd(L(a + 1, b, c + 1, 2), vz[1]);
-        atomicAdd(L(a, b + 1, c + 1, 2), vz[2]);
-        atomicAdd(L(a + 1, b + 1, c + 1, 2), vz[3]);
-#undef L
     }
 };
 
@@ -134,8 +98,7 @@ __device__ static inline void seg_values(const Grid &g, int i, int j, int k, dou
 }
 
 /* Deposit of one straight segment inside cell (i,j,k). */
-template <class S>
-__device__ static void deposit_seg(const S &v, const Grid &g, int i, int j, int k, double x1,
+__device__ static void deposit_seg(const GlobalSink &v, const Grid &g, int i, int j, int k, double x1,
                                    double x2, double y1, double y2, double z1, double z2,
                                    double rp)
 {
@@ -144,40 +107,10 @@ __device__ static void deposit_seg(const S &v, const Grid &g, int i, int j, int 
     v.seg(i, j, k, vx, vy, vz);
 }
 
-/* The first straight segment of a marker's path, in its start cell: the
- * tiled push keeps it (kKeep) to sum it over the run of markers that share
- * the cell (the markers are sorted by cell) before it reaches LDS. */
-struct FirstSeg {
-    int    i, j, k, on;
-    double x1, x2, y1, y2, z1, z2;
-};
-
-template <bool kKeep, class S>
-__device__ static inline void first_seg(const S &v, const Grid &g, FirstSeg *fs, int i, int j,
-                                        int k, double x1, double x2, double y1, double y2,
-                                        double z1, double z2, double rp)
-{
-    if constexpr (kKeep) {
-        fs->i = i;
-        fs->j = j;
-        fs->k = k;
-        fs->on = 1;
-        fs->x1 = x1;
-        fs->x2 = x2;
-        fs->y1 = y1;
-        fs->y2 = y2;
-        fs->z1 = z1;
-        fs->z2 = z2;
-    } else {
-        deposit_seg(v, g, i, j, k, x1, x2, y1, y2, z1, z2, rp);
-    }
-}
-
 /* Two or three face crossings, source/core/plasma_currentKernel.c:156-279. */
-template <bool kKeep, class S>
-__device__ static void deposit_multi(const S &v, const Grid &g, int i1, int j1, int k1, int i2,
-                                     int j2, int k2, double x1, double y1, double z1, double x2,
-                                     double y2, double z2, double rp, FirstSeg *fs)
+__device__ static void deposit_multi(const GlobalSink &v, const Grid &g, int i1, int j1, int k1,
+                                     int i2, int j2, int k2, double x1, double y1, double z1,
+                                     double x2, double y2, double z2, double rp)
 {
     const double h1 = g.h[0], h2 = g.h[1], h3 = g.h[2];
     const int di = abs(i2 - i1), dj = abs(j2 - j1), dk = abs(k2 - k1);
@@ -201,7 +134,7 @@ __device__ static void deposit_multi(const S &v, const Grid &g, int i1, int j1, 
         }
         const double xA = x1 + k1s * (x2 - x1), yA = y1 + k1s * (y2 - y1), zA = z1 + k1s * (z2 - z1);
         const double xB = x1 + k2s * (x2 - x1), yB = y1 + k2s * (y2 - y1), zB = z1 + k2s * (z2 - z1);
-        first_seg<kKeep>(v, g, fs, i, j, k, x1, xA, y1, yA, z1, zA, rp);
+        deposit_seg(v, g, i, j, k, x1, xA, y1, yA, z1, zA, rp);
         i += st ? dI1[0] : dI0[0];
         j += st ? dI1[1] : dI0[1];
         k += st ? dI1[2] : dI0[2];
@@ -232,8 +165,7 @@ __device__ static void deposit_multi(const S &v, const Grid &g, int i1, int j1, 
     if (a1 > a3) { int t = s1; s1 = s3; s3 = t; double d = a1; a1 = a3; a3 = d; }
     if (a2 > a3) { int t = s2; s2 = s3; s3 = t; double d = a2; a2 = a3; a3 = d; }
     int ii[3] = {i1, j1, k1};
-    first_seg<kKeep>(v, g, fs, ii[0], ii[1], ii[2], x1, rc[s1][0], y1, rc[s1][1], z1, rc[s1][2],
-                     rp);
+    deposit_seg(v, g, ii[0], ii[1], ii[2], x1, rc[s1][0], y1, rc[s1][1], z1, rc[s1][2], rp);
     ii[s1] += dI[s1];
     deposit_seg(v, g, ii[0], ii[1], ii[2], rc[s1][0], rc[s2][0], rc[s1][1], rc[s2][1], rc[s1][2],
                 rc[s2][2], rp);
@@ -268,10 +200,9 @@ __device__ static inline int walls(const PushConsts &c, double *r, double *u)
 /* Gather, Boris and deposit of one live marker; returns 0 for a marker off
  * the grid (deleted and flagged), else applies the walls and returns
  * whether the marker survives.  r/u are in/out. */
-template <bool kKeep = false, class S>
-__device__ static int push_marker(const S &sink, const F64View &v, const PushConsts &c, double r[3],
-                                  double u[3], float rhof, float qmf, double w3[3], unsigned *err,
-                                  FirstSeg *fs = nullptr)
+__device__ static int push_marker(const GlobalSink &sink, const F64View &v, const PushConsts &c,
+                                  double r[3], double u[3], float rhof, float qmf, double w3[3],
+                                  unsigned *err)
 {
     const Grid &g = v.g;
     const double h1 = g.h[0], h2 = g.h[1], h3 = g.h[2], tau = g.tau;
@@ -317,17 +248,17 @@ __device__ static int push_marker(const S &sink, const F64View &v, const PushCon
     if (fabs(z2 - z1) < 1e-10 * h3) { dk = 0; k2 = k; }
     const double rp = rhof;
     if (di + dj + dk == 0) {
-        first_seg<kKeep>(sink, g, fs, i, j, k, x1, x2, y1, y2, z1, z2, rp);
+        deposit_seg(sink, g, i, j, k, x1, x2, y1, y2, z1, z2, rp);
     } else if (di + dj + dk == 1) {
         const double alpha = dk * ((k + k2 + 1) * 0.5 * h3 - z1) / (z2 - z1 + ((1 - dk) << 16))
                            + dj * ((j + j2 + 1) * 0.5 * h2 - y1) / (y2 - y1 + ((1 - dj) << 16))
                            + di * ((i + i2 + 1) * 0.5 * h1 - x1) / (x2 - x1 + ((1 - di) << 16));
         const double xC = x1 + alpha * (x2 - x1), yC = y1 + alpha * (y2 - y1),
                      zC = z1 + alpha * (z2 - z1);
-        first_seg<kKeep>(sink, g, fs, i, j, k, x1, xC, y1, yC, z1, zC, rp);
+        deposit_seg(sink, g, i, j, k, x1, xC, y1, yC, z1, zC, rp);
         deposit_seg(sink, g, i2, j2, k2, xC, x2, yC, y2, zC, z2, rp);
     } else {
-        deposit_multi<kKeep>(sink, g, i, j, k, i2, j2, k2, x1, y1, z1, x2, y2, z2, rp, fs);
+        deposit_multi(sink, g, i, j, k, i2, j2, k2, x1, y1, z1, x2, y2, z2, rp);
     }
     r[0] = x2;
     r[1] = y2;
@@ -423,6 +354,305 @@ int launch_push64(hipStream_t s, const Markers64 &m, long n, const Fields64 &f, 
     return launch_def(s, a, (unsigned)((n + TPB - 1) / TPB));
 }
 
+/* ---------------- tiled push ---------------- */
+#define TW 64                  /* wavefront width */
+#define TILE 4
+#define TFN (TILE + 2)         /* E/H nodes per axis staged for a tile's gathers */
+#define TFN3 (TFN * TFN * TFN)
+
+struct Push64Consts {
+    PushConsts pc;
+    double     yh[3], yl[3];   /* 1/h as the sum of two doubles */
+    double     cj[3];          /* h/tau: J of a segment per unit charge density and cell */
+    double     vol;            /* h1*h2*h3 */
+};
+
+/* a / b, correctly rounded, from b's reciprocal yh + yl (yh = RN(1/b), yl
+ * the rounded rest): q is within one unit in the last place of a/b, the
+ * remainder a - q b is exact, and one correction with yh = RN(1/b) then
+ * rounds correctly (P. W. Markstein, "Computation of elementary functions on
+ * the IBM RISC System/6000 processor", IBM J. Res. Dev. 34, 1990).  Four
+ * instructions instead of the eleven of a division; a zero's sign may differ. */
+__device__ static inline double div_by(double a, double b, double yh, double yl)
+{
+    const double q = __builtin_fma(a, yh, a * yl);
+    return __builtin_fma(__builtin_fma(-b, q, a), yh, q);
+}
+
+/* 1/x to about one unit in the last place: the hardware's estimate and two
+ * Newton steps.  Used where the reference's rounding does not matter (the
+ * crossing fraction of a segment, the energy sums). */
+__device__ static inline double rcp64(double x)
+{
+    double y = __builtin_amdgcn_rcp(x);
+    y = __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+    return __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+}
+
+__device__ static inline void cswap(double &a, int &ia, double &b, int &ib)
+{
+    if (b < a) {
+        const double t = a; a = b; b = t;
+        const int u = ia; ia = ib; ib = u;
+    }
+}
+
+/* Marker state held in registers between the prefetch and the push, and
+ * between the push and the stores. */
+struct Marker64 {
+    double  r[3], u[3];
+    float   w, qm;
+    int32_t id;
+};
+
+/* Records are read once and written once per step: nontemporal, so that they
+ * do not push the fields out of the caches. */
+__device__ static inline void load_marker(const Markers64 &m, unsigned s, Marker64 &k)
+{
+    k.r[0] = __builtin_nontemporal_load(m.x + s);
+    k.r[1] = __builtin_nontemporal_load(m.y + s);
+    k.r[2] = __builtin_nontemporal_load(m.z + s);
+    k.u[0] = __builtin_nontemporal_load(m.ux + s);
+    k.u[1] = __builtin_nontemporal_load(m.uy + s);
+    k.u[2] = __builtin_nontemporal_load(m.uz + s);
+    k.w = __builtin_nontemporal_load(m.w + s);
+    k.qm = __builtin_nontemporal_load(m.qm + s);
+    k.id = __builtin_nontemporal_load(m.id + s);
+}
+
+/* Results of one batch, written back at the start of the next (after its
+ * prefetch is issued), so that no wait for the prefetch also waits for
+ * fresh stores. */
+struct Pending64 {
+    Marker64 k;
+    unsigned p;
+    int      key;              /* new key, -1 deleted */
+    bool     valid;            /* lane holds a marker of the order */
+    int      ckey, clen;       /* count run head: key (-1 none), length */
+};
+
+__device__ static inline void write_back(const Markers64 &d, const TileView &tv,
+                                         const Pending64 &q)
+{
+    if (q.valid) {
+        if (q.key >= 0) {
+            __builtin_nontemporal_store(q.k.r[0], d.x + q.p);
+            __builtin_nontemporal_store(q.k.r[1], d.y + q.p);
+            __builtin_nontemporal_store(q.k.r[2], d.z + q.p);
+            __builtin_nontemporal_store(q.k.u[0], d.ux + q.p);
+            __builtin_nontemporal_store(q.k.u[1], d.uy + q.p);
+            __builtin_nontemporal_store(q.k.u[2], d.uz + q.p);
+        }
+        __builtin_nontemporal_store(q.key >= 0 ? q.k.w : 0.0f, d.w + q.p);
+        __builtin_nontemporal_store(q.key >= 0 ? q.k.qm : 0.0f, d.qm + q.p);
+        __builtin_nontemporal_store(q.k.id, d.id + q.p);
+        tv.key[q.p] = q.key;                               /* read by the rank pass next */
+    }
+    if (q.ckey >= 0) atomicAdd(tv.count + q.ckey, q.clen);
+}
+
+/* The reference's trilinear sum over eight values, in its order. */
+__device__ static inline double lgather(const double *F, int a, double sx, int b, double sy,
+                                        int c, double sz)
+{
+    const double *p = F + (a * TFN + b) * TFN + c;
+    const int dj = TFN, di = TFN * TFN;
+    return p[0] * (1 - sx) * ((1 - sy) * (1 - sz)) + p[di] * sx * ((1 - sy) * (1 - sz)) +
+           p[dj] * (1 - sx) * (sy * (1 - sz)) + p[di + dj] * sx * (sy * (1 - sz)) +
+           p[1] * (1 - sx) * ((1 - sy) * sz) + p[di + 1] * sx * ((1 - sy) * sz) +
+           p[dj + 1] * (1 - sx) * (sy * sz) + p[di + dj + 1] * sx * (sy * sz);
+}
+
+/* 12 J values of one straight segment inside a cell, in cell units: start
+ * q1, end q2 relative to the cell's origin, w3[a] = rho h_a / tau.  The
+ * deposit's sums are rounded in any order anyway, so its arithmetic may fuse
+ * multiply and add. */
+__device__ static inline void seg_cell(const double q1[3], const double q2[3], const double w3[3],
+                                       double v[12])
+{
+#pragma clang fp contract(fast)
+    const double dx = q2[0] - q1[0], dy = q2[1] - q1[1], dz = q2[2] - q1[2];
+    const double tx = 0.5 * (q1[0] + q2[0]), ty = 0.5 * (q1[1] + q2[1]), tz = 0.5 * (q1[2] + q2[2]);
+    const double yz = dy * dz * (1.0 / 12), xz = dx * dz * (1.0 / 12), xy = dx * dy * (1.0 / 12);
+    const double ax = w3[0] * dx, ay = w3[1] * dy, az = w3[2] * dz;
+    v[0] = ax * ((1 - ty) * (1 - tz) + yz);
+    v[1] = ax * (ty * (1 - tz) - yz);
+    v[2] = ax * ((1 - ty) * tz - yz);
+    v[3] = ax * (ty * tz + yz);
+    v[4] = ay * ((1 - tx) * (1 - tz) + xz);
+    v[5] = ay * (tx * (1 - tz) - xz);
+    v[6] = ay * ((1 - tx) * tz - xz);
+    v[7] = ay * (tx * tz + xz);
+    v[8] = az * ((1 - tx) * (1 - ty) + xy);
+    v[9] = az * (tx * (1 - ty) - xy);
+    v[10] = az * ((1 - tx) * ty - xy);
+    v[11] = az * (tx * ty + xy);
+}
+
+/* Offset of node (+da,+db,+dc), component comp, from a node of the LDS J block. */
+#define LJO(da, db, dc, comp) (3 * (((da) * TJN + (db)) * TJN + (dc)) + (comp))
+
+/* A segment of the LDS block's cell (a, b, c), 0 to TJN - 2 each: a marker of
+ * the tile starts in block cells 1 to 4 and crosses at most one face per axis. */
+__device__ static inline void seg_add(double *lj, int a, int b, int c, const double s[12])
+{
+    double *p = lj + 3 * ((a * TJN + b) * TJN + c);
+    atomicAdd(p + LJO(1, 0, 0, 0), s[0]);
+    atomicAdd(p + LJO(1, 1, 0, 0), s[1]);
+    atomicAdd(p + LJO(1, 0, 1, 0), s[2]);
+    atomicAdd(p + LJO(1, 1, 1, 0), s[3]);
+    atomicAdd(p + LJO(0, 1, 0, 1), s[4]);
+    atomicAdd(p + LJO(1, 1, 0, 1), s[5]);
+    atomicAdd(p + LJO(0, 1, 1, 1), s[6]);
+    atomicAdd(p + LJO(1, 1, 1, 1), s[7]);
+    atomicAdd(p + LJO(0, 0, 1, 2), s[8]);
+    atomicAdd(p + LJO(1, 0, 1, 2), s[9]);
+    atomicAdd(p + LJO(0, 1, 1, 2), s[10]);
+    atomicAdd(p + LJO(1, 1, 1, 2), s[11]);
+}
+
+/* The tile being pushed: its index, first cell, neighbour strides (in tiles)
+ * and whether a wall lies within reach of its markers (they move less than a
+ * cell per step, so a tile one tile or more from every face is out of
+ * reach). */
+struct Tile64 {
+    int  t, c[3], s0, s1;
+    bool edge;
+};
+
+/* First segment of a lane's marker: the block cell that holds it (a << 8 | b
+ * << 4 | c), -1 when there is none to sum over the wavefront. */
+struct First64 {
+    int    cell;
+    double v[12];
+};
+
+/* Push of one marker: gather, Boris and move with the reference's arithmetic
+ * (bit for bit), deposit of every segment but the first into the tile's
+ * block.  Returns the new key (-1: deleted); k holds the new state.  A marker
+ * whose cell is not the tile's (its quotient rounds onto the box's far face,
+ * where its key was clamped, or it lies off the grid) is left untouched:
+ * OFF_TILE. */
+#define OFF_TILE -2
+__device__ static inline int push64_marker(Marker64 &k, const F64View &v, const Push64Consts &c,
+                                           const TileView &tv, const Tile64 &tl, const double *lf,
+                                           double *lj, First64 &first, double w3[3])
+{
+    const Grid &g = v.g;
+    const double tau = c.pc.tau;
+    double s[3], f[3], fh[3];
+    int ic[3], ih[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        s[a] = div_by(k.r[a], c.pc.h[a], c.yh[a], c.yl[a]);
+        const double sh = s[a] + 0.5;
+        ic[a] = DBL_TO_INT(s[a]);
+        ih[a] = DBL_TO_INT(sh);
+        f[a] = s[a] - ic[a];
+        fh[a] = sh - ih[a];
+    }
+    const int l[3] = {ic[0] - tl.c[0], ic[1] - tl.c[1], ic[2] - tl.c[2]};
+    if ((unsigned)l[0] >= TILE || (unsigned)l[1] >= TILE || (unsigned)l[2] >= TILE) return OFF_TILE;
+    const int m[3] = {ih[0] - tl.c[0], ih[1] - tl.c[1], ih[2] - tl.c[2]};
+    const double Ex = lgather(lf + 0 * TFN3, m[0], fh[0], l[1], f[1], l[2], f[2]),
+                 Ey = lgather(lf + 1 * TFN3, l[0], f[0], m[1], fh[1], l[2], f[2]),
+                 Ez = lgather(lf + 2 * TFN3, l[0], f[0], l[1], f[1], m[2], fh[2]),
+                 Hx = lgather(lf + 3 * TFN3, l[0], f[0], m[1], fh[1], m[2], fh[2]),
+                 Hy = lgather(lf + 4 * TFN3, m[0], fh[0], l[1], f[1], m[2], fh[2]),
+                 Hz = lgather(lf + 5 * TFN3, m[0], fh[0], m[1], fh[1], l[2], f[2]);
+    const double tauMass = 0.5 * tau * k.qm, px = k.u[0] + tauMass * Ex,
+                 py = k.u[1] + tauMass * Ey, pz = k.u[2] + tauMass * Ez,
+                 gamma = sqrt(1 + px * px + py * py + pz * pz);
+    {
+#pragma clang fp contract(fast)
+        const double p2 = px * px + py * py + pz * pz;
+        const double W = (gamma - 1.0) * k.w * c.vol * rcp64((p2 + 1e-19) * k.qm);
+        w3[0] += W * px * px;
+        w3[1] += W * py * py;
+        w3[2] += W * pz * pz;
+    }
+    const double tauGamma = tauMass / gamma;
+    const double aHx = tauGamma * Hx, aHy = tauGamma * Hy, aHz = tauGamma * Hz;
+    const double uu = px + py * aHz - pz * aHy, vv = py + pz * aHx - px * aHz,
+                 ww = pz + px * aHy - py * aHx;
+    const double bxx = aHx * aHx, byy = aHy * aHy, bzz = aHz * aHz, bxy = aHx * aHy,
+                 byz = aHy * aHz, bxz = aHz * aHx;
+    const double delta = 1.0 / (1 + bxx + byy + bzz);
+    k.u[0] = tauMass * Ex + ((1 + bxx) * uu + (bxy + aHz) * vv + (bxz - aHy) * ww) * delta;
+    k.u[1] = tauMass * Ey + ((bxy - aHz) * uu + (1 + byy) * vv + (byz + aHx) * ww) * delta;
+    k.u[2] = tauMass * Ez + ((bxz + aHy) * uu + (byz - aHx) * vv + (1 + bzz) * ww) * delta;
+    const double tg = tau / sqrt(1 + k.u[0] * k.u[0] + k.u[1] * k.u[1] + k.u[2] * k.u[2]);
+    /* the move: cells crossed per axis (-1, 0, 1) and the displacement in cells */
+    double d[3], rho3[3];
+    int to[3], fc[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const double x1 = k.r[a], x2 = x1 + k.u[a] * tg;
+        /* (a marker moves less than a cell: the clamp only keeps one that is
+         * not a number inside the block) */
+        to[a] = DBL_TO_INT(div_by(x2, c.pc.h[a], c.yh[a], c.yl[a])) - ic[a];
+        to[a] = to[a] < -1 ? -1 : (to[a] > 1 ? 1 : to[a]);
+        fc[a] = fabs(x2 - x1) < 1e-10 * c.pc.h[a] ? 0 : to[a];
+        d[a] = (x2 - x1) * c.yh[a];
+        rho3[a] = k.w * c.cj[a];
+        k.r[a] = x2;
+    }
+    /* Segments: from the start to the first face crossing (or the end), then
+     * one per crossed face.  Crossing fractions ascend; an axis that is not
+     * crossed gets 2 and sorts last. */
+    const int nc = (fc[0] != 0) + (fc[1] != 0) + (fc[2] != 0);
+    double a0 = 2.0, a1 = 2.0, a2 = 2.0, q[3] = {f[0] + d[0], f[1] + d[1], f[2] + d[2]};
+    const double e[3] = {q[0], q[1], q[2]};
+    int x0 = 0, x1 = 1, x2i = 2;
+    if (nc) {
+        if (fc[0]) a0 = ((fc[0] > 0 ? 1.0 : 0.0) - f[0]) * rcp64(d[0]);
+        if (fc[1]) a1 = ((fc[1] > 0 ? 1.0 : 0.0) - f[1]) * rcp64(d[1]);
+        if (fc[2]) a2 = ((fc[2] > 0 ? 1.0 : 0.0) - f[2]) * rcp64(d[2]);
+        cswap(a0, x0, a1, x1);
+        cswap(a1, x1, a2, x2i);
+        cswap(a0, x0, a1, x1);
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            q[a] = x0 == a ? (fc[a] > 0 ? 1.0 : 0.0) : __builtin_fma(a0, d[a], f[a]);
+    }
+    const double qf[3] = {q[0], q[1], q[2]};     /* the first segment's end */
+    if (nc) {
+        int sh[3] = {0, 0, 0}, axs = x0;
+#pragma unroll 1
+        for (int n = 1; n <= nc; ++n) {
+            double b[3], en[3], sv[12];
+            a0 = a1;
+            x0 = x1;
+            a1 = a2;
+            x1 = x2i;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                sh[a] += axs == a ? fc[a] : 0;
+                const double at = x0 == a ? (fc[a] > 0 ? 1.0 : 0.0) : __builtin_fma(a0, d[a], f[a]);
+                const double nx = n < nc ? at : e[a];
+                b[a] = q[a] - sh[a];
+                en[a] = nx - sh[a];
+                q[a] = nx;
+            }
+            seg_cell(b, en, rho3, sv);
+            seg_add(lj, l[0] + 1 + sh[0], l[1] + 1 + sh[1], l[2] + 1 + sh[2], sv);
+            axs = x0;
+        }
+    }
+    /* after the loop, so that its twelve values are not live through it */
+    seg_cell(f, qf, rho3, first.v);
+    first.cell = (l[0] + 1) << 8 | (l[1] + 1) << 4 | (l[2] + 1);
+    if (!tl.edge) {
+        /* no wall within reach: the new cell is within one cell of the tile,
+         * so its key follows from the tile's neighbour strides */
+        const int u0 = l[0] + to[0], u1 = l[1] + to[1], u2 = l[2] + to[2];
+        const int nt = tl.t + __mul24(u0 >> 2, tl.s0) + __mul24(u1 >> 2, tl.s1) + (u2 >> 2);
+        return nt * TILE_CELLS + (((u0 & 3) * TILE + (u1 & 3)) * TILE + (u2 & 3));
+    }
+    if (!walls(c.pc, k.r, k.u)) return -1;
+    return cell_key_of(tv, g, k.r);
+}
+
 /* Row shift of a double by D lanes inside rows of 16 (DPP row_shr on
  * both halves; 0 from outside the row).  Every lane must be active. */
 template <int D> __device__ static inline double row_shr(double x)
@@ -438,27 +668,13 @@ template <int D> __device__ static inline double row_shr(double x)
  * lanes, then added to LDS by the run's last lane in the row (at most 4
  * atomics per value and run instead of one per marker: LDS atomics to one
  * address serialise).  Called by every lane of the wavefront. */
-__device__ static inline void first_run_add(const TileSink &ts, const Grid &g, const FirstSeg &fs,
-                                            double rp)
+__device__ static inline void first_run_add(double *lj, First64 &fs)
 {
-    double vv[12];
-    int cell = -1, a = 0, b = 0, c = 0;
-    if (fs.on) {
-        seg_values(g, fs.i, fs.j, fs.k, fs.x1, fs.x2, fs.y1, fs.y2, fs.z1, fs.z2, rp, vv, vv + 4,
-                   vv + 8);
-        a = fs.i - ts.o0;
-        b = fs.j - ts.o1;
-        c = fs.k - ts.o2;
-        if (a < 0 || b < 0 || c < 0 || a > TJN - 2 || b > TJN - 2 || c > TJN - 2)
-            ts.gs.seg(fs.i, fs.j, fs.k, vv, vv + 4, vv + 8);   /* outside the block: to HBM */
-        else
-            cell = (a * TJN + b) * TJN + c;
-    }
-    if (cell < 0)
-        for (int q = 0; q < 12; ++q) vv[q] = 0.0;
+    if (fs.cell < 0)
+        for (int q = 0; q < 12; ++q) fs.v[q] = 0.0;
     int start, len;
     bool head;
-    wave_run(cell, start, len, head);
+    wave_run(fs.cell, start, len, head);
     const int lane = threadIdx.x & 63;
     /* fma(y, 1, x) is x + y rounded once, fma(y, 0, x) is x: one
      * instruction instead of a select of y and an add */
@@ -466,135 +682,220 @@ __device__ static inline void first_run_add(const TileSink &ts, const Grid &g, c
                  m4 = lane - 4 >= start ? 1.0 : 0.0, m8 = lane - 8 >= start ? 1.0 : 0.0;
 #pragma unroll
     for (int q = 0; q < 12; ++q) {
-        double x = vv[q];
+        double x = fs.v[q];
         x = __builtin_fma(row_shr<1>(x), m1, x);
         x = __builtin_fma(row_shr<2>(x), m2, x);
         x = __builtin_fma(row_shr<4>(x), m4, x);
         x = __builtin_fma(row_shr<8>(x), m8, x);
-        vv[q] = x;
+        fs.v[q] = x;
     }
     const bool tail = lane == start + len - 1 || ((lane & 15) == 15 && lane < start + len - 1);
-    if (tail && cell >= 0) ts.lds_add(a, b, c, vv, vv + 4, vv + 8);
+    if (tail && fs.cell >= 0) seg_add(lj, fs.cell >> 8, fs.cell >> 4 & 15, fs.cell & 15, fs.v);
 }
 
-/* Tiled push: persistent workgroups pull 4x4x4-cell tiles (the order's
- * markers by tile-major cell key, read through its permutation) from
- * per-XCD queues, accumulate the tile's J in LDS and flush it to HBM once;
- * every marker is written, with its id and new cell key, to the output
- * buffer at its position in the order, and the per-cell counts of the new
- * positions are kept for the next sort. */
+/* Tiled push: a workgroup of W wavefronts takes work items (a tile's markers
+ * in the order, read through its permutation) with stride = grid size,
+ * stages the tile's E/H nodes in LDS, accumulates the tile's J in an LDS block
+ * and flushes it to HBM once; every marker is written, with its id and new
+ * cell key, to the output buffer at its position in the order, and the
+ * per-cell counts of the new positions are kept for the next sort.
+ *
+ * Laser-foil (8.57 M markers) 600 -> 336 us, 3.3 TB/s of the 128 B per marker
+ * against 4.8 TB/s of a plain copy; 64^3 full box 469 -> 251 us, 64^3 foil
+ * 98 -> 43, 32^3 box 59 -> 45.  The 600 us were gathers from L2 with one batch
+ * in flight, 31 IEEE divisions per marker of which 27 had a divisor known
+ * before (h, 12, tau h h) and a branch per number of face crossings, each
+ * with its own segment code.  Two wavefronts per SIMD (231 VGPRs) measured
+ * 339 us, four (116 spilled) 381; the run sums take 24 us of it, the
+ * flush 4, the crossing loop 2. */
 struct Push64TArgs {
-    Markers64  m, d;           /* current buffer (read through tv.perm), output buffer */
-    F64View    v;
-    PushConsts c;
-    TileView   tv;
-    double    *kin;
-    unsigned  *err;
+    Markers64    m, d;         /* current buffer (read through tv.perm), output buffer */
+    F64View      v;
+    Push64Consts c;
+    TileView     tv;
+    double      *kin;
+    unsigned    *err;
 };
 
-__device__ __forceinline__ static void push64_tiled(const Markers64 &m, const Markers64 &d,
-                                           const F64View &v, const PushConsts &c,
-                                           const TileView &tv, double *kin, unsigned *err,
-                                           const VBlock &bk)
+/* Position min(p, last) of the order: unconditional, so that the loads of a
+ * batch are issued on every path (lanes past the end carry a duplicate). */
+__device__ static inline unsigned perm_at(const int *perm, unsigned p, unsigned last)
 {
-    __shared__ double lj[TJN * TJN * TJN * 3];
-    __shared__ int s_tile;
-    const Grid &g = v.g;
-    const int xcd = bk.x % MPIC_XCDS;
-    double w3[3] = {0, 0, 0};
+    return (unsigned)perm[p < last ? p : last];
+}
+
+/* The markers the tile's loop left: pushed straight from and to HBM by the
+ * general path, after the loop so that its registers are not the loop's. */
+__device__ static inline void push_off_tile(const Push64TArgs &A, const Tile64 &tl, unsigned p,
+                                            unsigned end, double w3[3])
+{
+    if (p >= end) return;
+    const TileView &tv = A.tv;
+    Pending64 q;
+    load_marker(A.m, (unsigned)tv.perm[p], q.k);
+    if (q.k.qm == 0.0f) return;
+    bool on = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const int l = DBL_TO_INT(div_by(q.k.r[a], A.c.pc.h[a], A.c.yh[a], A.c.yl[a])) - tl.c[a];
+        on = on && (unsigned)l < TILE;
+    }
+    if (on) return;
     GlobalSink gs;
-    for (int a = 0; a < 3; ++a) gs.J[a] = v.J[a];
-    gs.g = g;
-    for (;;) {
-        if (threadIdx.x == 0) s_tile = tile_next(tv, xcd);
-        __syncthreads();
-        const int t = s_tile;
-        if (t < 0) break;
+    for (int a = 0; a < 3; ++a) gs.J[a] = A.v.J[a];
+    gs.g = A.v.g;
+    q.p = p;
+    q.valid = true;
+    q.key = -1;
+    if (push_marker(gs, A.v, A.c.pc, q.k.r, q.k.u, q.k.w, q.k.qm, w3, A.err))
+        q.key = cell_key_of(tv, A.v.g, q.k.r);
+    q.ckey = q.key;
+    q.clen = 1;
+    write_back(A.d, tv, q);
+}
+
+template <int W>
+__device__ __forceinline__ static void push64_tiles(const Push64TArgs &A, const VBlock &bk,
+                                                    const VBlock &gd)
+{
+    constexpr int BS = TW * W;                       /* threads of the workgroup */
+    constexpr int NSTG = (TFN3 + BS - 1) / BS;       /* staged nodes per thread and component */
+    __shared__ double lj[TJB];
+    __shared__ double lf[6 * TFN3];
+    const TileView &tv = A.tv;
+    const F64View &v = A.v;
+    const Grid &g = v.g;
+    const int nitems = *tv.nitems;
+    double w3[3] = {0, 0, 0};
+    for (int it = (int)bk.x; it < nitems; it += (int)gd.x) {
+        const int4 work = tv.item[it];
+        const unsigned beg = work.y, end = work.z;
+        const unsigned s0 = perm_at(tv.perm, beg + threadIdx.x, end - 1);
+        unsigned snx = perm_at(tv.perm, beg + BS + threadIdx.x, end - 1);
+        Tile64 tl;
+        tl.t = work.x;
         int t0, t1, t2;
-        tile_coords(tv, t, t0, t1, t2);
-        TileSink ts;
-        ts.gs = gs;
-        ts.lj = lj;
-        ts.o0 = TILE * t0 - 1;
-        ts.o1 = TILE * t1 - 1;
-        ts.o2 = TILE * t2 - 1;
-        for (int q = threadIdx.x; q < TJN * TJN * TJN * 3; q += TPB) lj[q] = 0.0;
-        __syncthreads();
-        const long beg = tv.toff[t], end = tv.toff[t + 1];
-        for (long base = beg; base < end; base += TPB) {
-            const long p = base + threadIdx.x;
-            int key = -1;
-            FirstSeg fs;
-            fs.on = 0;
-            float wf = 0.0f;
-            if (p < end) {
-                const long q = tv.perm[p];
-                double r[3] = {m.x[q], m.y[q], m.z[q]};
-                double u[3] = {m.ux[q], m.uy[q], m.uz[q]};
-                const float qm = m.qm[q], w = m.w[q];
-                const int32_t id = m.id[q];
-                wf = w;
-                int alive = (qm != 0.0f) && push_marker<true>(ts, v, c, r, u, w, qm, w3, err, &fs);
-                if (!alive) {
-                    d.qm[p] = 0.0f;
-                    d.w[p] = 0.0f;
-                } else {
-                    d.x[p] = r[0];
-                    d.y[p] = r[1];
-                    d.z[p] = r[2];
-                    d.ux[p] = u[0];
-                    d.uy[p] = u[1];
-                    d.uz[p] = u[2];
-                    d.w[p] = w;
-                    d.qm[p] = qm;
-                    key = cell_key_of(tv, g, r);
-                }
-                d.id[p] = id;
-                tv.key[p] = key;
-            }
-            first_run_add(ts, g, fs, wf);
-            wave_run_count(tv.count, key);
+        tile_coords(tv, tl.t, t0, t1, t2);
+        tl.c[0] = TILE * t0;
+        tl.c[1] = TILE * t1;
+        tl.c[2] = TILE * t2;
+        tl.s0 = tv.nt[1] * tv.nt[2];
+        tl.s1 = tv.nt[2];
+        tl.edge = false;
+        for (int a = 0; a < 3; ++a) {
+            tl.edge = tl.edge || tl.c[a] < TILE || tl.c[a] + 2 * TILE > g.n[a];
         }
+        __syncthreads();                  /* the previous tile's LDS reads are done */
+        for (int q = threadIdx.x; q < TJB; q += BS) lj[q] = 0.0;
+        Marker64 cur;
+        {
+            /* nodes [c, c + TFN) per axis; those past the last ghost layer
+             * are never read by a gather and are staged as 0 */
+            const long base = gidx(g, tl.c[0], tl.c[1], tl.c[2]);
+            unsigned offs[NSTG];
+            bool ok[NSTG];
+#pragma unroll
+            for (int r = 0; r < NSTG; ++r) {
+                const int rr = (int)threadIdx.x + BS * r;
+                const int a = rr / (TFN * TFN), b = (rr / TFN) % TFN, cc = rr % TFN;
+                ok[r] = rr < TFN3 && tl.c[0] + a <= g.n[0] + 2 && tl.c[1] + b <= g.n[1] + 2 &&
+                        tl.c[2] + cc <= g.n[2] + 2;
+                offs[r] = ok[r] ? (unsigned)((a * g.GY + b) * g.GZ + cc) : 0u;
+            }
+            double st[6][NSTG];
+#pragma unroll
+            for (int comp = 0; comp < 6; ++comp) {
+                const double *F = (comp < 3 ? v.E[comp] : v.H[comp - 3]) + base;
+#pragma unroll
+                for (int r = 0; r < NSTG; ++r) st[comp][r] = F[offs[r]];
+            }
+            load_marker(A.m, s0, cur);
+#pragma unroll
+            for (int comp = 0; comp < 6; ++comp)
+#pragma unroll
+                for (int r = 0; r < NSTG; ++r) {
+                    const int rr = (int)threadIdx.x + BS * r;
+                    if (rr < TFN3) lf[comp * TFN3 + rr] = ok[r] ? st[comp][r] : 0.0;
+                }
+        }
+        /* everything outstanding completes here, so that the loop's waits
+         * only ever concern the prefetch of the batch in flight */
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        unsigned long long off_tile = 0;  /* lanes that met a marker of another cell */
+        Pending64 pend;
+        pend.valid = false;
+        pend.ckey = -1;
+        for (unsigned base = beg; base < end; base += BS) {
+            const unsigned p = base + threadIdx.x;
+            Marker64 nxt;
+            load_marker(A.m, snx, nxt);
+            snx = perm_at(tv.perm, p + 2 * BS, end - 1);
+            write_back(A.d, tv, pend);
+            First64 fs;
+            fs.cell = -1;
+            pend.k = cur;
+            pend.p = p;
+            pend.valid = p < end;
+            pend.key = -1;
+            if (pend.valid && cur.qm != 0.0f)
+                pend.key = push64_marker(pend.k, v, A.c, tv, tl, lf, lj, fs, w3);
+            const bool off = pend.key == OFF_TILE;
+            off_tile |= __ballot(off);
+            if (off) {
+                pend.key = -1;
+                pend.valid = false;
+            }
+            first_run_add(lj, fs);
+            /* count[new key] += run length, once per run of equal new keys */
+            int start, len;
+            bool head;
+            wave_run(pend.key, start, len, head);
+            pend.ckey = head ? pend.key : -1;
+            pend.clen = len;
+            cur = nxt;
+        }
+        write_back(A.d, tv, pend);
+        if (off_tile)
+            for (unsigned base = beg; base < end; base += BS)
+                push_off_tile(A, tl, base + threadIdx.x, end, w3);
         __syncthreads();
         /* flush the tile's J block: one HBM atomic per non-zero node value */
-        for (int q = threadIdx.x; q < TJN * TJN * TJN * 3; q += TPB) {
+        for (int q = threadIdx.x; q < TJB; q += BS) {
             const double val = lj[q];
             if (val == 0.0) continue;
             const int comp = q % 3, node = q / 3;
             const int cc = node % TJN, bb = (node / TJN) % TJN, aa = node / (TJN * TJN);
-            const int i = ts.o0 + aa, j = ts.o1 + bb, k = ts.o2 + cc;
+            const int i = tl.c[0] - 1 + aa, j = tl.c[1] - 1 + bb, k = tl.c[2] - 1 + cc;
             if (i < -2 || j < -2 || k < -2 || i > g.n[0] + 2 || j > g.n[1] + 2 || k > g.n[2] + 2)
                 continue;
             unsafeAtomicAdd(v.J[comp] + gidx(g, i, j, k), val);
         }
-        __syncthreads();
     }
-    block_sum3(w3, kin_slot(kin, bk.x));
+    for (int d = 32; d > 0; d >>= 1)
+        for (int a = 0; a < 3; ++a) w3[a] += __shfl_down(w3[a], d, 64);
+    if ((threadIdx.x & 63) == 0 && (w3[0] != 0.0 || w3[1] != 0.0 || w3[2] != 0.0)) {
+        double *ks = kin_slot(A.kin, bk.x);
+        for (int a = 0; a < 3; ++a) atomicAdd(ks + a, w3[a]);
+    }
 }
 
-template <> struct KernelDef<Push64TArgs> {
-    static constexpr int kBlock = TPB;
+/* W wavefronts per workgroup, a distinct argument type per W. */
+template <int W> struct Push64TArgsW : Push64TArgs {
+};
+
+template <int W> struct KernelDef<Push64TArgsW<W>> {
+    static constexpr int kBlock = TW * W;
     static constexpr int kWaves = 3;   /* register budget for 3 wavefronts per SIMD */
-    __device__ __forceinline__ static void body(const Push64TArgs &a, VBlock b, VBlock)
+    __device__ __forceinline__ static void body(const Push64TArgsW<W> &a, VBlock b, VBlock gd)
     {
-        push64_tiled(a.m, a.d, a.v, a.c, a.tv, a.kin, a.err, b);
+        push64_tiles<W>(a, b, gd);
     }
 };
 
-/* Workgroups of the persistent push that fit on one CU at once. */
-int push64_blocks_per_cu(void)
-{
-    int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_one_w<Push64TArgs>, TPB, 0) !=
-            hipSuccess ||
-        nb < 1)
-        nb = 1;
-    return nb;
-}
-
 int launch_push64_tiled(hipStream_t s, const Markers64 &m, const Markers64 &dst,
-                        const Fields64 &f, const Grid &g, const PushConsts &c,
-                        const TileView &tv, double *kin, unsigned *err, int nblocks)
+                        const Fields64 &f, const Grid &g, const PushConsts &pc,
+                        const TileView &tv, double *kin, unsigned *err, int nblocks, int waves)
 {
     F64View v;
     for (int a = 0; a < 3; ++a) {
@@ -603,8 +904,17 @@ int launch_push64_tiled(hipStream_t s, const Markers64 &m, const Markers64 &dst,
         v.J[a] = f.J[a];
     }
     v.g = g;
-    Push64TArgs a = {m, dst, v, c, tv, kin, err};
-    return launch_def(s, a, (unsigned)nblocks);
+    Push64Consts c;
+    c.pc = pc;
+    for (int a = 0; a < 3; ++a) {
+        c.yh[a] = 1.0 / g.h[a];
+        c.yl[a] = fma(-g.h[a], c.yh[a], 1.0) / g.h[a];
+        c.cj[a] = g.h[a] / g.tau;
+    }
+    c.vol = g.h[0] * g.h[1] * g.h[2];
+    const Push64TArgs a = {m, dst, v, c, tv, kin, err};
+    if (waves == 8) return launch_def(s, Push64TArgsW<8>{a}, (unsigned)nblocks);
+    return launch_def(s, Push64TArgsW<4>{a}, (unsigned)nblocks);
 }
 
 /* CIC charge density of the live markers, source/core/plasma_rho.c:160-173:

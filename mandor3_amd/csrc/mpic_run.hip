@@ -127,9 +127,8 @@ struct mpic_run {
     TileView      tv;
     unsigned long long *scanw;  /* the tile scan's published words and sequence number */
     int           parity;     /* tv.nmark[parity] = markers in the current order */
-    int           push_blocks;  /* FP64: resident workgroups of the persistent push */
-    int           tile_blocks;  /* FP32: workgroups of the tile push (work items taken in turn) */
-    int           tile_waves;   /* FP32: wavefronts per workgroup of the tile push */
+    int           tile_blocks;  /* workgroups of the tile push (work items taken in turn) */
+    int           tile_waves;   /* wavefronts per workgroup of the tile push */
     int           gather_blocks;/* FP32: workgroups of the J gather */
     long          items_cap;    /* work items (and FP32 J blocks) the buffers hold */
     int           ncu;          /* compute units of the device */
@@ -534,11 +533,10 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     MPIC_CHECK(hipMalloc(&tv.titem, sizeof(int2) * tv.ntiles));
     MPIC_CHECK(hipMemsetAsync(tv.titem, 0, sizeof(int2) * tv.ntiles, r->stream));
     if (r->fp32) MPIC_CHECK(hipMalloc(&r->tj, sizeof(float) * TJB * (size_t)r->items_cap));
-    MPIC_CHECK(hipMalloc(&tv.nactive, sizeof(int) * (4 + MPIC_XCDS)));
-    tv.queue = tv.nactive + 1;
-    tv.nmark = tv.nactive + 1 + MPIC_XCDS;
-    tv.nitems = tv.nactive + 3 + MPIC_XCDS;
-    MPIC_CHECK(hipMemsetAsync(tv.nactive, 0, sizeof(int) * (4 + MPIC_XCDS), r->stream));
+    MPIC_CHECK(hipMalloc(&tv.nactive, sizeof(int) * 4));
+    tv.nmark = tv.nactive + 1;
+    tv.nitems = tv.nactive + 3;
+    MPIC_CHECK(hipMemsetAsync(tv.nactive, 0, sizeof(int) * 4, r->stream));
     /* the tile scan's published words: zero never matches a scan's tag */
     MPIC_CHECK(hipMalloc(&r->scanw, sizeof(unsigned long long) * tile_scan_words(tv.ntiles)));
     MPIC_CHECK(hipMemsetAsync(r->scanw, 0, sizeof(unsigned long long) * tile_scan_words(tv.ntiles),
@@ -548,11 +546,6 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
         int ncu = 256;
         hipDeviceProp_t prop;
         if (hipGetDeviceProperties(&prop, r->dev) == hipSuccess) ncu = prop.multiProcessorCount;
-        /* exactly the resident workgroups of the persistent push (extra ones
-         * only arrive once the tile queues are drained), and no more than
-         * the tiles: a workgroup pushes whole tiles */
-        r->push_blocks = ncu * push64_blocks_per_cu();
-        if (r->push_blocks > tv.ntiles) r->push_blocks = tv.ntiles;
         /* The tile push: a workgroup per work item up to 16 per CU (it takes
          * items with stride = grid size), 4 wavefronts each; 8 on a box of
          * at most two tiles per CU, where every wavefront is resident
@@ -566,7 +559,7 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
         r->gather_blocks = 16 * ncu;
         r->ncu = ncu;
         const char *e = getenv("MPIC_PUSH_BLOCKS");
-        if (e && atoi(e) > 0) r->push_blocks = r->tile_blocks = atoi(e);
+        if (e && atoi(e) > 0) r->tile_blocks = atoi(e);
         const char *w = getenv("MPIC_TILE_WAVES");
         if (w && (atoi(w) == 1 || atoi(w) == 2 || atoi(w) == 4 || atoi(w) == 8))
             r->tile_waves = atoi(w);
@@ -1876,8 +1869,7 @@ extern "C" int mpic_push_deposit(mpic_run_t *r)
         TRY(launch_jgather32(r->stream, r->f32, r->g, r->tv, r->tj, r->gather_blocks));
     } else if (r->tiled) {
         TRY(launch_push64_tiled(r->stream, r->m, r->mbuf[r->cur ^ 1], r->f, r->g, r->pc, r->tv,
-                                r->dkin, r->derr,
-                                r->push_blocks));
+                                r->dkin, r->derr, r->tile_blocks, r->tile_waves));
     } else {
         TRY(launch_push64(r->stream, r->m, r->n, r->f, r->g, r->pc, r->dkin, 0, r->derr));
     }
@@ -2384,24 +2376,24 @@ static int ensemble_build(mpic_run *const *runs, int nruns, Ensemble **out)
     std::vector<Recorder> recs[2];
     recs[0].resize(nruns);
     recs[1].resize(nruns);
-    /* The FP64 tiled push of a run in the fused launch takes 2 workgroups
-     * per CU (at most its tiles), not the 3 that fit: the runs' workgroups
-     * then overlap more in the one launch (64-run scan ensemble: 7.30 ms per
-     * FP64 step against 7.78 ms; a share of the resident workgroups in
-     * proportion to the run's markers measured 8.07 ms). */
-    std::vector<int> own_blocks(nruns);
+    /* Launches fuse by kind, and the push's kind carries its wavefronts per
+     * workgroup: where small boxes (8 by their own rule) meet larger ones
+     * (4), all take 4, in one launch. */
+    std::vector<int> own_waves(nruns);
+    bool mixed = false;
     for (int q = 0; q < nruns; ++q) {
-        mpic_run *r = runs[q];
-        own_blocks[q] = r->push_blocks;
-        if (!r->fp32 && r->tiled && r->push_blocks > 2 * r->ncu) r->push_blocks = 2 * r->ncu;
+        own_waves[q] = runs[q]->tile_waves;
+        mixed = mixed || own_waves[q] != runs[0]->tile_waves;
     }
+    for (int q = 0; q < nruns && mixed; ++q)
+        if (runs[q]->tile_waves == 8) runs[q]->tile_waves = 4;
     for (int q = 0; q < nruns && rc == MPIC_OK; ++q) {
         Recorder two[2];
         rc = record_steps(runs[q], two);
         recs[0][q] = std::move(two[0]);
         recs[1][q] = std::move(two[1]);
     }
-    for (int q = 0; q < nruns; ++q) runs[q]->push_blocks = own_blocks[q];
+    for (int q = 0; q < nruns; ++q) runs[q]->tile_waves = own_waves[q];
     std::vector<std::vector<const LaunchRec *>> seq[2];
     std::vector<FusedLaunch> fl[2];
     size_t bytes = 0;
@@ -2617,14 +2609,14 @@ extern "C" int mpic_autotune(mpic_run_t *r, int steps, int *chosen)
     MPIC_CHECK(hipSetDevice(r->dev));
     if (!r->fp32 || !r->tiled) {
         if (chosen) {
-            chosen[0] = r->push_blocks;
+            chosen[0] = r->tile_blocks;
             chosen[1] = 1;
             chosen[2] = 0;
         }
         return MPIC_OK;
     }
     const int chms[3] = {0, 2048, 1024};
-    const int wavess[4] = {1, 2, 4, 8};
+    const int wavess[3] = {1, 2, 4};
     const char *verbose = getenv("MPIC_AUTOTUNE_VERBOSE");
     int best_nb = r->tile_blocks, best_w = r->tile_waves, best_chm = r->tv.chm;
     double best_ms = 1e300;
@@ -2636,7 +2628,7 @@ extern "C" int mpic_autotune(mpic_run_t *r, int steps, int *chosen)
         r->tv.chm = chm;
         TRY(sort_pass(r, 1));
         TRY(advance_timed(r, 1));          /* untimed: first launches of the new lists */
-        for (int wi = 0; wi < 4; ++wi) {
+        for (int wi = 0; wi < 3; ++wi) {
             const int w = wavess[wi];
             for (int per_cu = 4; per_cu <= 64; per_cu *= 2) {
                 int nb = per_cu * r->ncu / w;

@@ -1,6 +1,6 @@
 /*
  * mpic_tiles.h -- tile-major cell keys, the per-step counting sort and the
- * per-XCD tile queues shared by the FP64 and FP32 push kernels.
+ * work items shared by the FP64 and FP32 push kernels.
  *
  * The grid of cells is cut into 4x4x4-cell tiles; a marker's key is
  *   key = tile * 64 + (li * 4 + lj) * 4 + lk
@@ -29,11 +29,10 @@ struct TileView {
                               * current buffer (nmark[parity] of them; tiled runs) */
     int *active;             /* [ntiles] tiles holding markers, in tile order */
     int *nactive;            /* [1] */
-    int *queue;              /* [MPIC_XCDS] work counters */
     int *nmark;              /* [2] markers in the current / next order */
-    /* Work items of the FP32 push: an active tile's markers split evenly
-     * into ceil(count / chm) items of at most chm markers (chm = 0: one
-     * item per active tile). */
+    /* Work items of the push: an active tile's markers, in the FP32 form split
+     * evenly into ceil(count / chm) items of at most chm markers (chm = 0:
+     * one item per active tile). */
     int  chm;
     int4 *item;              /* [item capacity] work items in tile order: tile, first and last + 1
                               * position in the order (one load tells a workgroup its work: a
@@ -74,25 +73,6 @@ __device__ static inline int cell_key_of(const TileView &tv, const Grid &g, cons
     return cell_key_ijk(tv, g, i, j, k);
 }
 
-/* Next active tile for a workgroup of XCD 'xcd'; the active list is split
- * into one contiguous range per XCD (neighbouring tiles share an L2), and
- * a workgroup whose range is drained steals from the next XCDs.  Returns -1
- * when every range is drained, so every workgroup exits. */
-__device__ static inline int tile_next(const TileView &tv, int xcd)
-{
-    const int na = *tv.nactive;
-    for (int d = 0; d < MPIC_XCDS; ++d) {
-        const int x = (xcd + d) % MPIC_XCDS;
-        const int lo = (int)((long)na * x / MPIC_XCDS), hi = (int)((long)na * (x + 1) / MPIC_XCDS);
-        if (lo >= hi) continue;
-        if (lo + __hip_atomic_load(tv.queue + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= hi)
-            continue;                        /* drained: no contended atomic on the way out */
-        const int q = atomicAdd(tv.queue + x, 1);
-        if (lo + q < hi) return tv.active[lo + q];
-    }
-    return -1;
-}
-
 /* Wave-level run detection on a wave64: lanes holding equal keys in a row
  * form a run; returns (start lane, length) of the caller's run. */
 __device__ static inline void wave_run(int key, int &start, int &len, bool &head)
@@ -129,8 +109,7 @@ int launch_scatter64(hipStream_t s, const Markers64 &src, const Markers64 &dst, 
                      const TileView &tv, int parity);
 int launch_push64_tiled(hipStream_t s, const Markers64 &m, const Markers64 &dst,
                         const Fields64 &f, const Grid &g, const PushConsts &c,
-                        const TileView &tv, double *kin, unsigned *err, int nblocks);
-int push64_blocks_per_cu(void);
+                        const TileView &tv, double *kin, unsigned *err, int nblocks, int waves);
 int launch_counts_natural(hipStream_t s, const TileView &tv, const Grid &g, int32_t *out);
 
 /* J block of one tile: nodes [4t-1, 4t+5] per axis, xyz interleaved. */

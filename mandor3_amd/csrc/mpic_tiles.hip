@@ -4,8 +4,8 @@
  *
  * Per step: the push kernel writes each marker's new key and bumps
  * count[key] once per run of equal keys in a wavefront; the scan turns the
- * counts into per-key offsets, builds the list of non-empty tiles and resets
- * the tile queues; the rank pass gives every live marker its slot
+ * counts into per-key offsets and builds the lists of non-empty tiles and of
+ * work items; the rank pass gives every live marker its slot
  * (cursor[key] reserved once per run) and records the marker's position in
  * the next order's permutation, dropping deleted markers.  The next push
  * reads its markers through that permutation and writes them to the other
@@ -199,7 +199,6 @@ __device__ static inline void scan_pass(const ScanArgs &A, const VBlock &bk)
             *tv.nactive = na;
             *tv.nitems = ni;
             tv.nmark[A.parity_next] = tot;
-            for (int q = 0; q < MPIC_XCDS; ++q) tv.queue[q] = 0;
             *A.seq = seq + 1;
         }
     }
