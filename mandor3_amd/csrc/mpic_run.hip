@@ -548,14 +548,15 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
         if (hipGetDeviceProperties(&prop, r->dev) == hipSuccess) ncu = prop.multiProcessorCount;
         /* The tile push: a workgroup per work item up to 16 per CU (it takes
          * items with stride = grid size), 4 wavefronts each; 8 on a box of
-         * at most two tiles per CU, where every wavefront is resident
-         * at once and the time is that of one wavefront's serial batches.
-         * Push in us with 1 / 2 / 4 / 8 wavefronts: 32^3 box, 512 tiles
-         * 59 / 39 / 26 / 24; 12^3 box 55 / 35 / 22 / 17; 64^3 foil
+         * at most two tiles per CU (FP64 form: one), where every wavefront is
+         * resident at once and the time is that of one wavefront's serial
+         * batches.  FP32 push in us with 1 / 2 / 4 / 8 wavefronts: 32^3 box,
+         * 512 tiles 59 / 39 / 26 / 24; 12^3 box 55 / 35 / 22 / 17; 64^3 foil
          * 45 / 34 / 26 / 28; 64^3 full box 161 / 141 / 127 / 138; laser-foil
-         * 202 / 191 / 165 / 170. */
+         * 202 / 191 / 165 / 170.  FP64 with 4 / 8: 32^3 box 42 / 45, 12^3 box
+         * 31 / 23, 64^3 foil 43 / 64. */
         r->tile_blocks = 16 * ncu < r->items_cap ? 16 * ncu : (int)r->items_cap;
-        r->tile_waves = tv.ntiles <= 2 * ncu ? 8 : 4;
+        r->tile_waves = tv.ntiles <= (r->fp32 ? 2 : 1) * ncu ? 8 : 4;
         r->gather_blocks = 16 * ncu;
         r->ncu = ncu;
         const char *e = getenv("MPIC_PUSH_BLOCKS");
