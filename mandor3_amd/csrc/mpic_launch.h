@@ -265,4 +265,21 @@ static int launch_pair(hipStream_t s, const A &a, dim3 ga, const B &b, dim3 gb)
     return launch_def(s, p, na + nb);
 }
 
+/* Three bodies with no order between them; C's grid may be empty. */
+template <class A, class B, class C>
+static int launch_three(hipStream_t s, const A &a, dim3 ga, const B &b, dim3 gb, const C &c,
+                        dim3 gc)
+{
+    const unsigned na = ga.x * ga.y * ga.z, nb = gb.x * gb.y * gb.z;
+    if (na == 0) return launch_pair(s, b, gb, c, gc);
+    if (nb == 0) return launch_pair(s, a, ga, c, gc);
+    PairArgs<A, B> p;
+    p.a = a;
+    p.b = b;
+    p.ga = {ga.x, ga.y, ga.z};
+    p.gb = {gb.x, gb.y, gb.z};
+    p.na = na;
+    return launch_pair(s, p, dim3(na + nb), c, gc);
+}
+
 #endif

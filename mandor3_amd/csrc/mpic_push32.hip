@@ -651,123 +651,6 @@ template <int W> struct KernelDef<Push32ArgsW<W>> {
     }
 };
 
-/* Range of tiles u (along one axis) whose J block [4u-1, 4u+5] holds node i. */
-__device__ static inline void covering(int i, int nt, int &lo, int &hi)
-{
-    lo = (i - 2 + 1024) / 4 - 256;          /* ceil((i - 5) / 4) = floor((i - 2) / 4), i >= -1022 */
-    hi = (i + 1 + 1024) / 4 - 256;          /* floor((i + 1) / 4) */
-    lo = lo < 0 ? 0 : lo;
-    hi = hi > nt - 1 ? nt - 1 : hi;
-}
-
-/* J += sum of the item blocks of the tiles covering each node, in FP64.
- * Every node of an active tile's block is written once, by the first active
- * tile (in tile order) whose block holds it; the sum runs over the covering
- * tiles in tile order and over each tile's items in order, so the gather
- * adds in a fixed order (what a block holds follows the device order of
- * the tile's markers, which the sort's slot reservation by atomics does not
- * fix from run to run).  One thread per node and all three
- * components: a node lies in at most 2 blocks per axis, and the first item
- * of each of the (at most 8) covering tiles is loaded before any is added,
- * so the gather waits for one memory latency per node, not one per block. */
-#define TJN3 (TJN * TJN * TJN)
-struct JGatherArgs {
-    F32View      v;
-    TileView     tv;
-    const float *tj;
-};
-
-__device__ __forceinline__ static void jgather32(const F32View &v, const TileView &tv, const float *tj,
-                                        const VBlock &bk, const VBlock &gd)
-{
-    __shared__ int nfirst[27], nitem[27];    /* items of the 3x3x3 tiles around t (0: none) */
-    const Grid &g = v.g;
-    const int nact = *tv.nactive;
-    for (int sl = (int)bk.x; sl < nact; sl += (int)gd.x) {
-        const int t = tv.active[sl];
-        int t0, t1, t2;
-        tile_coords(tv, t, t0, t1, t2);
-        __syncthreads();
-        if (threadIdx.x < 27) {
-            const int ux = t0 - 1 + threadIdx.x / 9, uy = t1 - 1 + (threadIdx.x / 3) % 3,
-                      uz = t2 - 1 + threadIdx.x % 3;
-            const bool in = ux >= 0 && uy >= 0 && uz >= 0 && ux < tv.nt[0] && uy < tv.nt[1] &&
-                            uz < tv.nt[2];
-            const int2 ti = in ? tv.titem[(ux * tv.nt[1] + uy) * tv.nt[2] + uz] : make_int2(0, 0);
-            nfirst[threadIdx.x] = ti.x;
-            nitem[threadIdx.x] = ti.y;
-        }
-        __syncthreads();
-        /* nodes in reverse order: the nodes an interior tile owns (block
-         * positions 3..6 along each axis, the others belong to the tiles
-         * below) all fall in the first pass of the workgroup, so a tile
-         * inside the plasma waits on memory once */
-        for (int pass = threadIdx.x; pass < TJN3; pass += TPB) {
-            const int node = TJN3 - 1 - pass;
-            const int cc = node % TJN, bb = (node / TJN) % TJN, aa = node / (TJN * TJN);
-            const int i = TILE * t0 - 1 + aa, j = TILE * t1 - 1 + bb, k = TILE * t2 - 1 + cc;
-            if (i < -2 || j < -2 || k < -2 || i > g.n[0] + 2 || j > g.n[1] + 2 || k > g.n[2] + 2)
-                continue;
-            int xl, xh, yl, yh, zl, zh;
-            covering(i, tv.nt[0], xl, xh);
-            covering(j, tv.nt[1], yl, yh);
-            covering(k, tv.nt[2], zl, zh);
-            /* the covering tiles (2 per axis at most), in tile order */
-            int nb[8], off[8];
-            bool use[8];
-            int own = -1;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int ux = xl + (q >> 2), uy = yl + ((q >> 1) & 1), uz = zl + (q & 1);
-                const bool inr = ux <= xh && uy <= yh && uz <= zh;
-                const int b = inr ? ((ux - t0 + 1) * 3 + (uy - t1 + 1)) * 3 + (uz - t2 + 1) : 13;
-                use[q] = inr && nitem[b] > 0;
-                nb[q] = b;
-                const int a = i - (TILE * ux - 1), bq = j - (TILE * uy - 1), cz = k - (TILE * uz - 1);
-                off[q] = use[q] ? ((a * TJN + bq) * TJN + cz) * 3 : 0;
-                if (use[q] && own < 0) own = (ux * tv.nt[1] + uy) * tv.nt[2] + uz;
-            }
-            if (own != t) continue;
-            const long o = gidx(g, i, j, k);
-            const double J0 = v.J[0][o], J1 = v.J[1][o], J2 = v.J[2][o];
-            float f[8][3];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const float *blk = tj + (long)(use[q] ? nfirst[nb[q]] : 0) * TJB + off[q];
-                f[q][0] = blk[0];
-                f[q][1] = blk[1];
-                f[q][2] = blk[2];
-            }
-            double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                if (!use[q]) continue;
-                s0 += (double)f[q][0];
-                s1 += (double)f[q][1];
-                s2 += (double)f[q][2];
-                const int n_it = nitem[nb[q]];
-                for (int w = 1; w < n_it; ++w) {          /* tiles split into several items */
-                    const float *blk = tj + (long)(nfirst[nb[q]] + w) * TJB + off[q];
-                    s0 += (double)blk[0];
-                    s1 += (double)blk[1];
-                    s2 += (double)blk[2];
-                }
-            }
-            v.J[0][o] = J0 + s0;
-            v.J[1][o] = J1 + s1;
-            v.J[2][o] = J2 + s2;
-        }
-    }
-}
-
-template <> struct KernelDef<JGatherArgs> {
-    static constexpr int kBlock = TPB;
-    __device__ __forceinline__ static void body(const JGatherArgs &a, VBlock b, VBlock gd)
-    {
-        jgather32(a.v, a.tv, a.tj, b, gd);
-    }
-};
-
 int launch_push32(hipStream_t s, const Markers32 &m, const Markers32 &dst, const Fields32 &f,
                   const Grid &g, const PushConsts &pc, const float *qm, const TileView &tv,
                   float *tj, double *kin, int nblocks, int waves)
@@ -798,20 +681,6 @@ int launch_push32(hipStream_t s, const Markers32 &m, const Markers32 &dst, const
         mpic_set_error("launch_push32: %d wavefronts per tile (1, 2, 4 or 8)", waves);
         return MPIC_ERR_ARG;
     }
-}
-
-int launch_jgather32(hipStream_t s, const Fields32 &f, const Grid &g, const TileView &tv,
-                     const float *tj, int nblocks)
-{
-    F32View v;
-    for (int a = 0; a < 3; ++a) {
-        v.E[a] = f.E[a];
-        v.H[a] = f.H[a];
-        v.J[a] = f.J[a];
-    }
-    v.g = g;
-    JGatherArgs a = {v, tv, tj};
-    return launch_def(s, a, (unsigned)nblocks);
 }
 
 /* Keys and counts of the current buffer's first nmark[parity] markers

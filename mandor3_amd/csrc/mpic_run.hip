@@ -10,6 +10,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -122,6 +123,7 @@ struct mpic_run {
     Markers64     m;          /* current marker order */
     Markers64     mbuf[2];    /* double buffer of the per-step sort */
     int           cur;        /* m == mbuf[cur] */
+    int           hsw;        /* the loop body's swaps of H and Hc, modulo 2 */
     long          n, cap;     /* n: markers loaded (upper bound of the live count) */
     int           tiled;      /* 1: sorted tiled push (default), 0: untiled push */
     TileView      tv;
@@ -161,7 +163,7 @@ struct mpic_run {
     int           use_graphs; /* mpic_advance replays captured steps */
     int           graphs_ok;  /* exec[] match the current launch topology */
     hipGraphExec_t exec[2];   /* one step from each of the two marker-buffer parities */
-    int           exec_parity;     /* parity at which exec[0] was captured */
+    int           exec_phase;      /* the run's phase when exec[0] was captured */
     int           ev_steps;   /* timed steps of the last mpic_advance */
     double       *dnode;      /* node values of the Tecplot records, 3 (n+1)^3 doubles */
     int          *dprobe;     /* probe nodes, 3 ints each */
@@ -175,7 +177,6 @@ struct mpic_run {
     std::vector<long>   ring_step;  /* step whose row a slot holds (-1: none) */
     std::vector<double> ring_time;  /* Time at the start of that step */
     int           capturing;  /* step_body is being recorded into graphs, not run */
-    int           jclear_done;  /* the H half step cleared J and the temperature sums */
     double        vsp;        /* VSP convolution weight alpha (1: off) */
     long          topo;       /* bumped whenever the launch sequence of a step changes */
 };
@@ -533,10 +534,16 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     MPIC_CHECK(hipMalloc(&tv.titem, sizeof(int2) * tv.ntiles));
     MPIC_CHECK(hipMemsetAsync(tv.titem, 0, sizeof(int2) * tv.ntiles, r->stream));
     if (r->fp32) MPIC_CHECK(hipMalloc(&r->tj, sizeof(float) * TJB * (size_t)r->items_cap));
-    MPIC_CHECK(hipMalloc(&tv.nactive, sizeof(int) * 4));
+    MPIC_CHECK(hipMalloc(&tv.nactive, sizeof(int) * 6));
     tv.nmark = tv.nactive + 1;
     tv.nitems = tv.nactive + 3;
+    tv.xr = tv.nactive + 4;
     MPIC_CHECK(hipMemsetAsync(tv.nactive, 0, sizeof(int) * 4, r->stream));
+    {
+        /* a tiled run without markers pushes nothing */
+        const int xr[2] = {r->tiled ? 0 : -2, r->tiled ? -1 : g.n[0] + 2};
+        MPIC_CHECK(hipMemcpy(tv.xr, xr, sizeof(xr), hipMemcpyHostToDevice));
+    }
     /* the tile scan's published words: zero never matches a scan's tag */
     MPIC_CHECK(hipMalloc(&r->scanw, sizeof(unsigned long long) * tile_scan_words(tv.ntiles)));
     MPIC_CHECK(hipMemsetAsync(r->scanw, 0, sizeof(unsigned long long) * tile_scan_words(tv.ntiles),
@@ -583,7 +590,7 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
         MPIC_CHECK(hipMalloc(&r->djr, sizeof(full)));
         MPIC_CHECK(hipMemcpy(r->djr, full, sizeof(full), hipMemcpyHostToDevice));
     }
-    r->nparts = h_update_blocks(g, cfg->precision == MPIC_FP32_SPLIT);
+    r->nparts = h_full_blocks(g, cfg->precision == MPIC_FP32_SPLIT);
     MPIC_CHECK(hipMalloc(&r->dpart, sizeof(double) * 2 * r->nparts));
     MPIC_CHECK(hipMalloc(&r->dring, sizeof(double) * 5 * DIAG_RING));
     r->ring_step.assign(DIAG_RING, -1);
@@ -1505,6 +1512,21 @@ generic:
 template <class T>
 static int init_ghosts(mpic_run *r, T *const E[3], T *const H[3]);
 
+/* Where the run's double buffers stand: a loop step toggles all three bits
+ * (a tiled run's marker buffer and order, and the H buffers), stage calls
+ * and sorts some of them.  A step's launch arguments depend on it. */
+static int phase_of(const mpic_run *r) { return r->cur | r->parity << 1 | r->hsw << 2; }
+
+/* The H buffer that the loop body's update wrote becomes the current one. */
+static void swap_fields(mpic_run *r)
+{
+    for (int c = 0; c < 3; ++c) {
+        std::swap(r->f32.H[c], r->f32.Hc[c]);
+        std::swap(r->f.H[c], r->f.Hc[c]);
+    }
+    r->hsw ^= 1;
+}
+
 /* The sorted array becomes the current one. */
 static void swap_markers(mpic_run *r)
 {
@@ -1782,47 +1804,35 @@ static int laser_E(mpic_run *r, T *Ey, T *Ez, const Box &tu)
     return MPIC_OK;
 }
 
-/* em_HHalfStep; with 'part' the H update also writes em_energy's partial
- * sums of E and of the H it leaves (H^n). */
-static int h_half(mpic_run *r, double *part, bool with_clear = false);
+/* TFSF_preHStep in record mode, source/core/em.c:92 */
+static int tfsf_record(mpic_run *r)
+{
+    if (!r->trec.on) return MPIC_OK;
+    const TfsfRec &tr = r->trec;
+    if (r->fp32)
+        return launch_tfsf_record<float>(r->stream, r->f32.E, r->f32.H, r->g, tr.fe, tr.fh, tr.maxvol,
+                                         tr.dfac, tr.dbuf, r->dstep, (int)tr.step0, tr.cap);
+    return launch_tfsf_record<double>(r->stream, r->f.E, r->f.H, r->g, tr.fe, tr.fh, tr.maxvol,
+                                      tr.dfac, tr.dbuf, r->dstep, (int)tr.step0, tr.cap);
+}
 
 extern "C" int mpic_em_h_half(mpic_run_t *r)
 {
     if (!r) return MPIC_ERR_ARG;
-    return h_half(r, nullptr);
-}
-
-/* The J clear of the push that follows the H half step; with_clear runs it
- * in the H update's launch (nothing between them reads or writes J). */
-static int h_half(mpic_run *r, double *part, bool with_clear)
-{
     TRY(check_stage(r, 0));
     MPIC_CHECK(hipSetDevice(r->dev));
     TRY(laser_tables(r, 1));
-    if (r->trec.on) {                    /* TFSF_preHStep in record mode, source/core/em.c:92 */
-        const TfsfRec &tr = r->trec;
-        if (r->fp32)
-            TRY(launch_tfsf_record<float>(r->stream, r->f32.E, r->f32.H, r->g, tr.fe, tr.fh, tr.maxvol,
-                                          tr.dfac, tr.dbuf, r->dstep, (int)tr.step0, tr.cap));
-        else
-            TRY(launch_tfsf_record<double>(r->stream, r->f.E, r->f.H, r->g, tr.fe, tr.fh, tr.maxvol,
-                                           tr.dfac, tr.dbuf, r->dstep, (int)tr.step0, tr.cap));
-    }
+    TRY(tfsf_record(r));
     /* cap_cacheEH: cap H, walls on cap H, cap E, walls on cap E.  Sources
      * never reach the cap layer (checked in mpic_add_laser). */
     FCALL(launch_cap_H, r->g, r->updH);
+    for (FaceOp &op : r->bcH)            /* H and Hc swap in loop steps */
+        for (int c = 0; c < 3; ++c) op.X[c] = r->fp32 ? (void *)r->f32.Hc[c] : (void *)r->f.Hc[c];
     TRY(walls_on(r, r->bcH));
     FCALL(launch_cap_E, r->g, r->updE);
     TRY(walls_on(r, r->bcE));
     /* em_HSmallStep + cap_flushHalfH */
-    if (with_clear) {
-        FCALL(launch_h_update_jclear, r->g, r->flH, 0, part, r->jp.J[0], r->dkin, r->djr,
-              r->dstep, r->tiled ? r->tv.active : nullptr, r->tiled ? r->tv.nactive : nullptr,
-              r->tiled ? r->tv.nt[1] * r->tv.nt[2] : 1, r->tiled ? 0 : 1);
-        r->jclear_done = 1;
-    } else {
-        FCALL(launch_h_update, r->g, r->flH, 0, part);
-    }
+    FCALL(launch_h_update, r->g, r->flH, 0);
     r->stage = 1;
     return MPIC_OK;
 }
@@ -1848,36 +1858,34 @@ static int record(mpic_run *r, int k)
     return MPIC_OK;
 }
 
+/* The push and its deposit, reading H from f / f32. */
+static int push(mpic_run *r, const Fields32 &f32, const Fields64 &f)
+{
+    if (r->timed >= 0) TRY(record(r, 1));
+    if (r->fp32)
+        TRY(launch_push32(r->stream, r->m32, r->m32buf[r->cur ^ 1], f32, r->g, r->pc, r->qm, r->tv,
+                          r->tj, r->dkin, r->tile_blocks, r->tile_waves));
+    else if (r->tiled)
+        TRY(launch_push64_tiled(r->stream, r->m, r->mbuf[r->cur ^ 1], f, r->g, r->pc, r->tv,
+                                r->dkin, r->derr, r->tile_blocks, r->tile_waves));
+    else
+        TRY(launch_push64(r->stream, r->m, r->n, f, r->g, r->pc, r->dkin, 0, r->derr));
+    if (r->timed >= 0) TRY(record(r, 2));
+    return MPIC_OK;
+}
+
 extern "C" int mpic_push_deposit(mpic_run_t *r)
 {
     if (!r) return MPIC_ERR_ARG;
     TRY(check_stage(r, 1));
     MPIC_CHECK(hipSetDevice(r->dev));
-    /* J (the planes the last deposit wrote) and the temperature sums: a
-     * kernel, not a memset (the step may be replayed from a graph), unless
-     * the H half step's launch cleared them */
-    if (!r->jclear_done)
-        TRY(launch_jclear(r->stream, r->jp.J[0], r->g, r->dkin, r->djr, r->dstep,
-                          r->tiled ? r->tv.active : nullptr, r->tiled ? r->tv.nactive : nullptr,
-                          r->tiled ? r->tv.nt[1] * r->tv.nt[2] : 1, r->tiled ? 0 : 1));
-    r->jclear_done = 0;
-    if (r->timed >= 0) TRY(record(r, 1));
-    if (r->fp32) {
-        TRY(launch_push32(r->stream, r->m32, r->m32buf[r->cur ^ 1], r->f32, r->g, r->pc, r->qm,
-                          r->tv, r->tj, r->dkin,
-                          r->tile_blocks, r->tile_waves));
-        if (r->timed >= 0) TRY(record(r, 2));
-        TRY(launch_jgather32(r->stream, r->f32, r->g, r->tv, r->tj, r->gather_blocks));
-    } else if (r->tiled) {
-        TRY(launch_push64_tiled(r->stream, r->m, r->mbuf[r->cur ^ 1], r->f, r->g, r->pc, r->tv,
-                                r->dkin, r->derr, r->tile_blocks, r->tile_waves));
-    } else {
-        TRY(launch_push64(r->stream, r->m, r->n, r->f, r->g, r->pc, r->dkin, 0, r->derr));
-    }
-    if (r->timed >= 0) {
-        if (!r->fp32) TRY(record(r, 2));
-        TRY(record(r, 3));
-    }
+    /* J (the planes the last deposit wrote) and the kinetic sums: a kernel,
+     * not a memset (the step may be replayed from a graph) */
+    TRY(launch_jclear(r->stream, r->jp.J[0], r->g, r->dkin, r->djr, r->dstep, r->tv.xr,
+                      r->tiled ? 0 : 1));
+    TRY(push(r, r->f32, r->f));
+    if (r->fp32)
+        TRY(launch_jgather32(r->stream, r->jp, r->g, r->tv, r->tj, r->gather_blocks));
     /* per-step marker sort by cell (keys written by the push) */
     if (r->tiled) TRY(sort_pass(r, 0));
     return MPIC_OK;
@@ -1899,22 +1907,12 @@ extern "C" int mpic_temperature(mpic_run_t *r, double *WTx, double *WTy, double 
     return MPIC_OK;
 }
 
-/* The H step; with_fold also runs the y and z J folds in the H update's
- * launch (the H step neither reads nor writes J) and then the VSP sweep,
- * the rest of mpic_j_finish after its x folds. */
-static int h_step(mpic_run *r, bool with_fold)
+/* The sources em_HStep adds to H after the update: the TFSF interface
+ * (TFSF_postHStep, source/core/em.c:125) and the lasers not added by the
+ * update itself. */
+static int h_sources(mpic_run *r, bool laser_done)
 {
-    TRY(check_stage(r, 1));
-    MPIC_CHECK(hipSetDevice(r->dev));
-    /* the laser's H source in the same pass where nothing comes between */
-    const LaserPlane lf = laser_fold(r, 1);
-    if (with_fold) {
-        FCALL(launch_h_update_jfold, r->g, r->flH, 1, lf, r->jp, r->cfg.bc, r->djr + 4);
-        if (fabs(r->vsp - 1.0) >= 1e-10) TRY(launch_vsp(r->stream, r->jp.J, 3, r->g, r->vsp));
-    } else {
-        FCALL(launch_h_update, r->g, r->flH, 1, nullptr, lf);
-    }
-    if (r->tfsf.on) {                    /* TFSF_postHStep, source/core/em.c:125 */
+    if (r->tfsf.on) {
         const Tfsf &tf = r->tfsf;
         if (r->fp32)
             TRY(launch_tfsf(r->stream, r->f32.H, r->g, tf.fh, tf.maxvol, tf.ddata, tf.dtab,
@@ -1923,21 +1921,23 @@ static int h_step(mpic_run *r, bool with_fold)
             TRY(launch_tfsf(r->stream, r->f.H, r->g, tf.fh, tf.maxvol, tf.ddata, tf.dtab,
                             r->dstep, LASER_CAP, 0, 1.0));
     }
-    if (!lf.on) {
-        const Box inner = laser_box_H(r);
-        if (r->fp32)
-            TRY(laser_H(r, r->f32.H[1], r->f32.H[2], inner));
-        else
-            TRY(laser_H(r, r->f.H[1], r->f.H[2], inner));
-    }
-    r->stage = 2;
-    return MPIC_OK;
+    if (laser_done) return MPIC_OK;
+    const Box inner = laser_box_H(r);
+    if (r->fp32) return laser_H(r, r->f32.H[1], r->f32.H[2], inner);
+    return laser_H(r, r->f.H[1], r->f.H[2], inner);
 }
 
 extern "C" int mpic_em_h_step(mpic_run_t *r)
 {
     if (!r) return MPIC_ERR_ARG;
-    return h_step(r, false);
+    TRY(check_stage(r, 1));
+    MPIC_CHECK(hipSetDevice(r->dev));
+    /* the laser's H source in the same pass where nothing comes between */
+    const LaserPlane lf = laser_fold(r, 1);
+    FCALL(launch_h_update, r->g, r->flH, 1, lf);
+    TRY(h_sources(r, lf.on != 0));
+    r->stage = 2;
+    return MPIC_OK;
 }
 
 extern "C" int mpic_em_e_start(mpic_run_t *r)
@@ -1952,11 +1952,11 @@ extern "C" int mpic_em_e_start(mpic_run_t *r)
     return MPIC_OK;
 }
 
-/* jbc_finish's x walls: the first part of mpic_j_finish. */
-static int j_fold_x(mpic_run *r)
+/* VSP_vectorSweep after the boundary fold (source/core/plasma_currentWalls.c:204) */
+static int vsp_J(mpic_run *r)
 {
-    const int *bc = r->cfg.bc;
-    return launch_jfold(r->stream, r->jp, r->g, 0, bc[0], bc[3], r->djr + 4);
+    if (fabs(r->vsp - 1.0) < 1e-10) return MPIC_OK;
+    return launch_vsp(r->stream, r->jp.J, 3, r->g, r->vsp);
 }
 
 extern "C" int mpic_j_finish(mpic_run_t *r)
@@ -1965,11 +1965,9 @@ extern "C" int mpic_j_finish(mpic_run_t *r)
     MPIC_CHECK(hipSetDevice(r->dev));
     const int *bc = r->cfg.bc;
     /* x walls, then the y and z walls plane by plane */
-    TRY(j_fold_x(r));
+    TRY(launch_jfold(r->stream, r->jp, r->g, 0, bc[0], bc[3], r->djr + 4));
     TRY(launch_jfold_planes(r->stream, r->jp, r->g, bc, r->djr + 4));
-    /* VSP_vectorSweep after the boundary fold (source/core/plasma_currentWalls.c:204) */
-    if (fabs(r->vsp - 1.0) >= 1e-10) TRY(launch_vsp(r->stream, r->jp.J, 3, r->g, r->vsp));
-    return MPIC_OK;
+    return vsp_J(r);
 }
 
 /* VSP_configure (source/core/plasma_VSP.c:18-27). */
@@ -2063,19 +2061,59 @@ static void mark_ring(mpic_run *r)
  * after the deposit: slots 1, 2, 3 of the step's five) are recorded. */
 static int step_body(mpic_run *r)
 {
+    TRY(check_stage(r, 0));
+    MPIC_CHECK(hipSetDevice(r->dev));
     if (!r->capturing) mark_ring(r);
-    /* em_energy after the H half step (its sums come out of the H update),
-     * plasma_temperature after the push (source/core/main.c:371,383): one
-     * ring row per step, nothing copied back, so the step stays
-     * asynchronous */
-    /* the J clear joins the H half step's launch, the y and z J folds the
-     * H step's */
-    TRY(h_half(r, r->dpart, true));
-    TRY(mpic_push_deposit(r));
-    /* jbc_finish reads and writes J only and the H step does not read J:
-     * the fold goes first, so that E -= tau J can join the E update */
-    TRY(j_fold_x(r));
-    TRY(h_step(r, true));
+    TRY(laser_tables(r, 1));
+    TRY(tfsf_record(r));
+    /* em_HHalfStep and em_HStep in one pass (the E caps follow the push: they
+     * need H^{n+1/2} and E^n only, and their walls are wanted by the E
+     * update).  em_energy after the half step (its sums come out of this
+     * pass), plasma_temperature after the push (source/core/main.c:371,383):
+     * one ring row per step, nothing copied back, so the step stays
+     * asynchronous. */
+    const LaserPlane lh = laser_fold(r, 1);
+    FCALL(launch_h_full_jclear, r->g, r->cfg.bc, r->dpart, lh, r->jp.J[0], r->dkin, r->djr,
+          r->dstep, r->tv.xr, r->tiled ? 0 : 1);
+    swap_fields(r);
+    TRY(h_sources(r, lh.on != 0));
+    /* the push reads H^n, which lies where the E caps go afterwards */
+    Fields32 p32 = r->f32;
+    Fields64 p64 = r->f;
+    for (int c = 0; c < 3; ++c) {
+        p32.H[c] = r->f32.Ec[c];
+        p64.H[c] = r->f.Ec[c];
+    }
+    TRY(push(r, p32, p64));
+    AfterPush ap;
+    ap.updE = &r->updE;
+    ap.ops = r->bcE.data();
+    ap.nop = (int)r->bcE.size();
+    ap.jp = r->jp;
+    for (int q = 0; q < 6; ++q) ap.bc[q] = r->cfg.bc[q];
+    ap.jr = r->djr + 4;
+    ap.tv = &r->tv;
+    ap.scanw = r->scanw;
+    ap.err = r->derr;
+    ap.parity = r->parity;
+    ap.sorted = r->tiled;
+    ap.nbound = r->n;
+    ap.tj = r->tj;
+    ap.gather_blocks = r->gather_blocks;
+    ap.after_gather = r->timed >= 0 && r->fp32 ? r->evpool[5 * r->timed + 3] : nullptr;
+    /* the caps of E take the cap H from the current H, its copy */
+    Fields32 c32 = r->f32;
+    Fields64 c64 = r->f;
+    for (int c = 0; c < 3; ++c) {
+        c32.Hc[c] = r->f32.H[c];
+        c64.Hc[c] = r->f.H[c];
+    }
+    if (r->timed >= 0 && !r->fp32) TRY(record(r, 3));
+    TRY(r->fp32 ? launch_after_push(r->stream, c32, r->g, ap)
+                : launch_after_push(r->stream, c64, r->g, ap));
+    if (r->tiled) swap_markers(r);
+    TRY(vsp_J(r));
+    r->stage = 2;
     /* one pass for em_EStep_start, the laser's E plane and E -= tau J where
      * no other source adds to E between them (FP64 form: no TFSF interface,
      * at most one laser, which the pass adds in the reference's order),
@@ -2146,6 +2184,7 @@ static void host_step(mpic_run *r)
 {
     mark_ring(r);
     if (r->tiled) swap_markers(r);
+    swap_fields(r);
     r->time = r->time + r->g.tau;
     ++r->step;
     r->stage = 0;
@@ -2174,9 +2213,10 @@ static int graph_of(const Recorder &rec, hipGraphExec_t *exec)
     return rc;
 }
 
-/* Graphs of one step from each marker-buffer parity in exec[0..1]: the
- * kernel arguments of a step differ only by which buffer holds the sorted
- * markers, so two graphs replay every step.  The step is recorded, not run,
+/* Graphs of one step from the current phase and the one after it in
+ * exec[0..1]: the kernel arguments of a step differ only by which of the
+ * double buffers are current, and a step toggles them all, so two graphs
+ * replay every step.  The step is recorded, not run,
  * and the host state is restored afterwards. */
 static int capture(mpic_run *r)
 {
@@ -2190,7 +2230,7 @@ static int capture(mpic_run *r)
             hipGraphExecDestroy(r->exec[k]);
             r->exec[k] = nullptr;
         }
-    r->exec_parity = r->parity;
+    r->exec_phase = phase_of(r);
     Recorder two[2];
     int rc = record_steps(r, two);
     for (int k = 0; k < 2 && rc == MPIC_OK; ++k) rc = graph_of(two[k], &r->exec[k]);
@@ -2198,9 +2238,16 @@ static int capture(mpic_run *r)
     return rc;
 }
 
+/* The run's phase is one of the two its graphs start from (stage calls and
+ * sorts can leave it at another). */
+static bool graphs_current(const mpic_run *r)
+{
+    return r->graphs_ok && (phase_of(r) == r->exec_phase || phase_of(r) == (r->exec_phase ^ 7));
+}
+
 static int replay(mpic_run *r)
 {
-    const int k = (r->parity == r->exec_parity) ? 0 : 1;
+    const int k = (phase_of(r) == r->exec_phase) ? 0 : 1;
     MPIC_CHECK(hipGraphLaunch(r->exec[k], r->stream));
     host_step(r);
     return MPIC_OK;
@@ -2257,9 +2304,8 @@ struct FusedLaunch {
 struct Ensemble {
     std::vector<mpic_run *> runs;
     std::vector<long>       topo;      /* runs' topo counters when built */
-    std::vector<int>        rel;       /* parity of run q relative to run 0 */
+    std::vector<int>        phase;     /* runs' phases at which exec[0] starts */
     int                     dev;
-    int                     parity0;   /* run 0's parity at phase 0 */
     hipStream_t             stream;
     void                   *dmem;
     hipGraphExec_t          exec[2];
@@ -2299,11 +2345,12 @@ static void ensemble_forget(mpic_run *r)
 static bool ensemble_matches(const Ensemble *e, mpic_run *const *runs, int nruns)
 {
     if (!e || (int)e->runs.size() != nruns) return false;
+    const int flip = nruns ? phase_of(runs[0]) ^ e->phase[0] : 0;   /* 0 or 7, for every run */
     for (int q = 0; q < nruns; ++q)
         if (e->runs[q] != runs[q] || e->topo[q] != runs[q]->topo ||
-            e->rel[q] != (runs[q]->parity ^ runs[0]->parity))
+            (phase_of(runs[q]) ^ e->phase[q]) != flip)
             return false;
-    return true;
+    return flip == 0 || flip == 7;
 }
 
 /* Records one step of run r at each marker-buffer phase (k = 0: its current
@@ -2312,9 +2359,11 @@ static int record_steps(mpic_run *r, Recorder rec[2])
 {
     const double time = r->time;
     const long step = r->step;
-    const int cur = r->cur, parity = r->parity;
+    const int cur = r->cur, parity = r->parity, hsw = r->hsw;
     const Markers32 m32 = r->m32;
     const Markers64 m = r->m;
+    const Fields32 f32 = r->f32;
+    const Fields64 f = r->f;
     int rc = MPIC_OK;
     for (int k = 0; k < 2 && rc == MPIC_OK; ++k) {
         g_recorder = &rec[k];
@@ -2327,8 +2376,11 @@ static int record_steps(mpic_run *r, Recorder rec[2])
     r->step = step;
     r->cur = cur;
     r->parity = parity;
+    r->hsw = hsw;
     r->m32 = m32;
     r->m = m;
+    r->f32 = f32;
+    r->f = f;
     r->stage = 0;
     return rc;
 }
@@ -2367,11 +2419,10 @@ static int ensemble_build(mpic_run *const *runs, int nruns, Ensemble **out)
 {
     Ensemble *e = new Ensemble();
     e->dev = runs[0]->dev;
-    e->parity0 = runs[0]->parity;
     for (int q = 0; q < nruns; ++q) {
         e->runs.push_back(runs[q]);
         e->topo.push_back(runs[q]->topo);
-        e->rel.push_back(runs[q]->parity ^ runs[0]->parity);
+        e->phase.push_back(phase_of(runs[q]));
     }
     int rc = MPIC_OK;
     std::vector<Recorder> recs[2];
@@ -2488,7 +2539,7 @@ static int ensemble_build(mpic_run *const *runs, int nruns, Ensemble **out)
 static int batch_streams(mpic_run *const *runs, int nruns, long chunk)
 {
     for (int q = 0; q < nruns; ++q)
-        if (!runs[q]->graphs_ok) TRY(capture(runs[q]));
+        if (!graphs_current(runs[q])) TRY(capture(runs[q]));
     int dev = -1;
     for (long s = 0; s < chunk; ++s)
         for (int q = 0; q < nruns; ++q) {
@@ -2520,7 +2571,7 @@ static int batch_fused(mpic_run *const *runs, int nruns, long chunk)
         MPIC_CHECK(hipStreamWaitEvent(e->stream, e->ev[q], 0));
     }
     for (long s = 0; s < chunk; ++s) {
-        const int k = runs[0]->parity == e->parity0 ? 0 : 1;
+        const int k = phase_of(runs[0]) == e->phase[0] ? 0 : 1;
         MPIC_CHECK(hipGraphLaunch(e->exec[k], e->stream));
         for (int q = 0; q < nruns; ++q) host_step(runs[q]);
     }

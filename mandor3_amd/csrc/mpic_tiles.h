@@ -30,6 +30,8 @@ struct TileView {
     int *active;             /* [ntiles] tiles holding markers, in tile order */
     int *nactive;            /* [1] */
     int *nmark;              /* [2] markers in the current / next order */
+    int *xr;                 /* [2] x planes of nodes that the active tiles' gathers read
+                              * (tiled runs: kept by the rank pass; else the whole grid) */
     /* Work items of the push: an active tile's markers, in the FP32 form split
      * evenly into ceil(count / chm) items of at most chm markers (chm = 0:
      * one item per active tile). */
@@ -120,8 +122,28 @@ int launch_counts_natural(hipStream_t s, const TileView &tv, const Grid &g, int3
 int launch_push32(hipStream_t s, const Markers32 &m, const Markers32 &dst, const Fields32 &f,
                   const Grid &g, const PushConsts &pc, const float *qm, const TileView &tv,
                   float *tj, double *kin, int nblocks, int waves);
-int launch_jgather32(hipStream_t s, const Fields32 &f, const Grid &g, const TileView &tv,
+int launch_jgather32(hipStream_t s, const JPtrs &j, const Grid &g, const TileView &tv,
                      const float *tj, int nblocks);
+
+/* What the loop body's launches between the push and the E update work on. */
+struct AfterPush {
+    const BoxSet       *updE;          /* the E caps' update boxes */
+    const FaceOp       *ops;           /* the walls on the E caps, x then y then z */
+    int                 nop;
+    JPtrs               jp;
+    int                 bc[6];
+    const int          *jr;            /* x planes where J may be non-zero */
+    const TileView     *tv;
+    unsigned long long *scanw;
+    unsigned           *err;
+    int                 parity, sorted;   /* sorted: a tiled run, ranked here */
+    long                nbound;
+    const float        *tj;            /* FP32: the J blocks */
+    int                 gather_blocks;
+    hipEvent_t          after_gather;  /* recorded after the J gather (null: not timed) */
+};
+template <class T>
+int launch_after_push(hipStream_t s, const FieldsT<T> &f, const Grid &g, const AfterPush &p);
 int launch_keys32(hipStream_t s, const Markers32 &m, long n, const TileView &tv, int parity);
 int launch_rho32(hipStream_t s, const Markers32 &m, long n, double *rho, const Grid &g,
                  const TileView &tv, int parity);
