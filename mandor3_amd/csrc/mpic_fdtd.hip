@@ -86,11 +86,18 @@ __device__ static inline bool span_group(const Span &sp, int V, const VBlock &b,
 __device__ static inline bool box_decode(const BoxSet &bs, long t, int &i, int &j, int &k)
 {
     if (t >= bs.off[bs.n]) return false;
-    int b = 0;
-    while (t >= bs.off[b + 1]) ++b;
+    /* the box is selected by value: indexed by lane, its fields would be a
+     * chain of vector loads from the argument block */
+    Box B = bs.b[0];
+    long off = 0;
+#pragma unroll
+    for (int b = 1; b < 6; ++b)
+        if (b < bs.n && t >= bs.off[b]) {
+            B = bs.b[b];
+            off = bs.off[b];
+        }
     /* boxes hold fewer than 2^32 nodes: 32-bit division */
-    unsigned l = (unsigned)(t - bs.off[b]);
-    const Box &B = bs.b[b];
+    unsigned l = (unsigned)(t - off);
     const unsigned dz = B.hi[2] - B.lo[2] + 1, dy = B.hi[1] - B.lo[1] + 1;
     const unsigned l2 = l / dz;
     k = B.lo[2] + (int)(l - l2 * dz);
@@ -355,17 +362,18 @@ template <class T> struct KernelDef<FacePlanesArgs<T>> {
     {
         const int i = a.ilo + (int)b.x;
         for (int q = 0; q < a.nop;) {
-            /* a phase is one op, or the two walls of an axis: their lines
-             * side by side */
+            /* a phase is one op, or the two walls of an axis, each taken by
+             * half the wavefronts (the op uniform over a wavefront: its
+             * fields are scalar loads) */
             const int two = q + 1 < a.nop && a.phase[q + 1] == a.phase[q];
             if (q) __syncthreads();           /* the plane's lines of the earlier phase are done */
-            long first[2], count[2] = {0, 0};
-            plane_lines(a.op[q], i, first[0], count[0]);
-            if (two) plane_lines(a.op[q + 1], i, first[1], count[1]);
-            for (long u = threadIdx.x; u < count[0] + count[1]; u += TPB) {
-                const bool second = u >= count[0];
-                face_apply<T>(a.g, a.op[q + second], second ? first[1] + u - count[0] : first[0] + u);
-            }
+            const int half = TPB / 2, second =
+                two & __builtin_amdgcn_readfirstlane((int)threadIdx.x >= half);
+            const FaceOp &op = a.op[q + second];
+            long first, count;
+            plane_lines(op, i, first, count);
+            for (long u = (int)threadIdx.x - second * half; u < count; u += two ? half : TPB)
+                face_apply<T>(a.g, op, first + u);
             q += 1 + two;
         }
     }
@@ -1006,6 +1014,8 @@ template <class T> struct EFusedArgs {
     const int *jr;         /* x planes [jr[0], jr[1]] of nodes where J may be non-zero */
     LaserPlane lp;         /* a laser's E plane, added between the update and E -= tau J
                             * as the reference's sequence does (on = 0: none) */
+    const int *estep;      /* this step (what the E side's sources read) */
+    int       *step;       /* the step counter, advanced here: nothing in this launch reads it */
 };
 
 template <class T>
@@ -1083,17 +1093,18 @@ template <class T> struct KernelDef<EFusedArgs<T>> {
     static constexpr int kBlock = TPB;
     __device__ __forceinline__ static void body(const EFusedArgs<T> &a, VBlock b, VBlock gd)
     {
+        if (b.x == 0 && threadIdx.x == 0) *a.step = *a.estep + 1;
         e_fused<T>(a.f, a.g, a.fl, a.sp, a.c1, a.c2, a.c3, a.jr, a.lp, b, gd);
     }
 };
 
 template <class T>
 int launch_e_fused(hipStream_t s, const FieldsT<T> &f, const Grid &g, const BoxSet &flush,
-                   const int *jr, const LaserPlane &lp)
+                   const int *jr, const LaserPlane &lp, const int *estep, int *step)
 {
     const Span sp = span_of<Vec<T>::N>(-1, -1, g.n[1] + 1, -1, g.n[2] + 1);
     EFusedArgs<T> a = {f, g, flush, sp, (T)(g.tau / g.h[0]), (T)(g.tau / g.h[1]),
-                       (T)(g.tau / g.h[2]), jr, lp};
+                       (T)(g.tau / g.h[2]), jr, lp, estep, step};
     return launch_def(s, a, grid_span(sp, g.n[0] + 3));
 }
 
@@ -1628,66 +1639,6 @@ int launch_vsp(hipStream_t s, double *const F[3], int ncomp, const Grid &g, doub
     return MPIC_OK;
 }
 
-/* em_energy of the loop body (source/core/em.c:226-252) without atomics:
- * one wavefront per cell row (i, j), lanes along k, each workgroup's partial
- * sums stored in part[2 * block + {0, 1}] and combined in fixed order by
- * k_diag_ring. */
-/* Row of the diagnostics ring of the current step (device step counter
- * *step): the two energy sums of k_energy_part's nparts partials (fixed
- * order) and the three kinetic sums of the push (its slots). */
-struct DiagRingArgs {
-    const double *part;
-    int           nparts;
-    const double *kin;
-    double       *ring;
-    int          *step;
-    int           cap;
-    int           tick;    /* advance the step counter after the row (the step's last kernel) */
-};
-
-#define RING_TPB 1024
-
-__device__ static inline void diag_ring(const double *part, int nparts, const double *kin,
-                                        double *ring, int *step, int cap, int tick)
-{
-    __shared__ double sw[5][RING_TPB / 64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    double v[5] = {0, 0, 0, 0, 0};
-    if (threadIdx.x < KIN_SLOTS)
-        for (int a = 0; a < 3; ++a) v[2 + a] = kin[KIN_STRIDE * threadIdx.x + a];
-    for (int q = threadIdx.x; q < nparts; q += RING_TPB) {
-        v[0] += part[2 * q];
-        v[1] += part[2 * q + 1];
-    }
-    for (int a = 0; a < 5; ++a) {
-        for (int d = 32; d > 0; d >>= 1) v[a] += __shfl_down(v[a], d, 64);
-        if (lane == 0) sw[a][w] = v[a];
-    }
-    __syncthreads();
-    if (threadIdx.x < 5) {
-        double s = 0;
-        for (int q = 0; q < RING_TPB / 64; ++q) s += sw[threadIdx.x][q];
-        const int st = *step;
-        ring[5 * (long)(st % cap) + threadIdx.x] = s;
-        if (tick && threadIdx.x == 0) *step = st + 1;   /* one wavefront: read before written */
-    }
-}
-
-template <> struct KernelDef<DiagRingArgs> {
-    static constexpr int kBlock = RING_TPB;
-    __device__ __forceinline__ static void body(const DiagRingArgs &a, VBlock, VBlock)
-    {
-        diag_ring(a.part, a.nparts, a.kin, a.ring, a.step, a.cap, a.tick);
-    }
-};
-
-int launch_diag_ring(hipStream_t s, const double *part, int nparts, const double *kin,
-                     double *ring, int *step, int cap, int tick)
-{
-    DiagRingArgs a = {part, nparts, kin, ring, step, cap, tick};
-    return launch_def(s, a, 1);
-}
-
 __global__ void k_zero(double *p, long n)
 {
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1725,6 +1676,7 @@ struct JClearArgs {
     double       *kin;        /* the push's kinetic sums */
     int          *range;      /* [2][2] plane ranges by step parity, [2] this step's */
     const int    *step, *xr;
+    int          *estep;      /* loop steps: the counter that the E side reads, set here */
     int           full;
 };
 
@@ -1756,6 +1708,7 @@ __device__ static inline void jclear(const JClearArgs &a, const VBlock &b, const
         }
         a.range[2 * ((s + 1) & 1)] = nlo;
         a.range[2 * ((s + 1) & 1) + 1] = nhi;
+        if (a.estep) *a.estep = s;
         a.range[4] = nlo;                                    /* this step's, for E -= tau J */
         a.range[5] = nhi;
     }
@@ -1780,9 +1733,9 @@ template <> struct KernelDef<JClearArgs> {
 };
 
 static JClearArgs jclear_args(double *J, const Grid &g, double *kin, int *range, const int *step,
-                              const int *xr, int full)
+                              const int *xr, int *estep, int full)
 {
-    JClearArgs a = {J, g.ncell, (long)g.GY * g.GZ, g.n[0], kin, range, step, xr, full};
+    JClearArgs a = {J, g.ncell, (long)g.GY * g.GZ, g.n[0], kin, range, step, xr, estep, full};
     return a;
 }
 
@@ -1800,7 +1753,8 @@ static unsigned jclear_blocks(const Grid &g)
 int launch_jclear(hipStream_t s, double *J, const Grid &g, double *kin, int *range,
                   const int *step, const int *xr, int full)
 {
-    return launch_def(s, jclear_args(J, g, kin, range, step, xr, full), jclear_blocks(g));
+    return launch_def(s, jclear_args(J, g, kin, range, step, xr, nullptr, full),
+                      jclear_blocks(g));
 }
 
 /* CIC rho fold of one face, source/core/plasma_rho.c:23-96. */
@@ -1967,7 +1921,7 @@ int launch_probes(hipStream_t s, T *const E[3], T *const H[3], const Grid &g, co
 template <class T>
 int launch_h_full_jclear(hipStream_t s, const FieldsT<T> &f, const Grid &g, const int bc[6],
                          double *part, const LaserPlane &lp, double *J, double *kin, int *range,
-                         const int *step, const int *xr, int jfull)
+                         const int *step, const int *xr, int *estep, int jfull)
 {
     HEdgeArgs<T> e;
     HFullArgs<T> &a = e.h;
@@ -1993,7 +1947,8 @@ int launch_h_full_jclear(hipStream_t s, const FieldsT<T> &f, const Grid &g, cons
     p.ga = {ne, 1, 1};
     p.gb = {na, 1, 1};
     p.na = ne;
-    return launch_pair(s, p, dim3(ne + na), jclear_args(J, g, kin, range, step, xr, jfull),
+    return launch_pair(s, p, dim3(ne + na),
+                       jclear_args(J, g, kin, range, step, xr, estep, jfull),
                        dim3(jclear_blocks(g)));
 }
 
@@ -2004,6 +1959,64 @@ int launch_jgather32(hipStream_t s, const JPtrs &j, const Grid &g, const TileVie
     return launch_def(s, a, (unsigned)nblocks);
 }
 
+/* Row of the diagnostics ring of the current step (device step counter
+ * *step), one workgroup: the two energy sums of the H update's nparts partials
+ * (fixed order) and the three kinetic sums of the push (its slots). */
+struct DiagRingArgs {
+    const double *part;
+    int           nparts;
+    const double *kin;
+    double       *ring;
+    const int    *step;
+    int           cap;
+};
+
+__device__ static inline void diag_ring(const DiagRingArgs &A)
+{
+    typedef double D2 __attribute__((ext_vector_type(2)));
+    __shared__ double sw[5][TPB / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    double v[5] = {0, 0, 0, 0, 0};
+    for (int q = threadIdx.x; q < KIN_SLOTS; q += TPB)
+        for (int a = 0; a < 3; ++a) v[2 + a] += A.kin[KIN_STRIDE * q + a];
+    const D2 *part = (const D2 *)A.part;
+    const int n = A.nparts;
+    int q = threadIdx.x;
+    for (; q + 7 * TPB < n; q += 8 * TPB) {          /* eight loads in flight */
+        D2 x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = part[q + u * TPB];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            v[0] += x[u][0];
+            v[1] += x[u][1];
+        }
+    }
+    for (; q < n; q += TPB) {
+        const D2 x = part[q];
+        v[0] += x[0];
+        v[1] += x[1];
+    }
+    for (int a = 0; a < 5; ++a) {
+        for (int d = 32; d > 0; d >>= 1) v[a] += __shfl_down(v[a], d, 64);
+        if (lane == 0) sw[a][w] = v[a];
+    }
+    __syncthreads();
+    if (threadIdx.x < 5) {
+        double s = 0;
+        for (int u = 0; u < TPB / 64; ++u) s += sw[threadIdx.x][u];
+        A.ring[5 * (long)(*A.step % A.cap) + threadIdx.x] = s;
+    }
+}
+
+template <> struct KernelDef<DiagRingArgs> {
+    static constexpr int kBlock = TPB;
+    __device__ __forceinline__ static void body(const DiagRingArgs &a, VBlock, VBlock)
+    {
+        diag_ring(a);
+    }
+};
+
 /* The loop body between the push and the E update, two chains that need
  * nothing from each other beside the sort: the E caps and their walls (which
  * need H^{n+1/2}) and the J folds (which need the finished J).  Every tiny
@@ -2011,10 +2024,10 @@ int launch_jgather32(hipStream_t s, const JPtrs &j, const Grid &g, const TileVie
  * sort's passes (and the FP32 form's J gather), the few workgroups of the
  * links first, so that they do not wait behind the many of a pass:
  *   FP32  [E caps | J gather]   [x walls | x folds | scan]
- *         [y, z walls | y, z folds | rank]
- *   FP64  [E caps | x folds | scan]   [x walls | y, z folds | rank]
+ *         [ring | y, z walls | y, z folds | rank]
+ *   FP64  [E caps | x folds | scan]   [ring | x walls | y, z folds | rank]
  *         [y, z walls]
- * in place of nine launches.  The two walls of an axis (7 cells or more)
+ * in place of ten launches.  The two walls of an axis (7 cells or more)
  * touch disjoint node layers, and so do its two J folds, so each pair runs in
  * one launch whatever its kinds. */
 template <class T>
@@ -2043,15 +2056,17 @@ int launch_after_push(hipStream_t s, const FieldsT<T> &f, const Grid &g, const A
     const ScanArgs sc = scan_args(*p.tv, p.scanw, p.err, p.parity ^ 1);
     const RankArgs rk = {*p.tv, p.nbound, p.parity};
     const dim3 gsc(p.sorted ? sc.nb : 0), grk(p.sorted ? rank_blocks(p.nbound) : 0);
+    const DiagRingArgs ring = {p.part, p.nparts, p.kin, p.ring, p.step, p.ringcap};
     if (sizeof(T) == 4) {
         const JGatherArgs jg = {p.jp, g, *p.tv, p.tj};
         TRY_LAUNCH(launch_pair(s, cap, gcap, jg, dim3(p.gather_blocks)));
         if (p.after_gather) MPIC_CHECK(hipEventRecord(p.after_gather, s));
         TRY_LAUNCH(launch_three(s, fx, gfx, jx, gjx, sc, gsc));
-        return launch_three(s, fp, dim3(planes), jp, gjp, rk, grk);
+        return launch_three(s, pair_of(ring, 1, fp, planes), dim3(1 + planes), jp, gjp, rk, grk);
     }
+    const unsigned nfx = gfx.x * gfx.y;
     TRY_LAUNCH(launch_three(s, cap, gcap, jx, gjx, sc, gsc));
-    TRY_LAUNCH(launch_three(s, fx, gfx, jp, gjp, rk, grk));
+    TRY_LAUNCH(launch_three(s, pair_of(ring, 1, fx, gfx), dim3(1 + nfx), jp, gjp, rk, grk));
     return launch_def(s, fp, planes);
 }
 
@@ -2063,11 +2078,13 @@ int launch_after_push(hipStream_t s, const FieldsT<T> &f, const Grid &g, const A
                                     const BoxSet &, int, const LaserPlane &);                   \
     template int launch_h_full_jclear<T>(hipStream_t, const FieldsT<T> &, const Grid &,           \
                                          const int *, double *, const LaserPlane &, double *,   \
-                                         double *, int *, const int *, const int *, int);       \
+                                         double *, int *, const int *, const int *, int *,      \
+                                         int);                                                  \
     template int launch_after_push<T>(hipStream_t, const FieldsT<T> &, const Grid &,              \
                                       const AfterPush &);                                       \
     template int launch_e_fused<T>(hipStream_t, const FieldsT<T> &, const Grid &,                 \
-                                   const BoxSet &, const int *, const LaserPlane &);            \
+                                   const BoxSet &, const int *, const LaserPlane &,             \
+                                   const int *, int *);                                         \
     template int launch_e_update<T>(hipStream_t, const FieldsT<T> &, const Grid &,                \
                                     const BoxSet &, int, int);                                  \
     template int launch_e_tauJ<T>(hipStream_t, const FieldsT<T> &, const Grid &, int *,         \

@@ -179,13 +179,13 @@ int launch_face_planes(hipStream_t s, const Grid &g, const FaceOp *ops, int nop)
 template <class T>
 int launch_h_full_jclear(hipStream_t s, const FieldsT<T> &f, const Grid &g, const int bc[6],
                          double *part, const LaserPlane &lp, double *J, double *kin, int *range,
-                         const int *step, const int *xr, int jfull);
+                         const int *step, const int *xr, int *estep, int jfull);
 template <class T>
 int launch_h_update(hipStream_t s, const FieldsT<T> &f, const Grid &g, const BoxSet &flush,
                     int full, const LaserPlane &lp = LaserPlane());
 template <class T>
 int launch_e_fused(hipStream_t s, const FieldsT<T> &f, const Grid &g, const BoxSet &flush,
-                   const int *jr, const LaserPlane &lp = LaserPlane());
+                   const int *jr, const LaserPlane &lp, const int *estep, int *step);
 template <class T>
 int launch_e_update(hipStream_t s, const FieldsT<T> &f, const Grid &g, const BoxSet &flush,
                     int interior, int do_flush);
@@ -218,11 +218,10 @@ int launch_probes(hipStream_t s, T *const E[3], T *const H[3], const Grid &g, co
                   int np, double *out);
 template <class T> int launch_energy(hipStream_t s, const FieldsT<T> &f, const Grid &g, double *acc);
 /* Loop-body diagnostics: the one-pass H update writes em_energy partial sums
- * (two doubles per workgroup, h_full_blocks(g, fp32) workgroups); the ring row {W_E sum, W_M sum, WTx, WTy, WTz} of the device step
- * counter's step sums them, and with 'tick' advances the counter. */
+ * (two doubles per workgroup, h_full_blocks(g, fp32) workgroups); the ring
+ * row {W_E sum, W_M sum, WTx, WTy, WTz} of the device step counter's step
+ * sums them. */
 int h_full_blocks(const Grid &g, int fp32);
-int launch_diag_ring(hipStream_t s, const double *part, int nparts, const double *kin,
-                     double *ring, int *step, int cap, int tick);
 int launch_zero(hipStream_t s, double *p, long n);
 int launch_jclear(hipStream_t s, double *J, const Grid &g, double *kin, int *range,
                   const int *step, const int *xr, int full);

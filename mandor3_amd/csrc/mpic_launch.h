@@ -248,6 +248,19 @@ static int launch_def(hipStream_t s, const A &a, unsigned gx, unsigned gy = 1, u
     return MPIC_OK;
 }
 
+/* The argument struct of A over grid ga beside B over grid gb. */
+template <class A, class B>
+static PairArgs<A, B> pair_of(const A &a, dim3 ga, const B &b, dim3 gb)
+{
+    PairArgs<A, B> p;
+    p.a = a;
+    p.b = b;
+    p.ga = {ga.x, ga.y, ga.z};
+    p.gb = {gb.x, gb.y, gb.z};
+    p.na = ga.x * ga.y * ga.z;
+    return p;
+}
+
 /* A over grid ga and B over grid gb in one launch (one of them alone when
  * the other's grid is empty). */
 template <class A, class B>
@@ -256,13 +269,7 @@ static int launch_pair(hipStream_t s, const A &a, dim3 ga, const B &b, dim3 gb)
     const unsigned na = ga.x * ga.y * ga.z, nb = gb.x * gb.y * gb.z;
     if (na == 0) return launch_def(s, b, gb.x, gb.y, gb.z);
     if (nb == 0) return launch_def(s, a, ga.x, ga.y, ga.z);
-    PairArgs<A, B> p;
-    p.a = a;
-    p.b = b;
-    p.ga = {ga.x, ga.y, ga.z};
-    p.gb = {gb.x, gb.y, gb.z};
-    p.na = na;
-    return launch_def(s, p, na + nb);
+    return launch_def(s, pair_of(a, ga, b, gb), na + nb);
 }
 
 /* Three bodies with no order between them; C's grid may be empty. */
@@ -273,13 +280,7 @@ static int launch_three(hipStream_t s, const A &a, dim3 ga, const B &b, dim3 gb,
     const unsigned na = ga.x * ga.y * ga.z, nb = gb.x * gb.y * gb.z;
     if (na == 0) return launch_pair(s, b, gb, c, gc);
     if (nb == 0) return launch_pair(s, a, ga, c, gc);
-    PairArgs<A, B> p;
-    p.a = a;
-    p.b = b;
-    p.ga = {ga.x, ga.y, ga.z};
-    p.gb = {gb.x, gb.y, gb.z};
-    p.na = na;
-    return launch_pair(s, p, dim3(na + nb), c, gc);
+    return launch_pair(s, pair_of(a, ga, b, gb), dim3(na + nb), c, gc);
 }
 
 #endif

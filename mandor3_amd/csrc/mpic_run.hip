@@ -152,7 +152,10 @@ struct mpic_run {
     int           timed;      /* >= 0: index of the timed step of mpic_advance */
     double        time;
     std::vector<hipEvent_t> evpool;  /* 5 events per timed step */
-    int          *dstep;      /* device step counter (indexes the laser tables) */
+    int          *dstep;      /* device step counter (indexes the laser tables); [1]: the copy
+                                 that the E side of a loop step reads, so that the E update can
+                                 advance the counter itself */
+    const int    *estep;      /* the counter of the E side's sources: dstep, in loop steps dstep + 1 */
     int          *djr;        /* device: x plane ranges of J written: by step parity [2][2],
                                  then the current step's [2] */
     Spot          spot;
@@ -582,8 +585,9 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     MPIC_CHECK(hipMalloc(&r->derr, sizeof(unsigned)));
     MPIC_CHECK(hipMemsetAsync(r->derr, 0, sizeof(unsigned), r->stream));
     r->timed = -1;
-    MPIC_CHECK(hipMalloc(&r->dstep, sizeof(int)));
-    MPIC_CHECK(hipMemsetAsync(r->dstep, 0, sizeof(int), r->stream));
+    MPIC_CHECK(hipMalloc(&r->dstep, 2 * sizeof(int)));
+    MPIC_CHECK(hipMemsetAsync(r->dstep, 0, 2 * sizeof(int), r->stream));
+    r->estep = r->dstep;
     {
         /* the first J clear clears the whole grid */
         const int full[6] = {-2, g.n[0] + 2, -2, g.n[0] + 2, -2, g.n[0] + 2};
@@ -1762,7 +1766,7 @@ static LaserPlane laser_plane(const mpic_run *r, const Laser &l, int h, const Bo
     lp.pos = I;
     lp.map = h ? l.dmap : l.dmap + 4 * l.nodes;
     lp.tab = h ? l.dtab : l.dtab + 3 * LASER_CAP;
-    lp.step = r->dstep;
+    lp.step = h ? r->dstep : r->estep;
     lp.cap = LASER_CAP;
     lp.on = lp.jmax >= lp.jmin && lp.kmax >= lp.kmin;
     return lp;
@@ -1996,10 +2000,10 @@ static int e_sources(mpic_run *r, bool laser_done = false)
         const double sign = tf.mode == 0 ? 1.0 : -1.0;
         if (r->fp32)
             TRY(launch_tfsf(r->stream, r->f32.E, r->g, tf.fe, tf.maxvol, tf.ddata, tf.dtab,
-                            r->dstep, LASER_CAP, 1, sign));
+                            r->estep, LASER_CAP, 1, sign));
         else
             TRY(launch_tfsf(r->stream, r->f.E, r->g, tf.fe, tf.maxvol, tf.ddata, tf.dtab,
-                            r->dstep, LASER_CAP, 1, sign));
+                            r->estep, LASER_CAP, 1, sign));
     }
     if (laser_done) return MPIC_OK;     /* added by the fused E update */
     const Box dom = laser_box_E(r);
@@ -2018,10 +2022,10 @@ static int e_spot(mpic_run *r)
         const long np = (long)(r->g.n[1] + 3) * (r->g.n[2] + 3);
         if (r->fp32)
             TRY(launch_spot(r->stream, r->f32.E[1], r->f32.E[2], r->g, sp.i, sp.dprof, sp.dprof + np,
-                            sp.dtab, r->dstep, LASER_CAP));
+                            sp.dtab, r->estep, LASER_CAP));
         else
             TRY(launch_spot(r->stream, r->f.E[1], r->f.E[2], r->g, sp.i, sp.dprof, sp.dprof + np,
-                            sp.dtab, r->dstep, LASER_CAP));
+                            sp.dtab, r->estep, LASER_CAP));
     }
     return MPIC_OK;
 }
@@ -2074,7 +2078,7 @@ static int step_body(mpic_run *r)
      * asynchronous. */
     const LaserPlane lh = laser_fold(r, 1);
     FCALL(launch_h_full_jclear, r->g, r->cfg.bc, r->dpart, lh, r->jp.J[0], r->dkin, r->djr,
-          r->dstep, r->tv.xr, r->tiled ? 0 : 1);
+          r->dstep, r->tv.xr, r->dstep + 1, r->tiled ? 0 : 1);
     swap_fields(r);
     TRY(h_sources(r, lh.on != 0));
     /* the push reads H^n, which lies where the E caps go afterwards */
@@ -2101,6 +2105,12 @@ static int step_body(mpic_run *r)
     ap.tj = r->tj;
     ap.gather_blocks = r->gather_blocks;
     ap.after_gather = r->timed >= 0 && r->fp32 ? r->evpool[5 * r->timed + 3] : nullptr;
+    ap.part = r->dpart;
+    ap.nparts = r->nparts;
+    ap.kin = r->dkin;
+    ap.ring = r->dring;
+    ap.step = r->dstep;
+    ap.ringcap = DIAG_RING;
     /* the caps of E take the cap H from the current H, its copy */
     Fields32 c32 = r->f32;
     Fields64 c64 = r->f;
@@ -2122,17 +2132,14 @@ static int step_body(mpic_run *r)
     const bool fused = r->fp32 || (!r->tfsf.on && r->lasers.size() <= 1);
     if (fused) {
         const LaserPlane lf = laser_fold(r, 0);
-        FCALL(launch_e_fused, r->g, r->flE, r->djr + 4, lf);
+        FCALL(launch_e_fused, r->g, r->flE, r->djr + 4, lf, r->estep, r->dstep);
         TRY(e_sources(r, lf.on != 0));
     } else {
         TRY(mpic_em_e_start(r));
         TRY(e_sources(r));
-        FCALL(launch_e_tauJ, r->g, nullptr, r->djr + 4);
+        FCALL(launch_e_tauJ, r->g, r->dstep, r->djr + 4);
     }
     TRY(e_spot(r));
-    /* the ring row of this step, then the device step counter advances */
-    TRY(launch_diag_ring(r->stream, r->dpart, r->nparts, r->dkin, r->dring, r->dstep,
-                         DIAG_RING, 1));
     step_done(r);
     return MPIC_OK;
 }
@@ -2140,7 +2147,9 @@ static int step_body(mpic_run *r)
 static int step_async(mpic_run *r, int idx)
 {
     r->timed = idx;
+    r->estep = r->dstep + 1;
     const int rc = step_body(r);
+    r->estep = r->dstep;
     r->timed = -1;
     return rc;
 }

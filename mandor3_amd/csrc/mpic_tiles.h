@@ -141,6 +141,12 @@ struct AfterPush {
     const float        *tj;            /* FP32: the J blocks */
     int                 gather_blocks;
     hipEvent_t          after_gather;  /* recorded after the J gather (null: not timed) */
+    /* the diagnostics ring's row of this step */
+    const double       *part, *kin;
+    int                 nparts;
+    double             *ring;
+    const int          *step;
+    int                 ringcap;
 };
 template <class T>
 int launch_after_push(hipStream_t s, const FieldsT<T> &f, const Grid &g, const AfterPush &p);
