@@ -1837,8 +1837,8 @@ int launch_gauss(hipStream_t s, const FieldsT<T> &f, const double *rho1, const d
     return MPIC_OK;
 }
 
-/* Node values of the Tecplot records and the probes (source/IO_tecplot.c:
- * 131-153, source/core/diag_probe.c:361-383), in FP64: kind 0 (E, J) is the
+/* Node values of the probes (source/IO_tecplot.c:131-153,
+ * source/core/diag_probe.c:361-383), in FP64: kind 0 (E, J) is the
  * mean of the two values along the component's own axis, kind 1 (H) the mean
  * of the four around the node in the plane normal to it, summed in the
  * reference's order. */
@@ -1858,32 +1858,6 @@ __device__ static inline void node_values(T *const F[3], const Grid &g, int kind
         v[2] = 0.25 * ((double)F[2][gidx(g, i, j, k)] + (double)F[2][gidx(g, i + 1, j, k)] +
                        (double)F[2][gidx(g, i, j + 1, k)] + (double)F[2][gidx(g, i + 1, j + 1, k)]);
     }
-}
-
-/* nodes [0, n] (k fastest), three interleaved doubles per node */
-template <class T>
-__global__ void k_node_fields(Ptr3<T> F, Grid g, int kind, double *out)
-{
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const unsigned nz = (unsigned)g.n[2] + 1, ny = (unsigned)g.n[1] + 1;
-    if (t >= (long)(g.n[0] + 1) * ny * nz) return;
-    const unsigned r = (unsigned)t / nz, i = r / ny;
-    const int k = (int)((unsigned)t - r * nz), j = (int)(r - i * ny);
-    double v[3];
-    node_values(F.p, g, kind, (int)i, j, k, v);
-    out[3 * t] = v[0];
-    out[3 * t + 1] = v[1];
-    out[3 * t + 2] = v[2];
-}
-
-template <class T>
-int launch_node_fields(hipStream_t s, T *const F[3], const Grid &g, int kind, double *out)
-{
-    Ptr3<T> P = {{F[0], F[1], F[2]}};
-    const long n = (long)(g.n[0] + 1) * (g.n[1] + 1) * (g.n[2] + 1);
-    k_node_fields<T><<<nblk(n), TPB, 0, s>>>(P, g, kind, out);
-    MPIC_CHECK(hipGetLastError());
-    return MPIC_OK;
 }
 
 /* probe p at node ijk[3p..3p+2] (checked on the host to lie in [0, n-1]):
@@ -2097,7 +2071,6 @@ int launch_after_push(hipStream_t s, const FieldsT<T> &f, const Grid &g, const A
                                 const double *, const int *, const int *, int, int, double);   \
     template int launch_gauss<T>(hipStream_t, const FieldsT<T> &, const double *,                \
                                  const double *, const Grid &, double *);                       \
-    template int launch_node_fields<T>(hipStream_t, T *const[3], const Grid &, int, double *);   \
     template int launch_tfsf_record<T>(hipStream_t, T *const[3], T *const[3], const Grid &,      \
                                        const TfsfSet &, const TfsfSet &, long, const double *,  \
                                        double *, const int *, int, int);                        \

@@ -208,8 +208,6 @@ int launch_jfold_planes(hipStream_t s, const JPtrs &f, const Grid &g, const int 
 /* VSP (beta, alpha, beta) sweeps along z, y, x of ncomp arrays on the padded grid. */
 int launch_vsp(hipStream_t s, double *const F[3], int ncomp, const Grid &g, double alpha);
 template <class T>
-int launch_node_fields(hipStream_t s, T *const F[3], const Grid &g, int kind, double *out);
-template <class T>
 int launch_tfsf_record(hipStream_t s, T *const E[3], T *const H[3], const Grid &g,
                        const TfsfSet &fe, const TfsfSet &fh, long maxvol, const double *factor,
                        double *out, const int *step, int step0, int cap);

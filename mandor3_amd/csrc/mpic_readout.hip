@@ -1,0 +1,297 @@
+/*
+ * mpic_readout.hip -- results on their way to the host: node blocks of the
+ * fields, J and rho, the Tecplot node values and the marker records, laid out
+ * on the device as the host wants them and written straight to pinned host
+ * memory (source/type_mesh.c:285-311, source/IO_tecplot.c:131-214,
+ * source/core/plasma_IO.c:273-287 hold the layouts).
+ *
+ * What bounds it is PCIe (57 GB/s measured) and, for large results, the
+ * caller's memory: fresh pages cost the host more than the transfer.  A result
+ * larger than one slot goes through several host threads, each with two pinned
+ * slots, so that packing, transfer, page faults and copies overlap.  The
+ * copies component by component into pageable memory and the interleaving on
+ * one host thread that this replaces took 30 ms for the E and H of a
+ * 256 x 128 x 128 run (208 MB).
+ *
+ * Built with -ffp-contract=off: values are those of the host expressions.
+ */
+#include <string.h>
+
+#include <algorithm>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "mpic_readout.h"
+
+#define TPB 256
+
+static inline unsigned nblk(long n) { return (unsigned)((n + TPB - 1) / TPB); }
+
+/* ---------------- packing kernels ----------------
+ * Each writes items [first, first + count) of its result to out[0 .. count):
+ * consecutive lanes write consecutive words, since partial lines over PCIe
+ * cost as much as whole ones. */
+
+/* Doubles of nc interleaved components on the nodes lo .. lo + d - 1 per axis,
+ * k fastest. */
+template <class T>
+__global__ void k_pack_block(NodeBlock b, const T *F0, const T *F1, const T *F2, long first,
+                             long count, double *out)
+{
+    const long t = (long)blockIdx.x * TPB + threadIdx.x;
+    if (t >= count) return;
+    const long e = first + t;
+    const unsigned long node = (unsigned long)e / (unsigned)b.nc;
+    const int c = (int)(e - (long)node * b.nc);
+    const unsigned long r = node / (unsigned)b.d[2];
+    const int k = (int)(node - r * b.d[2]), i = (int)(r / (unsigned)b.d[1]),
+              j = (int)(r - (unsigned long)i * b.d[1]);
+    const T *F = c == 0 ? F0 : (c == 1 ? F1 : F2);
+    out[t] = (double)F[gidx(b.g, b.lo + i, b.lo + j, b.lo + k)];
+}
+
+/* Node values of the Tecplot records (source/IO_tecplot.c:131-153), nodes
+ * [0, n]: kind 0 (E, J) the mean of the two values along the component's axis,
+ * kind 1 (H) the mean of the four around the node, in the reference's order. */
+template <class T>
+__global__ void k_pack_nodes(Grid g, int kind, const T *F0, const T *F1, const T *F2, long first,
+                             long count, double *out)
+{
+    const long t = (long)blockIdx.x * TPB + threadIdx.x;
+    if (t >= count) return;
+    const long e = first + t;
+    const unsigned long node = (unsigned long)e / 3u;
+    const int c = (int)(e - (long)node * 3);
+    const unsigned long r = node / (unsigned)(g.n[2] + 1);
+    const int k = (int)(node - r * (g.n[2] + 1)), i = (int)(r / (unsigned)(g.n[1] + 1)),
+              j = (int)(r - (unsigned long)i * (g.n[1] + 1));
+    const T *F = c == 0 ? F0 : (c == 1 ? F1 : F2);
+    const long o = gidx(g, i, j, k), s[3] = {(long)g.GY * g.GZ, g.GZ, 1};
+    if (kind == 0) {
+        const long a = c == 0 ? s[0] : (c == 1 ? s[1] : s[2]);
+        out[t] = 0.5 * ((double)F[o] + (double)F[o + a]);
+    } else {
+        const long p = c == 0 ? s[1] : s[0], q = c == 2 ? s[1] : s[2];
+        out[t] = 0.25 * ((double)F[o] + (double)F[o + p] + (double)F[o + q] + (double)F[o + p + q]);
+    }
+}
+
+/* Words of marker_t records (source/type_marker.h:12-25): 8 per record of 64
+ * bytes (the last: id and zero padding), 7 of 56.  Markers of the order's
+ * positions, through its permutation. */
+__device__ static inline unsigned long long two_words(float lo, float hi)
+{
+    return (unsigned long long)__float_as_uint(hi) << 32 | __float_as_uint(lo);
+}
+
+__global__ void k_pack_markers32(MarkerBlock b, Markers32 m, long first, long count,
+                                 unsigned long long *out)
+{
+    const long t = (long)blockIdx.x * TPB + threadIdx.x;
+    if (t >= count) return;
+    const long e = first + t, u = e / b.words;
+    const int w = (int)(e - u * b.words);
+    const long q = b.perm[u];
+    if (w == 7) {
+        out[t] = (unsigned)m.id[q];
+        return;
+    }
+    if (w >= 3 && w < 6) {
+        const float4 v = m.mom[q];
+        out[t] = __double_as_longlong((double)(w == 3 ? v.x : (w == 4 ? v.y : v.z)));
+        return;
+    }
+    const float4 p = m.pos[q];
+    const int word = __float_as_int(p.x), key = word & ((1 << 29) - 1);
+    if (w == 6) {
+        out[t] = two_words(m.mom[q].w, b.qm[(unsigned)word >> 29]);
+        return;
+    }
+    const int loc = key & 63, tile = key >> 6;
+    const int t2 = tile % b.nt[2], r = tile / b.nt[2], t1 = r % b.nt[1], t0 = r / b.nt[1];
+    const int c = w == 0 ? 4 * t0 + (loc >> 4) : (w == 1 ? 4 * t1 + (loc >> 2 & 3) : 4 * t2 + (loc & 3));
+    out[t] = __double_as_longlong((c + (double)(w == 0 ? p.y : (w == 1 ? p.z : p.w))) * b.h[w]);
+}
+
+__global__ void k_pack_markers64(MarkerBlock b, Markers64 m, long first, long count,
+                                 unsigned long long *out)
+{
+    const long t = (long)blockIdx.x * TPB + threadIdx.x;
+    if (t >= count) return;
+    const long e = first + t, u = e / b.words;
+    const int w = (int)(e - u * b.words);
+    const long q = b.perm[u];
+    if (w == 7) {
+        out[t] = (unsigned)m.id[q];
+    } else if (w == 6) {
+        out[t] = two_words(m.w[q], m.qm[q]);
+    } else {
+        const double *s = w == 0 ? m.x : (w == 1 ? m.y : (w == 2 ? m.z : (w == 3 ? m.ux : (w == 4 ? m.uy : m.uz))));
+        out[t] = __double_as_longlong(s[q]);
+    }
+}
+
+int Readout::launch(hipStream_t s, long first, long count, void *out) const
+{
+    const unsigned nb = nblk(count);
+    switch (kind) {
+    case BLOCK32:
+        k_pack_block<float><<<nb, TPB, 0, s>>>(block, (const float *)F[0], (const float *)F[1],
+                                              (const float *)F[2], first, count, (double *)out);
+        break;
+    case BLOCK64:
+        k_pack_block<double><<<nb, TPB, 0, s>>>(block, (const double *)F[0], (const double *)F[1],
+                                               (const double *)F[2], first, count, (double *)out);
+        break;
+    case NODES32:
+        k_pack_nodes<float><<<nb, TPB, 0, s>>>(block.g, mean, (const float *)F[0], (const float *)F[1],
+                                              (const float *)F[2], first, count, (double *)out);
+        break;
+    case NODES64:
+        k_pack_nodes<double><<<nb, TPB, 0, s>>>(block.g, mean, (const double *)F[0],
+                                               (const double *)F[1], (const double *)F[2], first,
+                                               count, (double *)out);
+        break;
+    case MARKERS32:
+        k_pack_markers32<<<nb, TPB, 0, s>>>(markers, m32, first, count, (unsigned long long *)out);
+        break;
+    case MARKERS64:
+        k_pack_markers64<<<nb, TPB, 0, s>>>(markers, m64, first, count, (unsigned long long *)out);
+        break;
+    }
+    MPIC_CHECK(hipGetLastError());
+    return MPIC_OK;
+}
+
+/* ---------------- pinned slots ----------------
+ * One set per process, shared by all runs (calls that overlap take turns),
+ * bounded at WORKERS x 2 slots, allocated when first needed and freed with the
+ * last run. */
+#define SLOT_WORDS (1L << 18)          /* 2 MiB */
+#define WORKERS 8
+
+static struct {
+    std::mutex mu;
+    int        runs = 0;
+    long       words = 0;              /* allocated */
+    void      *mem = nullptr;
+} g_slots;
+
+void readout_ref(void)
+{
+    std::lock_guard<std::mutex> lk(g_slots.mu);
+    ++g_slots.runs;
+}
+
+void readout_unref(void)
+{
+    std::lock_guard<std::mutex> lk(g_slots.mu);
+    if (--g_slots.runs > 0) return;
+    if (g_slots.mem) hipHostFree(g_slots.mem);
+    g_slots.mem = nullptr;
+    g_slots.words = 0;
+}
+
+static int slots_reserve(long words)
+{
+    if (words <= g_slots.words) return MPIC_OK;
+    if (g_slots.mem) hipHostFree(g_slots.mem);
+    g_slots.mem = nullptr;
+    g_slots.words = 0;
+    MPIC_CHECK(hipHostMalloc(&g_slots.mem, 8 * words, hipHostMallocPortable));
+    g_slots.words = words;
+    return MPIC_OK;
+}
+
+/* Chunks w, w + nw, ... of the result through two slots: the next chunk is
+ * packed while this one is copied out. */
+static int worker(const Readout &r, int dev, hipStream_t s, char *dst, long total, long chunk,
+                  int w, int nw, char *slots)
+{
+    MPIC_CHECK(hipSetDevice(dev));
+    hipEvent_t ev[2];
+    for (hipEvent_t &e : ev) MPIC_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    int rc = MPIC_OK;
+    long at[2] = {-1, -1};
+    int slot = 0;
+    for (long c = w; rc == MPIC_OK; c += nw, slot ^= 1) {
+        const long first = c * chunk;
+        if (first < total) {
+            at[slot] = first;
+            rc = r.launch(s, first, std::min(chunk, total - first), slots + 8 * chunk * slot);
+            if (rc == MPIC_OK && hipEventRecord(ev[slot], s) != hipSuccess) rc = MPIC_ERR_DEVICE;
+        }
+        const int o = slot ^ 1;
+        if (rc == MPIC_OK && at[o] >= 0) {
+            if (hipEventSynchronize(ev[o]) != hipSuccess) {
+                rc = MPIC_ERR_DEVICE;
+                break;
+            }
+            memcpy(dst + 8 * at[o], slots + 8 * chunk * o, 8 * std::min(chunk, total - at[o]));
+            at[o] = -1;
+        }
+        if (first >= total && at[0] < 0 && at[1] < 0) break;
+    }
+    if (rc != MPIC_OK) hipStreamSynchronize(s);     /* nothing writes the slots any more */
+    for (hipEvent_t &e : ev) hipEventDestroy(e);
+    return rc;
+}
+
+int readout(const Readout *r, int n, int dev, hipStream_t s)
+{
+    std::lock_guard<std::mutex> lk(g_slots.mu);
+    long all = 0;
+    for (int q = 0; q < n; ++q) all += r[q].words;
+    if (all <= SLOT_WORDS) {
+        /* everything through one slot, one wait */
+        TRY_READOUT(slots_reserve(SLOT_WORDS));
+        char *at = (char *)g_slots.mem;
+        for (int q = 0; q < n; ++q) {
+            if (r[q].words) TRY_READOUT(r[q].launch(s, 0, r[q].words, at));
+            at += 8 * r[q].words;
+        }
+        MPIC_CHECK(hipStreamSynchronize(s));
+        at = (char *)g_slots.mem;
+        for (int q = 0; q < n; ++q) {
+            if (r[q].words) memcpy(r[q].dst, at, 8 * r[q].words);
+            at += 8 * r[q].words;
+        }
+        return MPIC_OK;
+    }
+    TRY_READOUT(slots_reserve(SLOT_WORDS * 2 * WORKERS));
+    for (int q = 0; q < n; ++q) {
+        const long total = r[q].words;
+        if (!total) continue;
+        const long chunk = SLOT_WORDS;
+        const int nw = (int)std::min<long>(WORKERS, (total + chunk - 1) / chunk);
+        int rc[WORKERS];
+        std::thread th[WORKERS];
+        char *mem = (char *)g_slots.mem;
+        int started = 0;
+        for (int w = 1; w < nw; ++w) {
+            try {
+                th[w] = std::thread([&, w] {
+                    rc[w] = worker(r[q], dev, s, (char *)r[q].dst, total, chunk, w, nw,
+                                   mem + 8 * chunk * 2 * w);
+                });
+                started = w;
+            } catch (...) {
+                break;                              /* no more threads: the rest here */
+            }
+        }
+        rc[0] = worker(r[q], dev, s, (char *)r[q].dst, total, chunk, 0, nw, mem);
+        int bad = rc[0];
+        for (int w = 1; w <= started; ++w) {
+            th[w].join();
+            if (rc[w] != MPIC_OK) bad = rc[w];
+        }
+        for (int w = started + 1; w < nw && bad == MPIC_OK; ++w)
+            bad = worker(r[q], dev, s, (char *)r[q].dst, total, chunk, w, nw, mem);
+        if (bad != MPIC_OK) {
+            mpic_set_error("a result could not be read back from the device");
+            return bad;
+        }
+    }
+    return MPIC_OK;
+}

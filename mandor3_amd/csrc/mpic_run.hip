@@ -16,6 +16,7 @@
 
 #include "mpic_internal.h"
 #include "mpic_launch.h"
+#include "mpic_readout.h"
 #include "mpic_tiles.h"
 
 thread_local Recorder *g_recorder = nullptr;
@@ -168,7 +169,6 @@ struct mpic_run {
     hipGraphExec_t exec[2];   /* one step from each of the two marker-buffer parities */
     int           exec_phase;      /* the run's phase when exec[0] was captured */
     int           ev_steps;   /* timed steps of the last mpic_advance */
-    double       *dnode;      /* node values of the Tecplot records, 3 (n+1)^3 doubles */
     int          *dprobe;     /* probe nodes, 3 ints each */
     double       *dsample;    /* probe samples, 6 doubles each */
     int           nprobes;
@@ -446,6 +446,7 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     MPIC_CHECK(hipSetDevice(cfg->device));
     TRY(scratch_setup(cfg->device));
     mpic_run *r = new mpic_run();
+    readout_ref();
     r->cfg = *cfg;
     r->dev = cfg->device;
     MPIC_CHECK(hipSetDevice(r->dev));
@@ -670,7 +671,6 @@ extern "C" int mpic_destroy(mpic_run_t *r)
     hipFree(r->djr);
     hipFree(r->dpart);
     hipFree(r->dring);
-    hipFree(r->dnode);
     hipFree(r->dprobe);
     hipFree(r->dsample);
     hipFree(r->spot.dprof);
@@ -684,13 +684,12 @@ extern "C" int mpic_destroy(mpic_run_t *r)
     for (int k = 0; k < 2; ++k)
         if (r->exec[k]) hipGraphExecDestroy(r->exec[k]);
     if (r->stream) hipStreamDestroy(r->stream);
+    readout_unref();
     delete r;
     return MPIC_OK;
 }
 
 /* ---------------- host <-> device data ---------------- */
-static int nodes_of(const Grid &g) { return (g.n[0] + 1) * (g.n[1] + 1) * (g.n[2] + 1); }
-
 template <class T>
 static int scatter_block(mpic_run *r, const double *src, T *const dst[3])
 {
@@ -708,19 +707,24 @@ static int scatter_block(mpic_run *r, const double *src, T *const dst[3])
     return MPIC_OK;
 }
 
+/* The node block lo .. lo + d - 1 (d = n + 1 - 2 lo) of three interleaved
+ * components (or one) as a result to read back. */
 template <class T>
-static int gather_block(mpic_run *r, T *const src[3], double *out)
+static Readout block_readout(const mpic_run *r, T *const F[3], int nc, int lo, double *out)
 {
-    const Grid &g = r->g;
-    std::vector<T> tmp((size_t)g.ncell);
-    for (int c = 0; c < 3; ++c) {
-        MPIC_CHECK(hipMemcpy(tmp.data(), src[c], sizeof(T) * g.ncell, hipMemcpyDeviceToHost));
-        long q = 0;
-        for (int i = 0; i <= g.n[0]; ++i)
-            for (int j = 0; j <= g.n[1]; ++j)
-                for (int k = 0; k <= g.n[2]; ++k, ++q) out[3 * q + c] = (double)tmp[gidx(g, i, j, k)];
+    Readout q = {};
+    q.kind = sizeof(T) == 4 ? Readout::BLOCK32 : Readout::BLOCK64;
+    q.block.g = r->g;
+    q.block.lo = lo;
+    q.block.nc = nc;
+    q.words = nc;
+    for (int a = 0; a < 3; ++a) {
+        q.block.d[a] = r->g.n[a] + 1 - 2 * lo;
+        q.words *= q.block.d[a];
     }
-    return MPIC_OK;
+    for (int c = 0; c < nc; ++c) q.F[c] = F[c];
+    q.dst = out;
+    return q;
 }
 
 extern "C" int mpic_set_fields(mpic_run_t *r, const double *E, const double *H)
@@ -742,32 +746,19 @@ extern "C" int mpic_get_fields(mpic_run_t *r, double *E, double *H)
 {
     if (!r) return MPIC_ERR_ARG;
     MPIC_CHECK(hipSetDevice(r->dev));
-    MPIC_CHECK(hipStreamSynchronize(r->stream));
-    if (r->fp32) {
-        if (E) TRY(gather_block(r, r->f32.E, E));
-        if (H) TRY(gather_block(r, r->f32.H, H));
-    } else {
-        if (E) TRY(gather_block(r, r->f.E, E));
-        if (H) TRY(gather_block(r, r->f.H, H));
-    }
-    return MPIC_OK;
+    Readout q[2];
+    int n = 0;
+    if (E) q[n++] = r->fp32 ? block_readout(r, r->f32.E, 3, 0, E) : block_readout(r, r->f.E, 3, 0, E);
+    if (H) q[n++] = r->fp32 ? block_readout(r, r->f32.H, 3, 0, H) : block_readout(r, r->f.H, 3, 0, H);
+    return readout(q, n, r->dev, r->stream);
 }
 
 extern "C" int mpic_get_J(mpic_run_t *r, double *J)
 {
     if (!r || !J) return MPIC_ERR_ARG;
     MPIC_CHECK(hipSetDevice(r->dev));
-    MPIC_CHECK(hipStreamSynchronize(r->stream));
-    const Grid &g = r->g;
-    std::vector<double> tmp((size_t)g.ncell);
-    for (int c = 0; c < 3; ++c) {
-        MPIC_CHECK(hipMemcpy(tmp.data(), r->jp.J[c], sizeof(double) * g.ncell, hipMemcpyDeviceToHost));
-        long q = 0;
-        for (int i = -2; i <= g.n[0] + 2; ++i)
-            for (int j = -2; j <= g.n[1] + 2; ++j)
-                for (int k = -2; k <= g.n[2] + 2; ++k, ++q) J[3 * q + c] = tmp[gidx(g, i, j, k)];
-    }
-    return MPIC_OK;
+    const Readout q = block_readout(r, r->jp.J, 3, -2, J);
+    return readout(&q, 1, r->dev, r->stream);
 }
 
 /* tecIO_saveFields / tecIO_saveCurrents payloads (source/IO_tecplot.c:
@@ -776,20 +767,16 @@ extern "C" int mpic_node_fields(mpic_run_t *r, int what, double *out)
 {
     if (!r || !out || what < 0 || what > 2) return MPIC_ERR_ARG;
     MPIC_CHECK(hipSetDevice(r->dev));
-    const Grid &g = r->g;
-    const long nodes = (long)(g.n[0] + 1) * (g.n[1] + 1) * (g.n[2] + 1);
-    if (!r->dnode) MPIC_CHECK(hipMalloc(&r->dnode, sizeof(double) * 3 * nodes));
-    if (what == 2) {
-        TRY(launch_node_fields<double>(r->stream, r->jp.J, g, 0, r->dnode));
-    } else if (r->fp32) {
-        TRY(launch_node_fields<float>(r->stream, what ? r->f32.H : r->f32.E, g, what, r->dnode));
-    } else {
-        TRY(launch_node_fields<double>(r->stream, what ? r->f.H : r->f.E, g, what, r->dnode));
-    }
-    MPIC_CHECK(hipMemcpyAsync(out, r->dnode, sizeof(double) * 3 * nodes, hipMemcpyDeviceToHost,
-                              r->stream));
-    MPIC_CHECK(hipStreamSynchronize(r->stream));
-    return MPIC_OK;
+    Readout q;
+    if (what == 2)
+        q = block_readout(r, r->jp.J, 3, 0, out);
+    else if (r->fp32)
+        q = block_readout(r, what ? r->f32.H : r->f32.E, 3, 0, out);
+    else
+        q = block_readout(r, what ? r->f.H : r->f.E, 3, 0, out);
+    q.kind = q.kind == Readout::BLOCK32 ? Readout::NODES32 : Readout::NODES64;
+    q.mean = what == 1;
+    return readout(&q, 1, r->dev, r->stream);
 }
 
 extern "C" int mpic_set_probes(mpic_run_t *r, const int *ijk, int nprobes)
@@ -1020,36 +1007,46 @@ static int load_split(mpic_run *r, std::vector<double> *d, std::vector<float> &w
     return MPIC_OK;
 }
 
+/* The order's N markers as records, through its permutation (every marker of
+ * a tiled run's order is live). */
+static int save_order(mpic_run *r, void *rec, long *n, int recsize, long N)
+{
+    if (N > *n) {
+        mpic_set_error("mpic_markers_save: output holds %ld markers, more are live", *n);
+        return MPIC_ERR_CAPACITY;
+    }
+    Readout q = {};
+    q.kind = r->fp32 ? Readout::MARKERS32 : Readout::MARKERS64;
+    q.words = N * (recsize / 8);
+    q.dst = rec;
+    q.markers.perm = r->tv.perm;
+    q.markers.words = recsize / 8;
+    for (int a = 0; a < 3; ++a) {
+        q.markers.nt[a] = r->tv.nt[a];
+        q.markers.h[a] = r->g.h[a];
+    }
+    for (int s = 0; s < 8; ++s) q.markers.qm[s] = r->qm[s];
+    q.m32 = r->m32;
+    q.m64 = r->m;
+    TRY(readout(&q, 1, r->dev, r->stream));
+    *n = N;
+    return MPIC_OK;
+}
+
+/* The loaded FP32 records, before mpic_init sorts them. */
 static int save_split(mpic_run *r, void *rec, long *n, int recsize, long N)
 {
     Markers32 &M = r->m32;
-    /* the N markers of the order: through the permutation once initialised
-     * (the buffer's first E records are written), else the loaded records */
-    long E = N;
-    std::vector<int32_t> order;
-    if (r->inited) {
-        int ext = 0;
-        MPIC_CHECK(hipMemcpy(&ext, r->tv.nmark + (r->parity ^ 1), sizeof(int), hipMemcpyDeviceToHost));
-        E = ext;
-        order.resize(N);
-        if (N)
-            MPIC_CHECK(hipMemcpy(order.data(), r->tv.perm, sizeof(int32_t) * N, hipMemcpyDeviceToHost));
-    }
-    std::vector<int32_t> id(E);
-    std::vector<float> pos(4 * E), mom(4 * E);
-    if (E) {
-        MPIC_CHECK(hipMemcpy(pos.data(), M.pos, sizeof(float4) * E, hipMemcpyDeviceToHost));
-        MPIC_CHECK(hipMemcpy(mom.data(), M.mom, sizeof(float4) * E, hipMemcpyDeviceToHost));
-        MPIC_CHECK(hipMemcpy(id.data(), M.id, sizeof(int32_t) * E, hipMemcpyDeviceToHost));
+    std::vector<int32_t> id(N);
+    std::vector<float> pos(4 * N), mom(4 * N);
+    if (N) {
+        MPIC_CHECK(hipMemcpy(pos.data(), M.pos, sizeof(float4) * N, hipMemcpyDeviceToHost));
+        MPIC_CHECK(hipMemcpy(mom.data(), M.mom, sizeof(float4) * N, hipMemcpyDeviceToHost));
+        MPIC_CHECK(hipMemcpy(id.data(), M.id, sizeof(int32_t) * N, hipMemcpyDeviceToHost));
     }
     char *dst = (char *)rec;
     long o = 0;
-    for (long u = 0; u < N; ++u) {
-        const long q = r->inited ? order[u] : u;
-        if (q < 0 || q >= E) {
-            mpic_set_error("mpic_markers_save: order entry %ld names record %ld of %ld", u, q, E);
-            return MPIC_ERR_STATE;
-        }
+    for (long q = 0; q < N; ++q) {
         int32_t word;
         memcpy(&word, &pos[4 * q], sizeof(word));
         if (word < 0) continue;
@@ -1148,42 +1145,25 @@ extern "C" int mpic_markers_save(mpic_run_t *r, void *rec, long *n, int recsize)
     MPIC_CHECK(hipStreamSynchronize(r->stream));
     long N = 0;
     TRY(live_n(r, &N));
+    if (r->tiled && r->inited) return save_order(r, rec, n, recsize, N);
     if (r->fp32) return save_split(r, rec, n, recsize, N);
-    /* the N markers of the order: through the permutation once a tiled run
-     * is initialised (the buffer's first E records are written), else the
-     * first N records */
-    const bool through = r->tiled && r->inited;
-    long E = N;
-    std::vector<int32_t> order;
-    if (through) {
-        int ext = 0;
-        MPIC_CHECK(hipMemcpy(&ext, r->tv.nmark + (r->parity ^ 1), sizeof(int), hipMemcpyDeviceToHost));
-        E = ext;
-        order.resize(N);
-        if (N)
-            MPIC_CHECK(hipMemcpy(order.data(), r->tv.perm, sizeof(int32_t) * N, hipMemcpyDeviceToHost));
-    }
+    /* the first N records (loaded, or an untiled run's) */
     std::vector<double> d[6];
-    std::vector<float> w(E), qm(E);
-    std::vector<int32_t> id(E);
+    std::vector<float> w(N), qm(N);
+    std::vector<int32_t> id(N);
     double *src[6] = {r->m.x, r->m.y, r->m.z, r->m.ux, r->m.uy, r->m.uz};
     for (int c = 0; c < 6; ++c) {
-        d[c].resize(E);
-        if (E) MPIC_CHECK(hipMemcpy(d[c].data(), src[c], sizeof(double) * E, hipMemcpyDeviceToHost));
+        d[c].resize(N);
+        if (N) MPIC_CHECK(hipMemcpy(d[c].data(), src[c], sizeof(double) * N, hipMemcpyDeviceToHost));
     }
-    if (E) {
-        MPIC_CHECK(hipMemcpy(w.data(), r->m.w, sizeof(float) * E, hipMemcpyDeviceToHost));
-        MPIC_CHECK(hipMemcpy(qm.data(), r->m.qm, sizeof(float) * E, hipMemcpyDeviceToHost));
-        MPIC_CHECK(hipMemcpy(id.data(), r->m.id, sizeof(int32_t) * E, hipMemcpyDeviceToHost));
+    if (N) {
+        MPIC_CHECK(hipMemcpy(w.data(), r->m.w, sizeof(float) * N, hipMemcpyDeviceToHost));
+        MPIC_CHECK(hipMemcpy(qm.data(), r->m.qm, sizeof(float) * N, hipMemcpyDeviceToHost));
+        MPIC_CHECK(hipMemcpy(id.data(), r->m.id, sizeof(int32_t) * N, hipMemcpyDeviceToHost));
     }
     long o = 0;
     char *dst = (char *)rec;
-    for (long u = 0; u < N; ++u) {
-        const long q = through ? order[u] : u;
-        if (q < 0 || q >= E) {
-            mpic_set_error("mpic_markers_save: order entry %ld names record %ld of %ld", u, q, E);
-            return MPIC_ERR_STATE;
-        }
+    for (long q = 0; q < N; ++q) {
         if (qm[q] == 0.0f) continue;
         if (o >= *n) {
             mpic_set_error("mpic_markers_save: output holds %ld markers, more are live", *n);
@@ -2851,16 +2831,9 @@ extern "C" int mpic_rho(mpic_run_t *r, double *rho)
     if (!r || !rho) return MPIC_ERR_ARG;
     MPIC_CHECK(hipSetDevice(r->dev));
     TRY(rho_into(r, r->rho2));
-    const Grid &g = r->g;
-    std::vector<double> tmp((size_t)g.ncell);
-    MPIC_CHECK(hipMemcpyAsync(tmp.data(), r->rho2, sizeof(double) * g.ncell, hipMemcpyDeviceToHost,
-                              r->stream));
-    MPIC_CHECK(hipStreamSynchronize(r->stream));
-    long q = 0;
-    for (int i = -2; i <= g.n[0] + 2; ++i)
-        for (int j = -2; j <= g.n[1] + 2; ++j)
-            for (int k = -2; k <= g.n[2] + 2; ++k, ++q) rho[q] = tmp[gidx(g, i, j, k)];
-    return MPIC_OK;
+    double *const F[3] = {r->rho2, nullptr, nullptr};
+    const Readout q = block_readout(r, F, 1, -2, rho);
+    return readout(&q, 1, r->dev, r->stream);
 }
 
 extern "C" int mpic_gauss_before(mpic_run_t *r)
