@@ -651,27 +651,26 @@ __device__ static inline void block_sum2(double we, double wb, double *part)
  * component squared where the node is that component's point of a cell of
  * [0,n)^3 -- Ex at (i+1,j,k), Ey at (i,j+1,k), Ez at (i,j,k+1), Hx at
  * (i,j+1,k+1), Hy at (i+1,j,k+1), Hz at (i+1,j+1,k) of cell (i,j,k).
- * A thread's partial over its few nodes is kept in the field precision
- * (FP32 form: ~1e-7 relative); the workgroup sums are FP64. */
+ * Summed in FP64 in both forms. */
 template <class T>
 __device__ static inline void energy_terms(const Grid &g, int i, int j, int k, T ex, T ey, T ez,
-                                           T hx, T hy, T hz, T &we, T &wb)
+                                           T hx, T hy, T hz, double &we, double &wb)
 {
     const bool i0 = i >= 0 && i < g.n[0], i1 = i >= 1 && i <= g.n[0];
     const bool j0 = j >= 0 && j < g.n[1], j1 = j >= 1 && j <= g.n[1];
     const bool k0 = k >= 0 && k < g.n[2], k1 = k >= 1 && k <= g.n[2];
-    if (i1 && j0 && k0) we += ex * ex;
-    if (i0 && j1 && k0) we += ey * ey;
-    if (i0 && j0 && k1) we += ez * ez;
-    if (i0 && j1 && k1) wb += hx * hx;
-    if (i1 && j0 && k1) wb += hy * hy;
-    if (i1 && j1 && k0) wb += hz * hz;
+    if (i1 && j0 && k0) we = __builtin_fma((double)ex, (double)ex, we);
+    if (i0 && j1 && k0) we = __builtin_fma((double)ey, (double)ey, we);
+    if (i0 && j0 && k1) we = __builtin_fma((double)ez, (double)ez, we);
+    if (i0 && j1 && k1) wb = __builtin_fma((double)hx, (double)hx, wb);
+    if (i1 && j0 && k1) wb = __builtin_fma((double)hy, (double)hy, wb);
+    if (i1 && j1 && k0) wb = __builtin_fma((double)hz, (double)hz, wb);
 }
 
 /* Nodes [1, n]^3. */
 template <class T>
 __device__ static inline void h_full(const HFullArgs<T> &A, const VBlock &b, const VBlock &gd,
-                                     T &we, T &wb)
+                                     double &we, double &wb)
 {
     typedef typename Vec<T>::v VT;
     constexpr int V = Vec<T>::N;
@@ -759,7 +758,8 @@ template <class T> struct HEdgeArgs {
 };
 
 template <class T>
-__device__ static inline void h_edge(const HEdgeArgs<T> &B, const VBlock &b, T &we, T &wb)
+__device__ static inline void h_edge(const HEdgeArgs<T> &B, const VBlock &b, double &we,
+                                     double &wb)
 {
     const HFullArgs<T> &A = B.h;
     const Grid &g = A.g;
@@ -818,9 +818,9 @@ template <class T> struct KernelDef<HFullArgs<T>> {
     static constexpr int kBlock = TPB;
     __device__ __forceinline__ static void body(const HFullArgs<T> &a, VBlock b, VBlock gd)
     {
-        T we = 0, wb = 0;
+        double we = 0, wb = 0;
         h_full<T>(a, b, gd, we, wb);
-        block_sum2((double)we, (double)wb, a.part + 2 * (long)b.x);
+        block_sum2(we, wb, a.part + 2 * (long)b.x);
     }
 };
 
@@ -828,9 +828,9 @@ template <class T> struct KernelDef<HEdgeArgs<T>> {
     static constexpr int kBlock = TPB;
     __device__ __forceinline__ static void body(const HEdgeArgs<T> &a, VBlock b, VBlock)
     {
-        T we = 0, wb = 0;
+        double we = 0, wb = 0;
         h_edge<T>(a, b, we, wb);
-        block_sum2((double)we, (double)wb, a.h.part + 2 * (long)b.x);
+        block_sum2(we, wb, a.h.part + 2 * (long)b.x);
     }
 };
 

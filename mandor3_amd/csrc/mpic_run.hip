@@ -176,7 +176,8 @@ struct mpic_run {
      * per step in a device ring indexed by the device step counter */
     double       *dpart;      /* energy partial sums, 2 per workgroup */
     int           nparts;
-    double       *dring;      /* DIAG_RING rows {W_E sum, W_M sum, WTx, WTy, WTz} */
+    double       *dring;      /* DIAG_RING rows {W_E sum, W_M sum, WTx, WTy, WTz}, in pinned host
+                                 memory: a step's kernel writes its row, the host reads it */
     std::vector<long>   ring_step;  /* step whose row a slot holds (-1: none) */
     std::vector<double> ring_time;  /* Time at the start of that step */
     int           capturing;  /* step_body is being recorded into graphs, not run */
@@ -597,7 +598,7 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     }
     r->nparts = h_full_blocks(g, cfg->precision == MPIC_FP32_SPLIT);
     MPIC_CHECK(hipMalloc(&r->dpart, sizeof(double) * 2 * r->nparts));
-    MPIC_CHECK(hipMalloc(&r->dring, sizeof(double) * 5 * DIAG_RING));
+    MPIC_CHECK(hipHostMalloc(&r->dring, sizeof(double) * 5 * DIAG_RING, hipHostMallocDefault));
     r->ring_step.assign(DIAG_RING, -1);
     r->ring_time.assign(DIAG_RING, 0.0);
     cap_geometry(cfg->n, cfg->bc, kUpdH, kFlH, r->cH);
@@ -670,7 +671,7 @@ extern "C" int mpic_destroy(mpic_run_t *r)
     hipFree(r->dstep);
     hipFree(r->djr);
     hipFree(r->dpart);
-    hipFree(r->dring);
+    if (r->dring) hipHostFree(r->dring);
     hipFree(r->dprobe);
     hipFree(r->dsample);
     hipFree(r->spot.dprof);
@@ -2139,19 +2140,20 @@ extern "C" int mpic_step(mpic_run_t *r, double *diag)
     if (!r) return MPIC_ERR_ARG;
     MPIC_CHECK(hipSetDevice(r->dev));
     if (!diag) return step_async(r, -1);
+    /* the loop step, then its ring row: the one thing waited for.  The row is
+     * handed back here, so the history does not keep it. */
     const double t0 = r->time;
-    double WE, WM;
-    TRY(mpic_em_h_half(r));
-    TRY(mpic_em_energy(r, &WE, &WM));
-    TRY(mpic_push_deposit(r));
-    TRY(mpic_temperature(r, diag + 3, diag + 4, diag + 5));
-    TRY(mpic_em_h_step(r));
-    TRY(mpic_em_e_start(r));
-    TRY(mpic_j_finish(r));
-    TRY(mpic_em_e_finish(r));
+    const long slot = r->step % DIAG_RING;
+    TRY(step_async(r, -1));
+    r->ring_step[slot] = -1;
+    MPIC_CHECK(hipStreamSynchronize(r->stream));
+    const double vol = 0.5 * r->g.h[0] * r->g.h[1] * r->g.h[2], *v = r->dring + 5 * slot;
     diag[0] = t0;
-    diag[1] = WE;
-    diag[2] = WM;
+    diag[1] = vol * v[0];
+    diag[2] = vol * v[1];
+    diag[3] = v[2];
+    diag[4] = v[3];
+    diag[5] = v[4];
     return MPIC_OK;
 }
 
@@ -2771,10 +2773,7 @@ extern "C" int mpic_diag_history(mpic_run_t *r, double *rows, int max_rows, int 
 {
     if (!r || !nrows || max_rows < 0 || (max_rows && !rows)) return MPIC_ERR_ARG;
     MPIC_CHECK(hipSetDevice(r->dev));
-    std::vector<double> ring(5 * DIAG_RING);
     MPIC_CHECK(hipStreamSynchronize(r->stream));
-    MPIC_CHECK(hipMemcpy(ring.data(), r->dring, sizeof(double) * ring.size(),
-                         hipMemcpyDeviceToHost));
     const double vol = 0.5 * r->g.h[0] * r->g.h[1] * r->g.h[2];
     std::vector<long> steps;
     for (long s = r->step - 1; s >= 0 && s >= r->step - DIAG_RING && (int)steps.size() < max_rows;
@@ -2784,7 +2783,7 @@ extern "C" int mpic_diag_history(mpic_run_t *r, double *rows, int max_rows, int 
     for (int q = 0; q < m; ++q) {
         const long s = steps[m - 1 - q], slot = s % DIAG_RING;
         double *o = rows + 6 * q;
-        const double *v = ring.data() + 5 * slot;
+        const double *v = r->dring + 5 * slot;
         o[0] = r->ring_time[slot];
         o[1] = vol * v[0];
         o[2] = vol * v[1];
