@@ -187,7 +187,7 @@ struct Job {
     std::atomic<int>  rc{MPIC_OK};
 };
 
-static struct Pool {
+struct Pool {
     std::mutex call;                   /* one read-out at a time */
     int        runs = 0;
     long       words = 0;              /* pinned words allocated */
@@ -198,7 +198,11 @@ static struct Pool {
     std::shared_ptr<Job> job;
     long       serial = 0;             /* of the job */
     bool       stop = false;
-} g_pool;
+};
+
+/* Never destroyed: a process that ends with runs still open ends with the
+ * helpers waiting, and destroying what they wait on would never return. */
+static Pool &g_pool = *new Pool;
 
 /* Chunks of the job through two slots: the next is packed while this one is
  * copied out.  A claimed chunk is always accounted for. */

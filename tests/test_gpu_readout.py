@@ -3,6 +3,9 @@ pinned slot (2^17 words), through one and through several host threads, and
 from several threads of the caller at once.  Everything bit for bit: the fields
 against what was set, node values against the host expressions on them,
 markers against what was loaded."""
+import os
+import subprocess
+import sys
 import threading
 
 import numpy as np
@@ -119,3 +122,16 @@ def test_several_threads_at_once():
     assert not bad
     for r in runs:
         r[0].close()
+
+
+def test_process_ends_with_a_run_still_open():
+    """The helper threads of a large read-out do not keep the process."""
+    code = ("import numpy as np, os, mandor3_amd as ma\n"
+            "r = ma.Run((60, 60, 60), (.05,) * 3, (3.,) * 3, .012, (0,) * 6)\n"
+            "z = np.ones(3 * r.nodes)\n"
+            "r.set_fields(z, z)\n"
+            "assert r.fields()[0].sum() == z.size\n"
+            "keep = [r]; keep.append(keep); ma.Run.__del__ = lambda self: None\n")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    p = subprocess.run([sys.executable, "-c", code], cwd=root, timeout=60)
+    assert p.returncode == 0
