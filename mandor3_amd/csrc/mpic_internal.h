@@ -205,8 +205,10 @@ int launch_jfold(hipStream_t s, const JPtrs &f, const Grid &g, int ea, int bc0, 
                  const int *jr);
 int launch_jfold_planes(hipStream_t s, const JPtrs &f, const Grid &g, const int bc[6],
                         const int *jr);
-/* VSP (beta, alpha, beta) sweeps along z, y, x of ncomp arrays on the padded grid. */
-int launch_vsp(hipStream_t s, double *const F[3], int ncomp, const Grid &g, double alpha);
+/* VSP (beta, alpha, beta) sweeps along z, y, x of ncomp arrays on the padded grid; jr: the
+ * x planes where they may be non-zero (null: all). */
+int launch_vsp(hipStream_t s, double *const F[3], int ncomp, const Grid &g, double alpha,
+               const int *jr);
 template <class T>
 int launch_tfsf_record(hipStream_t s, T *const E[3], T *const H[3], const Grid &g,
                        const TfsfSet &fe, const TfsfSet &fh, long maxvol, const double *factor,

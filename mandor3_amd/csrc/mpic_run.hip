@@ -1941,7 +1941,7 @@ extern "C" int mpic_em_e_start(mpic_run_t *r)
 static int vsp_J(mpic_run *r)
 {
     if (fabs(r->vsp - 1.0) < 1e-10) return MPIC_OK;
-    return launch_vsp(r->stream, r->jp.J, 3, r->g, r->vsp);
+    return launch_vsp(r->stream, r->jp.J, 3, r->g, r->vsp, r->djr + 4);
 }
 
 extern "C" int mpic_j_finish(mpic_run_t *r)
@@ -2822,7 +2822,7 @@ static int rho_into(mpic_run *r, double *rho)
     /* VSP_scalarSweep after the boundary fold (source/core/plasma_rho.c:153) */
     if (fabs(r->vsp - 1.0) >= 1e-10) {
         double *F[3] = {rho, nullptr, nullptr};
-        TRY(launch_vsp(r->stream, F, 1, r->g, r->vsp));
+        TRY(launch_vsp(r->stream, F, 1, r->g, r->vsp, nullptr));
     }
     return MPIC_OK;
 }
