@@ -533,7 +533,12 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     tv.perm = nullptr;
     if (r->tiled) MPIC_CHECK(hipMalloc(&tv.perm, sizeof(int) * r->cap));
     MPIC_CHECK(hipMalloc(&tv.active, sizeof(int) * tv.ntiles));
-    tv.chm = r->fp32 ? push32_item_markers() : 0;
+    /* The FP64 push adds its blocks to J by atomics, so a tile may also be cut
+     * there: with fewer tiles than a quarter of the CUs, where a wavefront's
+     * serial batches are the time (push in us without and with 512 markers
+     * per item: 12^3 box 21 / 14, 16^3 box, 64 tiles, 21 / 15; 20^3 box,
+     * 125 tiles, 22 / 26). */
+    tv.chm = r->fp32 ? push32_item_markers() : (tv.ntiles <= 64 ? 512 : 0);
     r->items_cap = items_capacity(tv.ntiles, r->cap, tv.chm);
     MPIC_CHECK(hipMalloc(&tv.item, sizeof(int4) * r->items_cap));
     MPIC_CHECK(hipMalloc(&tv.titem, sizeof(int2) * tv.ntiles));
