@@ -52,6 +52,22 @@ template <class A> struct WavesOf<A, std::void_t<decltype(KernelDef<A>::kWaves)>
  * scratch) for the kernel's life. */
 #define CAS __attribute__((address_space(4)))
 
+/* Reads one word of every 64 bytes of an argument struct, all loads in flight
+ * together, which brings it into the scalar cache: read only where they are
+ * used, its fields are a chain of scalar loads that each wait for a line of
+ * their own.  A small box's step is such latencies: 12^3 FP64 48.8 -> 45.1 us
+ * a step, 12^3 FP32 47.6 -> 43.2, 32^3 FP32 62.3 -> 60.5; boxes whose kernels
+ * are long enough to hide it stay as they were (64^3 full FP64 304.3 -> 303.9). */
+template <class A>
+__device__ static inline void touch(const CAS A *ap)
+{
+    const CAS unsigned *p = (const CAS unsigned *)ap;
+    unsigned v = 0;
+#pragma unroll
+    for (unsigned q = 0; q < sizeof(A) / 4; q += 16) v |= p[q];
+    asm volatile("" ::"s"(v));
+}
+
 /* A one-run launch's argument struct is its first kernel argument, at the
  * start of the kernel-argument segment: the body reads it there.  With the
  * struct passed by value the compiler keeps every field it uses live in
@@ -61,6 +77,7 @@ template <class A>
 __device__ static inline void run_one()
 {
     const CAS A *ap = (const CAS A *)__builtin_amdgcn_kernarg_segment_ptr();
+    touch(ap);
     const VBlock b = {blockIdx.x, blockIdx.y, blockIdx.z}, g = {gridDim.x, gridDim.y, gridDim.z};
     KernelDef<A>::body(*(const A *)ap, b, g);
 }
@@ -77,6 +94,7 @@ __device__ static inline void run_multi(const CAS A *__restrict__ args,
         if (tab[mid] <= blk) lo = mid;
         else hi = mid;
     }
+    touch(args + lo);
     const CAS unsigned *gr = tab + (n + 1) + 3 * lo;
     const VBlock g = {gr[0], gr[1], gr[2]};
     const unsigned L = blk - tab[lo];
