@@ -1526,12 +1526,15 @@ int launch_jfold(hipStream_t s, const JPtrs &f, const Grid &g, int ea, int bc0, 
     return launch_def(s, a, nb, 1);
 }
 
-/* Field energy sums, source/core/em.c:226-252 (FP64; block partial sums
- * combined with FP64 atomics, so the order differs from the CPU loop). */
+/* Field energy sums, source/core/em.c:226-252, in FP64: one partial sum pair
+ * per workgroup in pinned host memory, which the caller adds up in block
+ * order (with an atomic per workgroup instead, all of them on two addresses,
+ * a 45 x 38 x 31 box took 9.1 us and needed the sums cleared before and copied
+ * after; 4.0 us now).  Bound by latency up to about 64^3 nodes, by its six
+ * field reads beyond. */
 template <class T>
-__global__ void k_energy(FieldsT<T> f, Grid g, double *acc)
+__global__ void __launch_bounds__(TPB) k_energy(FieldsT<T> f, Grid g, double *part)
 {
-    __shared__ double se[TPB], sb[TPB];
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long tot = (long)g.n[0] * g.n[1] * g.n[2];
     double we = 0, wb = 0;
@@ -1545,29 +1548,35 @@ __global__ void k_energy(FieldsT<T> f, Grid g, double *acc)
         we += ex * ex + ey * ey + ez * ez;
         wb += hx * hx + hy * hy + hz * hz;
     }
-    se[threadIdx.x] = we;
-    sb[threadIdx.x] = wb;
-    __syncthreads();
-    for (int w = TPB / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            se[threadIdx.x] += se[threadIdx.x + w];
-            sb[threadIdx.x] += sb[threadIdx.x + w];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        atomicAdd(acc + 0, se[0]);
-        atomicAdd(acc + 1, sb[0]);
-    }
+    block_sum2(we, wb, part + 2 * blockIdx.x);
+}
+
+int energy_blocks(const Grid &g)
+{
+    const long nb = ((long)g.n[0] * g.n[1] * g.n[2] + TPB - 1) / TPB;
+    return (int)(nb > 2048 ? 2048 : nb);
 }
 
 template <class T>
-int launch_energy(hipStream_t s, const FieldsT<T> &f, const Grid &g, double *acc)
+int launch_energy(hipStream_t s, const FieldsT<T> &f, const Grid &g, double *part)
 {
-    long tot = (long)g.n[0] * g.n[1] * g.n[2];
-    long nb = (tot + TPB - 1) / TPB;
-    if (nb > 2048) nb = 2048;
-    k_energy<T><<<(unsigned)nb, TPB, 0, s>>>(f, g, acc);
+    k_energy<T><<<(unsigned)energy_blocks(g), TPB, 0, s>>>(f, g, part);
+    MPIC_CHECK(hipGetLastError());
+    return MPIC_OK;
+}
+
+/* The slots of the kinetic sums (256 of 4 doubles) to pinned host memory: the
+ * host adds them in slot order.  A copy engine's or blit's copy of these 8 KiB
+ * costs the call more than this launch does. */
+__global__ void __launch_bounds__(KIN_SLOTS) k_kin_out(const double4 *kin, double4 *out)
+{
+    out[threadIdx.x] = kin[threadIdx.x];
+}
+
+int launch_kin_out(hipStream_t s, const double *kin, double *out)
+{
+    static_assert(KIN_STRIDE == 4, "one double4 per slot");
+    k_kin_out<<<1, KIN_SLOTS, 0, s>>>((const double4 *)kin, (double4 *)out);
     MPIC_CHECK(hipGetLastError());
     return MPIC_OK;
 }

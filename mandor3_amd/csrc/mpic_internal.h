@@ -216,7 +216,11 @@ int launch_tfsf_record(hipStream_t s, T *const E[3], T *const H[3], const Grid &
 template <class T>
 int launch_probes(hipStream_t s, T *const E[3], T *const H[3], const Grid &g, const int *ijk,
                   int np, double *out);
-template <class T> int launch_energy(hipStream_t s, const FieldsT<T> &f, const Grid &g, double *acc);
+/* em_energy partial sums, two doubles per workgroup; energy_blocks workgroups. */
+int energy_blocks(const Grid &g);
+template <class T> int launch_energy(hipStream_t s, const FieldsT<T> &f, const Grid &g, double *part);
+/* The kinetic sums' slots to pinned host memory. */
+int launch_kin_out(hipStream_t s, const double *kin, double *out);
 /* Loop-body diagnostics: the one-pass H update writes em_energy partial sums
  * (two doubles per workgroup, h_full_blocks(g, fp32) workgroups); the ring
  * row {W_E sum, W_M sum, WTx, WTy, WTz} of the device step counter's step

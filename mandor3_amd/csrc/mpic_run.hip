@@ -142,10 +142,11 @@ struct mpic_run {
     std::vector<double *> murbuf;
     std::vector<Laser> lasers;
     PushConsts    pc;
-    double       *dacc;       /* device scratch: [0..1] energy, [5..6] gauss */
+    double       *dacc;       /* device scratch: [5..6] gauss */
+    double       *henergy;    /* pinned: em_energy partial sums, 2 per workgroup */
     double       *hacc;       /* pinned host mirror */
     double       *dkin;       /* the push's kinetic sums: KIN_SLOTS partial sums */
-    double       *hkin;       /* pinned host mirror */
+    double       *hkin;       /* pinned: mpic_temperature's copy of the sums */
     unsigned     *derr;       /* device error flags (bit 0: marker off the grid, bit 1: a
                                  tile scan's wait for an earlier workgroup ran out) */
     int           stage;
@@ -170,7 +171,7 @@ struct mpic_run {
     int           exec_phase;      /* the run's phase when exec[0] was captured */
     int           ev_steps;   /* timed steps of the last mpic_advance */
     int          *dprobe;     /* probe nodes, 3 ints each */
-    double       *dsample;    /* probe samples, 6 doubles each */
+    double       *hsample;    /* pinned: probe samples, 6 doubles each */
     int           nprobes;
     /* diagnostics of the loop body (em_energy, plasma_temperature), one row
      * per step in a device ring indexed by the device step counter */
@@ -585,6 +586,8 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     r->n = 0;
     MPIC_CHECK(hipMalloc(&r->dacc, sizeof(double) * 8));
     MPIC_CHECK(hipHostMalloc(&r->hacc, sizeof(double) * 8, hipHostMallocDefault));
+    MPIC_CHECK(hipHostMalloc(&r->henergy, sizeof(double) * 2 * energy_blocks(r->g),
+                             hipHostMallocDefault));
     MPIC_CHECK(hipMalloc(&r->dkin, sizeof(double) * KIN_SLOTS * KIN_STRIDE));
     MPIC_CHECK(hipHostMalloc(&r->hkin, sizeof(double) * KIN_SLOTS * KIN_STRIDE,
                              hipHostMallocDefault));
@@ -666,6 +669,7 @@ extern "C" int mpic_destroy(mpic_run_t *r)
     if (r->hkin) hipHostFree(r->hkin);
     hipFree(r->derr);
     if (r->hacc) hipHostFree(r->hacc);
+    if (r->henergy) hipHostFree(r->henergy);
     for (double *b : r->murbuf) hipFree(b);
     for (Laser &l : r->lasers) hipFree(l.dmap);
     for (hipEvent_t e : r->evpool) hipEventDestroy(e);
@@ -678,7 +682,7 @@ extern "C" int mpic_destroy(mpic_run_t *r)
     hipFree(r->dpart);
     if (r->dring) hipHostFree(r->dring);
     hipFree(r->dprobe);
-    hipFree(r->dsample);
+    if (r->hsample) hipHostFree(r->hsample);
     hipFree(r->spot.dprof);
     hipFree(r->tfsf.ddata);
     hipFree(r->trec.dbuf);
@@ -798,13 +802,13 @@ extern "C" int mpic_set_probes(mpic_run_t *r, const int *ijk, int nprobes)
     MPIC_CHECK(hipSetDevice(r->dev));
     MPIC_CHECK(hipStreamSynchronize(r->stream));
     hipFree(r->dprobe);
-    hipFree(r->dsample);
+    if (r->hsample) hipHostFree(r->hsample);
     r->dprobe = nullptr;
-    r->dsample = nullptr;
+    r->hsample = nullptr;
     r->nprobes = 0;
     if (!nprobes) return MPIC_OK;
     MPIC_CHECK(hipMalloc(&r->dprobe, sizeof(int) * 3 * nprobes));
-    MPIC_CHECK(hipMalloc(&r->dsample, sizeof(double) * 6 * nprobes));
+    MPIC_CHECK(hipHostMalloc(&r->hsample, sizeof(double) * 6 * nprobes, hipHostMallocDefault));
     MPIC_CHECK(hipMemcpy(r->dprobe, ijk, sizeof(int) * 3 * nprobes, hipMemcpyHostToDevice));
     r->nprobes = nprobes;
     return MPIC_OK;
@@ -819,13 +823,12 @@ extern "C" int mpic_probe_sample(mpic_run_t *r, double *out)
     MPIC_CHECK(hipSetDevice(r->dev));
     if (r->fp32)
         TRY(launch_probes<float>(r->stream, r->f32.E, r->f32.H, r->g, r->dprobe, r->nprobes,
-                                 r->dsample));
+                                 r->hsample));
     else
         TRY(launch_probes<double>(r->stream, r->f.E, r->f.H, r->g, r->dprobe, r->nprobes,
-                                  r->dsample));
-    MPIC_CHECK(hipMemcpyAsync(out, r->dsample, sizeof(double) * 6 * r->nprobes,
-                              hipMemcpyDeviceToHost, r->stream));
+                                  r->hsample));
     MPIC_CHECK(hipStreamSynchronize(r->stream));
+    memcpy(out, r->hsample, sizeof(double) * 6 * r->nprobes);
     return MPIC_OK;
 }
 
@@ -1831,13 +1834,16 @@ extern "C" int mpic_em_energy(mpic_run_t *r, double *W_E, double *W_M)
 {
     if (!r) return MPIC_ERR_ARG;
     MPIC_CHECK(hipSetDevice(r->dev));
-    MPIC_CHECK(hipMemsetAsync(r->dacc, 0, 2 * sizeof(double), r->stream));
-    FCALL(launch_energy, r->g, r->dacc);
-    MPIC_CHECK(hipMemcpyAsync(r->hacc, r->dacc, 2 * sizeof(double), hipMemcpyDeviceToHost, r->stream));
+    FCALL(launch_energy, r->g, r->henergy);
     MPIC_CHECK(hipStreamSynchronize(r->stream));
+    double we = 0, wb = 0;
+    for (int q = 0, nb = energy_blocks(r->g); q < nb; ++q) {
+        we += r->henergy[2 * q];
+        wb += r->henergy[2 * q + 1];
+    }
     const double *h = r->g.h;
-    if (W_E) *W_E = 0.5 * r->hacc[0] * h[0] * h[1] * h[2];
-    if (W_M) *W_M = 0.5 * r->hacc[1] * h[0] * h[1] * h[2];
+    if (W_E) *W_E = 0.5 * we * h[0] * h[1] * h[2];
+    if (W_M) *W_M = 0.5 * wb * h[0] * h[1] * h[2];
     return MPIC_OK;
 }
 
@@ -1885,8 +1891,7 @@ extern "C" int mpic_temperature(mpic_run_t *r, double *WTx, double *WTy, double 
 {
     if (!r) return MPIC_ERR_ARG;
     MPIC_CHECK(hipSetDevice(r->dev));
-    MPIC_CHECK(hipMemcpyAsync(r->hkin, r->dkin, sizeof(double) * KIN_SLOTS * KIN_STRIDE,
-                              hipMemcpyDeviceToHost, r->stream));
+    TRY(launch_kin_out(r->stream, r->dkin, r->hkin));
     MPIC_CHECK(hipStreamSynchronize(r->stream));
     double w[3] = {0, 0, 0};
     for (int q = 0; q < KIN_SLOTS; ++q)

@@ -47,3 +47,32 @@ def test_kinetic_sums(n, prec):
     # FP32: momenta and each term rounded to 2^-24, all terms of one sign
     np.testing.assert_allclose(got, want, rtol=1e-11 if prec == ma.FP64 else 1e-6)
     r.close()
+
+
+@pytest.mark.parametrize("prec", [ma.FP64, ma.FP32_SPLIT])
+@pytest.mark.parametrize("n", [(7, 7, 7), (16, 16, 16), (16, 16, 17), (128, 64, 65)])
+def test_field_energy_sums(n, prec):
+    """Two, 16, 17 and 2048 (the most: a thread then sums several nodes)
+    workgroups, against the sums over em.c:226-252's points in longdouble."""
+    rng = np.random.default_rng(7)
+    h = (0.1, 0.2, 0.05)
+    r = ma.Run(n, h, tuple(a * b for a, b in zip(n, h)), 0.01, [0] * 6, 0.0, precision=prec)
+    d = tuple(a + 1 for a in n)
+    E, H = (rng.standard_normal(d + (3,)) for _ in range(2))
+    if prec == ma.FP32_SPLIT:
+        E, H = (F.astype(np.float32).astype(float) for F in (E, H))
+    r.set_fields(E.ravel(), H.ravel())
+
+    def total(F, off):
+        s = np.longdouble(0)
+        for c in range(3):
+            sl = tuple(slice(off[c][a], off[c][a] + n[a]) for a in range(3))
+            s += (F[sl + (c,)].astype(np.longdouble) ** 2).sum()
+        return float(s * 0.5 * h[0] * h[1] * h[2])
+
+    want = (total(E, ((1, 0, 0), (0, 1, 0), (0, 0, 1))),
+            total(H, ((0, 1, 1), (1, 0, 1), (1, 1, 0))))
+    # a thread adds at most 2 nodes of 3 squares, then 8 tree levels and 2048
+    # partial sums, all positive: (6 + 8 + 2048) 2^-53 < 3e-13
+    np.testing.assert_allclose(r.energy(), want, rtol=3e-13)
+    r.close()
