@@ -1973,9 +1973,9 @@ int launch_h_full_jclear(hipStream_t s, const FieldsT<T> &f, const Grid &g, cons
 }
 
 int launch_jgather32(hipStream_t s, const JPtrs &j, const Grid &g, const TileView &tv,
-                     const float *tj, int nblocks)
+                     const float *tj, int parity, int nblocks)
 {
-    JGatherArgs a = {j, g, tv, tj};
+    JGatherArgs a = {j, g, tv, tj, parity};
     return launch_def(s, a, (unsigned)nblocks);
 }
 
@@ -2043,8 +2043,8 @@ template <> struct KernelDef<DiagRingArgs> {
  * launch costs about 4 us, so the links of the chains share launches with the
  * sort's passes (and the FP32 form's J gather), the few workgroups of the
  * links first, so that they do not wait behind the many of a pass:
- *   FP32  [E caps | J gather]   [x walls | x folds | scan]
- *         [ring | y, z walls | y, z folds | rank]
+ *   FP32  [scan | E caps | J gather]   [ring | x walls | x folds | rank]
+ *         [y, z walls | y, z folds]
  *   FP64  [E caps | x folds | scan]   [ring | x walls | y, z folds | rank]
  *         [y, z walls]
  * in place of ten launches.  The two walls of an axis (7 cells or more)
@@ -2077,14 +2077,14 @@ int launch_after_push(hipStream_t s, const FieldsT<T> &f, const Grid &g, const A
     const RankArgs rk = {*p.tv, p.nbound, p.parity};
     const dim3 gsc(p.sorted ? sc.nb : 0), grk(p.sorted ? rank_blocks(p.nbound) : 0);
     const DiagRingArgs ring = {p.part, p.nparts, p.kin, p.ring, p.step, p.ringcap};
-    if (sizeof(T) == 4) {
-        const JGatherArgs jg = {p.jp, g, *p.tv, p.tj};
-        TRY_LAUNCH(launch_pair(s, cap, gcap, jg, dim3(p.gather_blocks)));
-        if (p.after_gather) MPIC_CHECK(hipEventRecord(p.after_gather, s));
-        TRY_LAUNCH(launch_three(s, fx, gfx, jx, gjx, sc, gsc));
-        return launch_three(s, pair_of(ring, 1, fp, planes), dim3(1 + planes), jp, gjp, rk, grk);
-    }
     const unsigned nfx = gfx.x * gfx.y;
+    if (sizeof(T) == 4) {
+        const JGatherArgs jg = {p.jp, g, *p.tv, p.tj, p.parity};
+        TRY_LAUNCH(launch_three(s, ScanLeanArgs{sc}, gsc, cap, gcap, jg, dim3(p.gather_blocks)));
+        if (p.after_gather) MPIC_CHECK(hipEventRecord(p.after_gather, s));
+        TRY_LAUNCH(launch_three(s, pair_of(ring, 1, fx, gfx), dim3(1 + nfx), jx, gjx, rk, grk));
+        return launch_pair(s, fp, dim3(planes), jp, gjp);
+    }
     TRY_LAUNCH(launch_three(s, cap, gcap, jx, gjx, sc, gsc));
     TRY_LAUNCH(launch_three(s, pair_of(ring, 1, fx, gfx), dim3(1 + nfx), jp, gjp, rk, grk));
     return launch_def(s, fp, planes);

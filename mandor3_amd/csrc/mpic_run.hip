@@ -533,7 +533,7 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     MPIC_CHECK(hipMalloc(&tv.key, sizeof(int) * r->cap));
     tv.perm = nullptr;
     if (r->tiled) MPIC_CHECK(hipMalloc(&tv.perm, sizeof(int) * r->cap));
-    MPIC_CHECK(hipMalloc(&tv.active, sizeof(int) * tv.ntiles));
+    MPIC_CHECK(hipMalloc(&tv.active, sizeof(int) * 2 * tv.ntiles));
     /* The FP64 push adds its blocks to J by atomics, so a tile may also be cut
      * there: with fewer tiles than a quarter of the CUs, where a wavefront's
      * serial batches are the time (push in us without and with 512 markers
@@ -542,14 +542,14 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     tv.chm = r->fp32 ? push32_item_markers() : (tv.ntiles <= 64 ? 512 : 0);
     r->items_cap = items_capacity(tv.ntiles, r->cap, tv.chm);
     MPIC_CHECK(hipMalloc(&tv.item, sizeof(int4) * r->items_cap));
-    MPIC_CHECK(hipMalloc(&tv.titem, sizeof(int2) * tv.ntiles));
-    MPIC_CHECK(hipMemsetAsync(tv.titem, 0, sizeof(int2) * tv.ntiles, r->stream));
+    MPIC_CHECK(hipMalloc(&tv.titem, sizeof(int2) * 2 * tv.ntiles));
+    MPIC_CHECK(hipMemsetAsync(tv.titem, 0, sizeof(int2) * 2 * tv.ntiles, r->stream));
     if (r->fp32) MPIC_CHECK(hipMalloc(&r->tj, sizeof(float) * TJB * (size_t)r->items_cap));
-    MPIC_CHECK(hipMalloc(&tv.nactive, sizeof(int) * 6));
-    tv.nmark = tv.nactive + 1;
-    tv.nitems = tv.nactive + 3;
-    tv.xr = tv.nactive + 4;
-    MPIC_CHECK(hipMemsetAsync(tv.nactive, 0, sizeof(int) * 4, r->stream));
+    MPIC_CHECK(hipMalloc(&tv.nactive, sizeof(int) * 7));
+    tv.nmark = tv.nactive + 2;
+    tv.nitems = tv.nactive + 4;
+    tv.xr = tv.nactive + 5;
+    MPIC_CHECK(hipMemsetAsync(tv.nactive, 0, sizeof(int) * 5, r->stream));
     {
         /* a tiled run without markers pushes nothing */
         const int xr[2] = {r->tiled ? 0 : -2, r->tiled ? -1 : g.n[0] + 2};
@@ -1881,7 +1881,7 @@ extern "C" int mpic_push_deposit(mpic_run_t *r)
                       r->tiled ? 0 : 1));
     TRY(push(r, r->f32, r->f));
     if (r->fp32)
-        TRY(launch_jgather32(r->stream, r->jp, r->g, r->tv, r->tj, r->gather_blocks));
+        TRY(launch_jgather32(r->stream, r->jp, r->g, r->tv, r->tj, r->parity, r->gather_blocks));
     /* per-step marker sort by cell (keys written by the push) */
     if (r->tiled) TRY(sort_pass(r, 0));
     return MPIC_OK;

@@ -11,7 +11,9 @@
 #include "mpic_launch.h"
 #include "mpic_tiles.h"
 
-#define SB MPIC_SCAN_BLOCK       /* tiles per scan block */
+#define SCAN_TPB 256
+#define SCAN_WT 64               /* tiles per wavefront of the scan */
+#define SB (SCAN_TPB / 64 * SCAN_WT) /* tiles per scan workgroup */
 #define JG_TPB 256
 
 /* The tile scan, in one pass: every workgroup takes SB consecutive tiles,
@@ -34,8 +36,13 @@
  * all of them), i.e. after every workgroup has read it.
  *
  * Layout of the counts: a tile's 64 per-key counts are 16 int4; 16 lanes of
- * a wavefront read one tile (coalesced), a wavefront four tiles per load,
- * and keep them in registers for the per-key offsets written at the end. */
+ * a wavefront read one tile (coalesced), a wavefront four tiles per load.
+ * With LD = SCAN_WT / 4 all its loads are in flight together and stay in
+ * registers for the per-key offsets written at the end (130 VGPRs); with
+ * fewer, they are read in rounds of LD and again at the end, which costs
+ * 1.5 us on a 32^3 box but leaves the launch the J gather's registers: shared
+ * with the 130 of the former, the gather of laser-foil took 48 us, with LD = 8
+ * 39 (34 and 13 for gather and scan in launches of their own). */
 #define NSCAN 3
 #define SCAN_SPIN (1 << 20)
 struct ScanArgs {
@@ -71,29 +78,31 @@ __device__ static inline int wave_sum(int x)
     return x;
 }
 
+template <int LD>
 __device__ static inline void scan_pass(const ScanArgs &A, const VBlock &bk)
 {
+    constexpr int NV = SCAN_WT / 4;                  /* loads of a wavefront */
     const TileView &tv = A.tv;
-    __shared__ int wsum[NSCAN][SB / 64];
+    __shared__ int wsum[NSCAN][SCAN_TPB / 64];
     __shared__ int spre[NSCAN];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, blk = (int)bk.x;
-    const int wt0 = blk * SB + w * 64;               /* first tile of the wavefront */
+    const int wt0 = blk * SB + w * SCAN_WT;          /* first tile of the wavefront */
     const int4 *cnt4 = (const int4 *)tv.count;
-    int4 x[16];
-    int ex[16];                                      /* this lane's first key, within its tile */
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int t = wt0 + v * 4 + (lane >> 4);
-        x[v] = t < tv.ntiles ? cnt4[(long)t * 16 + (lane & 15)] : make_int4(0, 0, 0, 0);
-    }
     int c = 0;                                       /* markers of tile wt0 + lane */
+    int4 x[LD];
+#pragma unroll 1
+    for (int v0 = 0; v0 < NV; v0 += LD) {
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int s = x[v].x + x[v].y + x[v].z + x[v].w;
-        const int inc = row_sum(s);
-        ex[v] = inc - s;
-        const int tot = __shfl(inc, (lane & 3) * 16 + 15, 64);   /* tile v*4 + (lane & 3) */
-        if ((lane >> 2) == v) c = tot;
+        for (int v = 0; v < LD; ++v) {
+            const int t = wt0 + (v0 + v) * 4 + (lane >> 4);
+            x[v] = t < tv.ntiles ? cnt4[(long)t * 16 + (lane & 15)] : make_int4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int v = 0; v < LD; ++v) {
+            const int inc = row_sum(x[v].x + x[v].y + x[v].z + x[v].w);
+            const int tot = __shfl(inc, (lane & 3) * 16 + 15, 64);   /* tile 4 (v0 + v) + (lane & 3) */
+            if ((lane >> 2) == v0 + v) c = tot;
+        }
     }
     const int own[NSCAN] = {c, c > 0, tile_items(c, tv.chm)};
     int inc[NSCAN];
@@ -105,7 +114,7 @@ __device__ static inline void scan_pass(const ScanArgs &A, const VBlock &bk)
     int agg[NSCAN];
     for (int a = 0; a < NSCAN; ++a) {
         agg[a] = 0;
-        for (int q = 0; q < SB / 64; ++q) {
+        for (int q = 0; q < SCAN_TPB / 64; ++q) {
             if (q < w) inc[a] += wsum[a][q];
             agg[a] += wsum[a][q];
         }
@@ -174,7 +183,7 @@ __device__ static inline void scan_pass(const ScanArgs &A, const VBlock &bk)
             const int tot = pre[0] + agg[0], na = pre[1] + agg[1], ni = pre[2] + agg[2];
             tv.off[tv.ncellp] = tot;
             tv.toff[tv.ntiles] = tot;
-            *tv.nactive = na;
+            tv.nactive[A.parity_next] = na;
             *tv.nitems = ni;
             tv.nmark[A.parity_next] = tot;
             *A.seq = seq + 1;
@@ -184,28 +193,38 @@ __device__ static inline void scan_pass(const ScanArgs &A, const VBlock &bk)
     /* tile offsets, the active list, the work items */
     const int base = spre[0] + inc[0] - own[0];
     const int t = wt0 + lane;
-    if (t < tv.ntiles) {
+    const long po = (long)A.parity_next * tv.ntiles;
+    if (lane < SCAN_WT && t < tv.ntiles) {
         tv.toff[t] = base;
         const int is = spre[2] + inc[2] - own[2], nu = own[2];
         if (c > 0) {
-            tv.active[spre[1] + inc[1] - own[1]] = t;
+            tv.active[po + spre[1] + inc[1] - own[1]] = t;
             /* item u of nu: an even share of the tile's markers */
             for (int u = 0; u < nu; ++u)
                 tv.item[is + u] = make_int4(t, base + (int)((long)u * c / nu),
                                             base + (int)((long)(u + 1) * c / nu), 0);
         }
-        tv.titem[t] = make_int2(is, nu);
+        tv.titem[po + t] = make_int2(is, nu);
     }
     /* per-key offsets and cursors of the non-empty tiles, counters reset
      * (entries of empty tiles are not maintained) */
     int4 *off4 = (int4 *)tv.off, *cur4 = (int4 *)tv.cursor, *cnt4w = (int4 *)tv.count;
+#pragma unroll 1
+    for (int v0 = 0; v0 < NV; v0 += LD) {
+        int tb[LD];
+        bool on[LD];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int tt = v * 4 + (lane >> 4);
-        const int tb = __shfl(base, tt, 64), tc = __shfl(c, tt, 64);
-        if (tc > 0) {
-            const long q = (long)(wt0 + tt) * 16 + (lane & 15);
-            const int o0 = tb + ex[v];
+        for (int v = 0; v < LD; ++v) {
+            const int tt = (v0 + v) * 4 + (lane >> 4);
+            tb[v] = __shfl(base, tt, 64);
+            on[v] = __shfl(c, tt, 64) > 0;
+            if (LD < NV) x[v] = on[v] ? cnt4[(long)(wt0 + tt) * 16 + (lane & 15)] : make_int4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int v = 0; v < LD; ++v) {
+            const int s = x[v].x + x[v].y + x[v].z + x[v].w, o0 = tb[v] + row_sum(s) - s;
+            if (!on[v]) continue;
+            const long q = (long)(wt0 + (v0 + v) * 4 + (lane >> 4)) * 16 + (lane & 15);
             const int4 o = make_int4(o0, o0 + x[v].x, o0 + x[v].x + x[v].y,
                                      o0 + x[v].x + x[v].y + x[v].z);
             off4[q] = o;
@@ -216,10 +235,22 @@ __device__ static inline void scan_pass(const ScanArgs &A, const VBlock &bk)
 }
 
 template <> struct KernelDef<ScanArgs> {
-    static constexpr int kBlock = SB;
+    static constexpr int kBlock = SCAN_TPB;
     __device__ __forceinline__ static void body(const ScanArgs &a, VBlock b, VBlock)
     {
-        scan_pass(a, b);
+        scan_pass<SCAN_WT / 4>(a, b);
+    }
+};
+
+/* The scan in few registers, for a launch shared with the J gather. */
+struct ScanLeanArgs : ScanArgs {
+};
+
+template <> struct KernelDef<ScanLeanArgs> {
+    static constexpr int kBlock = SCAN_TPB;
+    __device__ __forceinline__ static void body(const ScanLeanArgs &a, VBlock b, VBlock)
+    {
+        scan_pass<8>(a, b);
     }
 };
 
@@ -277,9 +308,10 @@ template <> struct KernelDef<RankArgs> {
     {
         if (b.x == 0 && threadIdx.x == 0) {
             /* the active list is in tile order, tiles i-major */
-            const int na = *a.tv.nactive, tpp = a.tv.nt[1] * a.tv.nt[2];
-            a.tv.xr[0] = na > 0 ? 4 * (a.tv.active[0] / tpp) : 0;
-            a.tv.xr[1] = na > 0 ? 4 * (a.tv.active[na - 1] / tpp) + 5 : -1;
+            const int nx = a.parity ^ 1, na = a.tv.nactive[nx], tpp = a.tv.nt[1] * a.tv.nt[2];
+            const int *act = a.tv.active + (long)nx * a.tv.ntiles;
+            a.tv.xr[0] = na > 0 ? 4 * (act[0] / tpp) : 0;
+            a.tv.xr[1] = na > 0 ? 4 * (act[na - 1] / tpp) + 5 : -1;
         }
         rank_pass(a.tv, a.nbound, a.parity, (long)b.x * (256 * RANK_BATCHES));
     }
@@ -317,16 +349,19 @@ struct JGatherArgs {
     Grid         g;
     TileView     tv;
     const float *tj;
+    int          parity;     /* of the order that was pushed */
 };
 
 __device__ __forceinline__ static void jgather32(const JPtrs &v, const Grid &g, const TileView &tv,
-                                                const float *tj, const VBlock &bk,
-                                                const VBlock &gd)
+                                                const float *tj, int parity,
+                                                const VBlock &bk, const VBlock &gd)
 {
     __shared__ int nfirst[27], nitem[27];    /* items of the 3x3x3 tiles around t (0: none) */
-    const int nact = *tv.nactive;
+    const int nact = tv.nactive[parity];
+    const int *active = tv.active + (long)parity * tv.ntiles;
+    const int2 *titem = tv.titem + (long)parity * tv.ntiles;
     for (int sl = (int)bk.x; sl < nact; sl += (int)gd.x) {
-        const int t = tv.active[sl];
+        const int t = active[sl];
         int t0, t1, t2;
         tile_coords(tv, t, t0, t1, t2);
         __syncthreads();
@@ -335,7 +370,7 @@ __device__ __forceinline__ static void jgather32(const JPtrs &v, const Grid &g, 
                       uz = t2 - 1 + threadIdx.x % 3;
             const bool in = ux >= 0 && uy >= 0 && uz >= 0 && ux < tv.nt[0] && uy < tv.nt[1] &&
                             uz < tv.nt[2];
-            const int2 ti = in ? tv.titem[(ux * tv.nt[1] + uy) * tv.nt[2] + uz] : make_int2(0, 0);
+            const int2 ti = in ? titem[(ux * tv.nt[1] + uy) * tv.nt[2] + uz] : make_int2(0, 0);
             nfirst[threadIdx.x] = ti.x;
             nitem[threadIdx.x] = ti.y;
         }
@@ -406,7 +441,7 @@ template <> struct KernelDef<JGatherArgs> {
     static constexpr int kBlock = JG_TPB;
     __device__ __forceinline__ static void body(const JGatherArgs &a, VBlock b, VBlock gd)
     {
-        jgather32(a.v, a.g, a.tv, a.tj, b, gd);
+        jgather32(a.v, a.g, a.tv, a.tj, a.parity, b, gd);
     }
 };
 

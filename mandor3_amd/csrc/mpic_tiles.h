@@ -13,7 +13,6 @@
 #include "mpic_internal.h"
 
 #define TILE_CELLS 64
-#define MPIC_SCAN_BLOCK 256     /* tiles per workgroup of the tile scan */
 
 struct TileView {
     int  nt[3];              /* tiles per axis */
@@ -27,8 +26,10 @@ struct TileView {
     int *key;                /* [capacity] new key of every marker, -1 = deleted */
     int *perm;               /* [capacity] the current order as indices into the
                               * current buffer (nmark[parity] of them; tiled runs) */
-    int *active;             /* [ntiles] tiles holding markers, in tile order */
-    int *nactive;            /* [1] */
+    /* What the J gather reads of the order is kept for two orders, by parity:
+     * the scan then writes the next order's in the gather's launch. */
+    int *active;             /* [2][ntiles] tiles holding markers, in tile order */
+    int *nactive;            /* [2] */
     int *nmark;              /* [2] markers in the current / next order */
     int *xr;                 /* [2] x planes of nodes that the active tiles' gathers read
                               * (tiled runs: kept by the rank pass; else the whole grid) */
@@ -39,7 +40,8 @@ struct TileView {
     int4 *item;              /* [item capacity] work items in tile order: tile, first and last + 1
                               * position in the order (one load tells a workgroup its work: a
                               * chain of lookups costs a memory latency per link) */
-    int2 *titem;             /* [ntiles] first item and item count of every tile (count 0: empty) */
+    int2 *titem;             /* [2][ntiles] first item and item count of every tile (count 0:
+                              * empty), by parity like active */
     int *nitems;             /* [1] */
 };
 
@@ -118,12 +120,12 @@ int launch_counts_natural(hipStream_t s, const TileView &tv, const Grid &g, int3
 #define TJN 7
 #define TJB (TJN * TJN * TJN * 3)
 
-/* nblocks workgroups of 'waves' (1, 2 or 4) wavefronts each. */
+/* nblocks workgroups of 'waves' (1, 2, 4 or 8) wavefronts each. */
 int launch_push32(hipStream_t s, const Markers32 &m, const Markers32 &dst, const Fields32 &f,
                   const Grid &g, const PushConsts &pc, const float *qm, const TileView &tv,
                   float *tj, double *kin, int nblocks, int waves);
 int launch_jgather32(hipStream_t s, const JPtrs &j, const Grid &g, const TileView &tv,
-                     const float *tj, int nblocks);
+                     const float *tj, int parity, int nblocks);
 
 /* What the loop body's launches between the push and the E update work on. */
 struct AfterPush {

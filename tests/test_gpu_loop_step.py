@@ -20,13 +20,15 @@ WALLS = ["pp", "mm", "oo", "om", "mo"]
 CODE = {"p": ma.BC_PERIODIC, "m": ma.BC_MIRROR, "o": ma.BC_OPEN}
 
 
-def make(n, walls, prec, markers, seed):
+def make(n, walls, prec, markers, seed, x=(0.0, 1.0)):
     rng = np.random.default_rng(seed)
     bc = [CODE[w[0]] for w in walls] + [CODE[w[1]] for w in walls]
     N = 3 * int(np.prod(n)) if markers else 0
     M = np.zeros(N, dtype=ma.MARKER_DTYPE)
     for a, c in enumerate("xyz"):
         M[c] = rng.uniform(0, n[a] * H[a], N)
+        if a == 0:
+            M[c] = x[0] * n[0] * H[0] + (x[1] - x[0]) * M[c]
         M["v" + c] = rng.normal(0, 0.5, N)
     M["rho"], M["qDivM"], M["id"] = -0.5, -1.0, np.arange(1, N + 1)
     nodes = 3 * int(np.prod([v + 1 for v in n]))
@@ -110,6 +112,25 @@ def test_graphs_after_sorts_and_stage_steps(prec):
         staged(b)
     x, y = by_id(a.markers()), by_id(b.markers())
     assert np.array_equal(x["id"], y["id"])
+    for f in ("x", "y", "z"):
+        np.testing.assert_allclose(x[f], y[f], rtol=0, atol=1e-12 if prec == ma.FP64 else 1e-5)
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("prec", [ma.FP64, ma.FP32_SPLIT])
+@pytest.mark.parametrize("n", [(32, 32, 16), (33, 32, 16), (36, 33, 29)])
+def test_order_over_several_scan_workgroups(n, prec):
+    """One scan workgroup of 256 tiles exactly, 288 and 648 tiles (two and
+    three workgroups), a third of the tiles empty: every marker is in the order
+    the loop's scan (FP32: in the gather's launch, in rounds of few registers)
+    and rank leave exactly once, and the next push agrees with the stages'."""
+    a, b = make(n, ("oo", "pp", "mm"), prec, True, 3, (0.3, 0.8))
+    for _ in range(3):
+        a.step(diag=False)
+        staged(b)
+    x, y = by_id(a.markers()), by_id(b.markers())
+    assert np.array_equal(x["id"], np.unique(x["id"])) and np.array_equal(x["id"], y["id"])
     for f in ("x", "y", "z"):
         np.testing.assert_allclose(x[f], y[f], rtol=0, atol=1e-12 if prec == ma.FP64 else 1e-5)
     a.close()
