@@ -609,7 +609,7 @@ int launch_h_update(hipStream_t s, const FieldsT<T> &f, const Grid &g, const Box
  * Laser-foil (256 x 128 x 128), J clear included: 47 us FP32, 87 us FP64,
  * against 105 and 167 us for cap update, two wall launches and two H passes
  * (36 B moved per node in FP32 instead of 60, four dependent launches fewer);
- * HBM-bound, 165 MB at 4.0 TB/s in FP32.  32^3 box: 10 us against 29. */
+ * HBM-bound, 165 MB at 4.0 TB/s in FP32.  32^3 box: 6.7 us against 29. */
 template <class T> struct HFullArgs {
     FieldsT<T>    f;           /* H: H^{n-1/2}, Hc: H^{n+1/2}, Ec: H^n */
     Grid          g;
@@ -757,6 +757,12 @@ template <class T> struct HEdgeArgs {
     int          bc[6];
 };
 
+/* Component c of them, one component per workgroup: a third of the
+ * instructions of a thread that takes a node's three components, and in a
+ * launch this short their fetch is what takes the time (32^3 box: 8.9 us
+ * before, 6.7 now).  Workgroups go to the eight XCDs in turn, so those of
+ * the three components of 256 nodes are eight apart and share an L2. */
+#define EDGE_GROUP 24
 template <class T>
 __device__ static inline void h_edge(const HEdgeArgs<T> &B, const VBlock &b, double &we,
                                      double &wb)
@@ -764,54 +770,48 @@ __device__ static inline void h_edge(const HEdgeArgs<T> &B, const VBlock &b, dou
     const HFullArgs<T> &A = B.h;
     const Grid &g = A.g;
     const FieldsT<T> &f = A.f;
+    const int c = (int)(b.x % EDGE_GROUP) >> 3, u = c == 2 ? 0 : c + 1, w = c == 0 ? 2 : c - 1;   /* c + 1, c + 2 */
     int r[3];
-    if (!box_decode(B.bs, (long)b.x * TPB + threadIdx.x, r[0], r[1], r[2])) return;
+    const long blk = (long)(b.x / EDGE_GROUP) * 8 + (b.x & 7);
+    if (!box_decode(B.bs, blk * TPB + threadIdx.x, r[0], r[1], r[2])) return;
     const long o = gidx(g, r[0], r[1], r[2]);
-    const long st[3] = {(long)g.GY * g.GZ, g.GZ, 1};
-    T old[3], full[3];
-    bool zero[3], none[3];
-    long src[3];
+    const long si = (long)g.GY * g.GZ, sj = g.GZ;
+    const long su = u == 0 ? si : u == 1 ? sj : 1, sw = w == 0 ? si : w == 1 ? sj : 1;
+    int s[3];
+    bool zero = false, none = false, in_e = true, in_h = true;
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        int s[3];
-        zero[c] = none[c] = false;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const int N = g.n[a], lo = B.bc[a], hi = B.bc[3 + a];
-            int v = r[a];
-            if (v == 0) {
-                if (lo == MPIC_BC_PERIODIC) v = N;
-                else if (a != c) v = 1;
-                else zero[c] = zero[c] || lo == MPIC_BC_MIRROR;
-            } else if (v == N + 1) {
-                if (hi == MPIC_BC_PERIODIC) v = 1;
-                else if (a != c) v = N;
-                else none[c] = true;
-            } else if (v == N && a == c && hi == MPIC_BC_MIRROR) {
-                zero[c] = true;
-            }
-            s[a] = v;
+    for (int a = 0; a < 3; ++a) {
+        const int N = g.n[a], lo = B.bc[a], hi = B.bc[3 + a], v = r[a];
+        int src = v;
+        if (v == 0) {
+            if (lo == MPIC_BC_PERIODIC) src = N;
+            else if (a != c) src = 1;
+            else zero = zero || lo == MPIC_BC_MIRROR;
+        } else if (v == N + 1) {
+            if (hi == MPIC_BC_PERIODIC) src = 1;
+            else if (a != c) src = N;
+            else none = true;
+        } else if (v == N && a == c && hi == MPIC_BC_MIRROR) {
+            zero = true;
         }
-        src[c] = gidx(g, s[0], s[1], s[2]);
-        old[c] = f.H[c][o];
+        s[a] = src;
+        /* energy_terms' points: E_c shifted along its own axis, H_c along the others */
+        const bool z0 = v >= 0 && v < N, z1 = v >= 1 && v <= N;
+        in_e = in_e && (a == c ? z1 : z0);
+        in_h = in_h && (a == c ? z0 : z1);
     }
-    const T *E0 = f.E[0], *E1 = f.E[1], *E2 = f.E[2];
-    const long p = src[0], q = src[1], t = src[2];
-    full[0] = f.H[0][p] + A.d[2] * (E1[p] - E1[p - st[2]]) - A.d[1] * (E2[p] - E2[p - st[1]]);
-    full[1] = f.H[1][q] + A.d[0] * (E2[q] - E2[q - st[0]]) - A.d[2] * (E0[q] - E0[q - st[2]]);
-    full[2] = f.H[2][t] + A.d[1] * (E0[t] - E0[t - st[1]]) - A.d[0] * (E1[t] - E1[t - st[0]]);
-    const bool want = r[0] >= A.xr[0] && r[0] <= A.xr[1];
-    const T e[3] = {E0[o], E1[o], E2[o]};
-    T half[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        if (zero[c]) full[c] = 0;
-        half[c] = (T)0.5 * (old[c] + full[c]);
-        if (none[c]) continue;
-        f.Hc[c][o] = full[c];
-        if (want) f.Ec[c][o] = half[c];
+    const long p = gidx(g, s[0], s[1], s[2]);
+    const T *Eu = f.E[u], *Ew = f.E[w];
+    const T old = f.H[c][o], e = f.E[c][o];
+    T full = f.H[c][p] + A.d[w] * (Eu[p] - Eu[p - sw]) - A.d[u] * (Ew[p] - Ew[p - su]);
+    if (zero) full = 0;
+    const T half = (T)0.5 * (old + full);
+    if (!none) {
+        f.Hc[c][o] = full;
+        if (r[0] >= A.xr[0] && r[0] <= A.xr[1]) f.Ec[c][o] = half;
     }
-    energy_terms<T>(g, r[0], r[1], r[2], e[0], e[1], e[2], half[0], half[1], half[2], we, wb);
+    if (in_e) we = (double)e * (double)e;
+    if (in_h) wb = (double)half * (double)half;
 }
 
 template <class T> struct KernelDef<HFullArgs<T>> {
@@ -859,12 +859,17 @@ static BoxSet h_edge_set(const Grid &g)
     return s;
 }
 
+static unsigned h_edge_blocks(const BoxSet &s)
+{
+    return EDGE_GROUP * ((nblk(s.off[s.n]) + 7) / 8);
+}
+
 /* Workgroups of the one-pass H update: the energy partial sums it writes. */
 int h_full_blocks(const Grid &g, int fp32)
 {
     const BoxSet s = h_edge_set(g);
     return (int)(grid_span(h_full_span(g, fp32 ? Vec<float>::N : Vec<double>::N), g.n[0]) +
-                 nblk(s.off[s.n]));
+                 h_edge_blocks(s));
 }
 
 /* Interior E step (source/core/em.c:134-161) and/or the flush of the cap
@@ -1957,7 +1962,7 @@ int launch_h_full_jclear(hipStream_t s, const FieldsT<T> &f, const Grid &g, cons
     a.xr = xr;
     e.bs = h_edge_set(g);
     for (int q = 0; q < 6; ++q) e.bc[q] = bc[q];
-    const unsigned na = grid_span(a.sp, g.n[0]), ne = nblk(e.bs.off[e.bs.n]);
+    const unsigned na = grid_span(a.sp, g.n[0]), ne = h_edge_blocks(e.bs);
     HFullArgs<T> inner = a;
     inner.part = part;
     a.part = part + 2 * (long)na;

@@ -135,3 +135,18 @@ def test_order_over_several_scan_workgroups(n, prec):
         np.testing.assert_allclose(x[f], y[f], rtol=0, atol=1e-12 if prec == ma.FP64 else 1e-5)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("prec", [ma.FP64, ma.FP32_SPLIT])
+@pytest.mark.parametrize("walls", [("pp", "om", "mm"), ("mo", "pp", "oo")])
+def test_vacuum_over_several_groups_of_edge_workgroups(walls, prec):
+    """24 x 33 x 40: 27 workgroups of edge nodes, four groups of eight (the
+    components' workgroups lie eight apart) with the last one partly empty."""
+    a, b = make((24, 33, 40), walls, prec, False, 2)
+    for _ in range(2):
+        a.step(diag=False)
+        staged(b)
+    for x, y in zip(a.fields(), b.fields()):
+        assert np.array_equal(x, y)
+    a.close()
+    b.close()
