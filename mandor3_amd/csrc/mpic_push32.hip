@@ -52,7 +52,6 @@
 
 struct F32View {
     const float *E[3], *H[3];
-    double *J[3];
     Grid g;
 };
 
@@ -86,11 +85,16 @@ __device__ static inline void seg_values(float x1, float y1, float z1, float x2,
 /* Offset of node (+da,+db,+dc), component comp, from a node of the LDS J block. */
 #define LJO(da, db, dc, comp) (3 * (((da) * TJN + (db)) * TJN + (dc)) + (comp))
 
-/* Adds a segment of local cell (a,b,c) (LDS block coordinates) to LDS:
- * one address, the twelve nodes as constant offsets of it. */
-__device__ static inline void seg_to_lds(float *lj, int a, int b, int c, const Seg12 &s)
+/* The LDS block's cell (a, b, c): its first node's first component. */
+__device__ static inline int lj_cell(int a, int b, int c)
 {
-    float *p = lj + __mul24(__mul24(__mul24(a, TJN) + b, TJN) + c, 3);
+    return __mul24(__mul24(__mul24(a, TJN) + b, TJN) + c, 3);
+}
+
+/* Adds a segment of the block's cell at p: one address, the twelve nodes as
+ * constant offsets of it. */
+__device__ static inline void seg_to_lds(float *p, const Seg12 &s)
+{
     atomicAdd(p + LJO(1, 0, 0, 0), s.v[0]);
     atomicAdd(p + LJO(1, 1, 0, 0), s.v[1]);
     atomicAdd(p + LJO(1, 0, 1, 0), s.v[2]);
@@ -103,34 +107,6 @@ __device__ static inline void seg_to_lds(float *lj, int a, int b, int c, const S
     atomicAdd(p + LJO(1, 0, 1, 2), s.v[9]);
     atomicAdd(p + LJO(0, 1, 1, 2), s.v[10]);
     atomicAdd(p + LJO(1, 1, 1, 2), s.v[11]);
-}
-
-/* Same, straight to the FP64 J in HBM (segment outside the LDS block). */
-__device__ static inline void seg_to_hbm(const F32View &v, int i, int j, int k, const Seg12 &s)
-{
-    const Grid &g = v.g;
-    unsafeAtomicAdd(v.J[0] + gidx(g, i + 1, j, k), (double)s.v[0]);
-    unsafeAtomicAdd(v.J[0] + gidx(g, i + 1, j + 1, k), (double)s.v[1]);
-    unsafeAtomicAdd(v.J[0] + gidx(g, i + 1, j, k + 1), (double)s.v[2]);
-    unsafeAtomicAdd(v.J[0] + gidx(g, i + 1, j + 1, k + 1), (double)s.v[3]);
-    unsafeAtomicAdd(v.J[1] + gidx(g, i, j + 1, k), (double)s.v[4]);
-    unsafeAtomicAdd(v.J[1] + gidx(g, i + 1, j + 1, k), (double)s.v[5]);
-    unsafeAtomicAdd(v.J[1] + gidx(g, i, j + 1, k + 1), (double)s.v[6]);
-    unsafeAtomicAdd(v.J[1] + gidx(g, i + 1, j + 1, k + 1), (double)s.v[7]);
-    unsafeAtomicAdd(v.J[2] + gidx(g, i, j, k + 1), (double)s.v[8]);
-    unsafeAtomicAdd(v.J[2] + gidx(g, i + 1, j, k + 1), (double)s.v[9]);
-    unsafeAtomicAdd(v.J[2] + gidx(g, i, j + 1, k + 1), (double)s.v[10]);
-    unsafeAtomicAdd(v.J[2] + gidx(g, i + 1, j + 1, k + 1), (double)s.v[11]);
-}
-
-__device__ static inline void seg_add(const F32View &v, float *lj, int o0, int o1, int o2, int i,
-                                      int j, int k, const Seg12 &s)
-{
-    const int a = i - o0, b = j - o1, c = k - o2;
-    if (a < 0 || b < 0 || c < 0 || a > TJN - 2 || b > TJN - 2 || c > TJN - 2)
-        seg_to_hbm(v, i, j, k, s);
-    else
-        seg_to_lds(lj, a, b, c, s);
 }
 
 struct Push32Consts {
@@ -271,21 +247,24 @@ struct TilePos {
     bool edge;
 };
 
+__device__ static inline int clamp1(float f)
+{
+    return (int)__builtin_amdgcn_fmed3f(f, -1.0f, 1.0f);
+}
+
 /* Push of one marker of tile-local cell (li,lj,lk) (cell (ci,cj,ck)):
  * gather from the staged fields, Boris, move, deposit of every segment but
- * the first into the tile's LDS J (or HBM beyond it), walls.  Returns the
+ * the first into the tile's LDS J, walls.  Returns the
  * new cell word (-1: deleted), the new offsets and momenta in 'out' and the
  * first segment, which lies inside the start cell. */
 __device__ static inline int push32_marker(MarkerRegs &out, const MarkerRegs &r, int li,
                                            int lj_, int lk, int ci, int cj, int ck,
-                                           const float *lf, const float *lqm, float *lj, int o0,
-                                           int o1, int o2,
-                                           const F32View &v, const Push32Consts &c,
+                                           const float *lf, const float *lqm, float *lj,
+                                           const Grid &g, const Push32Consts &c,
                                            const TileView &tv, const TilePos &tp,
                                            Seg12 &first, float &w0,
                                            float &w1, float &w2)
 {
-    const Grid &g = v.g;
     const int sp = (int)((unsigned)r.word >> SPECIES_SHIFT);
     const float ox = r.ox, oy = r.oy, oz = r.oz;
     float ux = r.ux, uy = r.uy, uz = r.uz;
@@ -326,7 +305,12 @@ __device__ static inline int push32_marker(MarkerRegs &out, const MarkerRegs &r,
     const float ig = rsq(1.0f + ux * ux + uy * uy + uz * uz);
     /* move in cell units from (ox,oy,oz) of cell (ci,cj,ck) */
     const float x2 = ox + ux * c.dtn[0] * ig, y2 = oy + uy * c.dtn[1] * ig, z2 = oz + uz * c.dtn[2] * ig;
-    const int fx = (int)floorf(x2), fy = (int)floorf(y2), fz = (int)floorf(z2);
+    const float flx = floorf(x2), fly = floorf(y2), flz = floorf(z2);
+    /* -1, 0 or 1: a marker moves less than a cell per step, mpic_create's
+     * Courant condition.  The clamp only keeps one that is not a number inside
+     * the block, so a segment needs no range check: a tile's markers start in
+     * block cells 1 to 4 and cross at most one face per axis. */
+    const int fx = clamp1(flx), fy = clamp1(fly), fz = clamp1(flz);
     const float wx = w * c.cj[0], wy = w * c.cj[1], wz = w * c.cj[2];
     /* Segments: from the start to the first face crossing (or the end),
      * then one per crossed face.  Crossing fractions ascend; an axis that is
@@ -348,12 +332,18 @@ __device__ static inline int push32_marker(MarkerRegs &out, const MarkerRegs &r,
     }
     seg_values(ox, oy, oz, qx, qy, qz, wx, wy, wz, first);
     if (nc) {
-        int sx = 0, sy = 0, sz = 0, axs = x0;
+        /* the cell's address and the shift of its frame, moved by the
+         * crossed axis' stride and direction */
+        float *p = lj + lj_cell(li + 1, lj_ + 1, lk + 1);
+        float sx = 0, sy = 0, sz = 0;
+        int axs = x0;
 #pragma unroll 1
         for (int s = 1; s <= nc; ++s) {
-            sx += (axs == 0) ? fx : 0;
-            sy += (axs == 1) ? fy : 0;
-            sz += (axs == 2) ? fz : 0;
+            const bool cx = axs == 0, cy = axs == 1, cz = axs == 2;
+            p += cx ? fx * LJO(1, 0, 0, 0) : cy ? fy * LJO(0, 1, 0, 0) : fz * LJO(0, 0, 1, 0);
+            sx += cx ? flx : 0.0f;
+            sy += cy ? fly : 0.0f;
+            sz += cz ? flz : 0.0f;
             a0 = a1;
             x0 = x1;
             a1 = a2;
@@ -362,7 +352,7 @@ __device__ static inline int push32_marker(MarkerRegs &out, const MarkerRegs &r,
             if (s < nc) crossing_point(ox, oy, oz, x2, y2, z2, fx, fy, fz, a0, x0, ex, ey, ez);
             Seg12 sg;
             seg_values(qx - sx, qy - sy, qz - sz, ex - sx, ey - sy, ez - sz, wx, wy, wz, sg);
-            seg_add(v, lj, o0, o1, o2, ci + sx, cj + sy, ck + sz, sg);
+            seg_to_lds(p, sg);
             qx = ex;
             qy = ey;
             qz = ez;
@@ -371,7 +361,7 @@ __device__ static inline int push32_marker(MarkerRegs &out, const MarkerRegs &r,
     }
     /* new cell and offset, then the walls */
     int ni = ci + fx, nj = cj + fy, nk = ck + fz;
-    float nx = x2 - (float)fx, ny = y2 - (float)fy, nz = z2 - (float)fz;
+    float nx = x2 - flx, ny = y2 - fly, nz = z2 - flz;
     if (nx >= 1.0f) { nx = 0.0f; ++ni; }
     if (ny >= 1.0f) { ny = 0.0f; ++nj; }
     if (nz >= 1.0f) { nz = 0.0f; ++nk; }
@@ -488,9 +478,13 @@ __device__ static inline void write_back(const Markers32 &d, const TileView &tv,
  * mpic_create) share the staging and the block, shorten a tile's serial chain
  * of batches and let the hardware balance tiles of very different occupancy;
  * each wavefront loads its next batch before pushing the current.  Laser-foil
- * push (8.57 M markers) 202 us with one wavefront per tile, 165 us with
- * four; it is bound by VALU issue (about 530 instructions per batch of 64
- * at 4 cycles each, 65 % of the time on a full box). */
+ * push (8.57 M markers) 202 us with one wavefront per tile, 162 us with
+ * four: 4.2 TB/s of its 80 B per marker, against 4.8 TB/s of a copy.  A full
+ * box (64^3, 121 us) is bound by VALU issue, about 530 instructions per batch
+ * of 64 at 4 cycles each; without the range check of every segment and its
+ * path to HBM for cells a marker cannot reach, and with the run heads found by
+ * DPP instead of a shuffle, 124 -> 121 us there, 33.5 -> 32.6 on a
+ * 128x64x64 foil (FP64, by the run heads alone, 60 -> 58.6). */
 struct Push32Args {
     Markers32    m, d;         /* current buffer (read through tv.perm), output buffer */
     F32View      v;
@@ -529,7 +523,6 @@ __device__ __forceinline__ static void push32_tiles(const Markers32 &m, const Ma
         int t0, t1, t2;
         tile_coords(tv, t, t0, t1, t2);
         const int c0 = TILE * t0, c1 = TILE * t1, c2 = TILE * t2;
-        const int o0 = c0 - 1, o1 = c1 - 1, o2 = c2 - 1;
         TilePos tp;
         tp.t = t;
         tp.s0 = tv.nt[1] * tv.nt[2];
@@ -583,7 +576,7 @@ __device__ __forceinline__ static void push32_tiles(const Markers32 &m, const Ma
             load_marker(m, snx, nxt);
             snx = perm_at(tv.perm, p + 2 * BS, end - 1);
             write_back(d, tv, pend);
-            int rkey = -1, newword = -1, ci = 0, cj = 0, ck = 0;
+            int rkey = -1, newword = -1, cell = 0;
             Seg12 first;
             for (int q = 0; q < 12; ++q) first.v[q] = 0.0f;
             const bool in = p < end && cur.word >= 0;
@@ -591,11 +584,9 @@ __device__ __forceinline__ static void push32_tiles(const Markers32 &m, const Ma
                 rkey = cur.word & KEY_MASK;
                 const int loc = rkey & (TILE_CELLS - 1);
                 const int li = loc >> 4, lj_ = (loc >> 2) & 3, lk = loc & 3;
-                ci = c0 + li;
-                cj = c1 + lj_;
-                ck = c2 + lk;
-                newword = push32_marker(pend.r, cur, li, lj_, lk, ci, cj, ck, lf, lqm, lj, o0, o1, o2,
-                                        v, c, tv, tp, first, w0, w1, w2);
+                newword = push32_marker(pend.r, cur, li, lj_, lk, c0 + li, c1 + lj_, c2 + lk, lf, lqm,
+                                        lj, g, c, tv, tp, first, w0, w1, w2);
+                cell = lj_cell(li + 1, lj_ + 1, lk + 1);
             }
             pend.r.id = cur.id;
             pend.valid = in;
@@ -608,7 +599,7 @@ __device__ __forceinline__ static void push32_tiles(const Markers32 &m, const Ma
             /* last lane of the run inside its row: adds the row's part */
             const int ln = threadIdx.x & 63;
             const bool tail = ln == start + len - 1 || ((ln & 15) == 15 && ln < start + len - 1);
-            if (tail && rkey >= 0) seg_add(v, lj, o0, o1, o2, ci, cj, ck, first);
+            if (tail && rkey >= 0) seg_to_lds(lj + cell, first);
             /* count[new key] += run length, once per run of equal new keys */
             const int nkey = newword < 0 ? -1 : (newword & KEY_MASK);
             wave_run(nkey, start, len, head);
@@ -659,7 +650,6 @@ int launch_push32(hipStream_t s, const Markers32 &m, const Markers32 &dst, const
     for (int a = 0; a < 3; ++a) {
         v.E[a] = f.E[a];
         v.H[a] = f.H[a];
-        v.J[a] = f.J[a];
     }
     v.g = g;
     Push32Consts c;

@@ -82,7 +82,8 @@ __device__ static inline int cell_key_of(const TileView &tv, const Grid &g, cons
 __device__ static inline void wave_run(int key, int &start, int &len, bool &head)
 {
     const int lane = threadIdx.x & 63;
-    const int prev = __shfl_up(key, 1, 64);
+    /* DPP wave_shr:1, a VALU move (a shuffle is a trip through the LDS unit) */
+    const int prev = __builtin_amdgcn_update_dpp(key, key, 0x138, 0xf, 0xf, false);
     head = (lane == 0) || (key != prev);
     const unsigned long long hm = __ballot(head);
     const unsigned long long le = (lane == 63) ? ~0ull : ((1ull << (lane + 1)) - 1ull);
