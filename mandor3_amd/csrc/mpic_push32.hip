@@ -510,8 +510,10 @@ __device__ __forceinline__ static void push32_tiles(const Markers32 &m, const Ma
     const int lane = threadIdx.x & 63;
     const int nitems = *tv.nitems;
     float w0 = 0, w1 = 0, w2 = 0;         /* per-thread kinetic energy partials */
+    int4 work = tv.item[bk.x];            /* not behind the load of nitems: the grid is at
+                                           * most the item capacity */
     for (int it = (int)bk.x; it < nitems; it += (int)gd.x) {
-        const int4 work = tv.item[it];
+        if (it != (int)bk.x) work = tv.item[it];
         const int t = work.x;
         const unsigned beg = work.y, end = work.z;
         /* the order's indices are loaded two batches ahead and the records

@@ -767,8 +767,10 @@ __device__ __forceinline__ static void push64_tiles(const Push64TArgs &A, const 
     const Grid &g = v.g;
     const int nitems = *tv.nitems;
     double w3[3] = {0, 0, 0};
+    int4 work = tv.item[bk.x];            /* not behind the load of nitems: the grid is at
+                                           * most the item capacity */
     for (int it = (int)bk.x; it < nitems; it += (int)gd.x) {
-        const int4 work = tv.item[it];
+        if (it != (int)bk.x) work = tv.item[it];
         const unsigned beg = work.y, end = work.z;
         const unsigned s0 = perm_at(tv.perm, beg + threadIdx.x, end - 1);
         unsigned snx = perm_at(tv.perm, beg + BS + threadIdx.x, end - 1);

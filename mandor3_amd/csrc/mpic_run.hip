@@ -403,7 +403,7 @@ extern "C" int mpic_footprint(const mpic_config_t *cfg, size_t *bytes)
     const long cap = cfg->max_markers > 0 ? cfg->max_markers : 1;
     const size_t items = (size_t)items_capacity((int)tiles, cap, fp32 ? push32_item_markers() : 0);
     *bytes = field_bytes(cfg->n, fp32) + 2 * sizeof(double) * cells +
-             2 * (size_t)cap * mk + tiles * 64 * 3 * sizeof(int) + tiles * 6 * sizeof(int) +
+             2 * (size_t)cap * mk + tiles * 64 * 3 * sizeof(int) + tiles * 9 * sizeof(int) +
              items * sizeof(int4) + (fp32 ? items * TJB * sizeof(float) : 0);
     return MPIC_OK;
 }
@@ -1857,13 +1857,15 @@ static int record(mpic_run *r, int k)
 /* The push and its deposit, reading H from f / f32. */
 static int push(mpic_run *r, const Fields32 &f32, const Fields64 &f)
 {
+    /* (a request for more workgroups than items have room leaves the rest idle) */
+    const int nb = r->tile_blocks < r->items_cap ? r->tile_blocks : (int)r->items_cap;
     if (r->timed >= 0) TRY(record(r, 1));
     if (r->fp32)
         TRY(launch_push32(r->stream, r->m32, r->m32buf[r->cur ^ 1], f32, r->g, r->pc, r->qm, r->tv,
-                          r->tj, r->dkin, r->tile_blocks, r->tile_waves));
+                          r->tj, r->dkin, nb, r->tile_waves));
     else if (r->tiled)
         TRY(launch_push64_tiled(r->stream, r->m, r->mbuf[r->cur ^ 1], f, r->g, r->pc, r->tv,
-                                r->dkin, r->derr, r->tile_blocks, r->tile_waves));
+                                r->dkin, r->derr, nb, r->tile_waves));
     else
         TRY(launch_push64(r->stream, r->m, r->n, f, r->g, r->pc, r->dkin, 0, r->derr));
     if (r->timed >= 0) TRY(record(r, 2));

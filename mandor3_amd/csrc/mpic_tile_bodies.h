@@ -88,6 +88,7 @@ __device__ static inline void scan_pass(const ScanArgs &A, const VBlock &bk)
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, blk = (int)bk.x;
     const int wt0 = blk * SB + w * SCAN_WT;          /* first tile of the wavefront */
     const int4 *cnt4 = (const int4 *)tv.count;
+    const int seq = *A.seq;                          /* with the counts' latency, not after it */
     int c = 0;                                       /* markers of tile wt0 + lane */
     int4 x[LD];
 #pragma unroll 1
@@ -121,7 +122,6 @@ __device__ static inline void scan_pass(const ScanArgs &A, const VBlock &bk)
     }
     if (w == 0) {                                    /* the look-back, one wavefront */
         unsigned long long *F = A.flags;
-        const int seq = *A.seq;
         const unsigned tag = (unsigned)(seq % 0x7fffffff) + 1u;
         int pre[NSCAN] = {0, 0, 0};
         if (blk > 0) {
@@ -284,12 +284,13 @@ __device__ static inline void rank_pass(const TileView &tv, long nbound, int par
 #pragma unroll
     for (int u = 0; u < RANK_BATCHES; ++u) {
         const long p = b0 + 256 * u + threadIdx.x;
-        key[u] = (p < n && p < nbound) ? tv.key[p] : -1;
+        key[u] = p < nbound ? tv.key[p] : -1;    /* not behind the load of n */
     }
 #pragma unroll
     for (int u = 0; u < RANK_BATCHES; ++u) {
         int len;
         bool head;
+        if (b0 + 256 * u + threadIdx.x >= n) key[u] = -1;
         wave_run(key[u], start[u], len, head);
         base[u] = 0;
         if (head && key[u] >= 0) base[u] = atomicAdd(tv.cursor + key[u], len);
@@ -360,8 +361,11 @@ __device__ __forceinline__ static void jgather32(const JPtrs &v, const Grid &g, 
     const int nact = tv.nactive[parity];
     const int *active = tv.active + (long)parity * tv.ntiles;
     const int2 *titem = tv.titem + (long)parity * tv.ntiles;
+    /* the first tile's load does not wait for the number of tiles: entries
+     * past it are stale, and not used */
+    const int first = active[(int)bk.x < tv.ntiles ? (int)bk.x : tv.ntiles - 1];
     for (int sl = (int)bk.x; sl < nact; sl += (int)gd.x) {
-        const int t = active[sl];
+        const int t = sl == (int)bk.x ? first : active[sl];
         int t0, t1, t2;
         tile_coords(tv, t, t0, t1, t2);
         __syncthreads();
