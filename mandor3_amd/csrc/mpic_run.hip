@@ -2420,6 +2420,25 @@ static void fuse(const std::vector<Recorder> &recs, std::vector<std::vector<cons
     }
 }
 
+/* Workgroups of a run's push and J gather in a fused launch.  A run's own
+ * (up to 16 per CU each) are more than its tiles with markers; the idle ones
+ * cost a run alone about 1 us, but a dozen runs' 40000 cost the FP32 push of
+ * twelve scan runs 30 us of 276 and their gather 28 of 85.  So a fused launch
+ * has as many per CU over all runs, shared out by markers (push) and tiles
+ * (gather).  Step in us with each run's own and with 16 / 24 / 32 push
+ * workgroups per CU: twelve FP32 runs 503, 440 / 442 / 443, five 420, 385 /
+ * 394 / 404, three 167, 157 / 162 / 162; five FP64 runs 685, 656 / 659 / 662,
+ * three 229, 233 / 233 / 230 (a run's workgroups just short of its items
+ * leave a second round nearly empty, which the slower FP64 push feels). */
+#define ENS_PUSH32 16
+#define ENS_PUSH64 32
+#define ENS_GATHER 24
+static int ensemble_share(int blocks, int ncu, double n, double total)
+{
+    const double s = total > 0 ? (double)blocks * ncu * n / total : 0;
+    return (int)s < ncu / 2 ? ncu / 2 : (int)s;
+}
+
 static int ensemble_build(mpic_run *const *runs, int nruns, Ensemble **out)
 {
     Ensemble *e = new Ensemble();
@@ -2436,10 +2455,22 @@ static int ensemble_build(mpic_run *const *runs, int nruns, Ensemble **out)
     /* Launches fuse by kind, and the push's kind carries its wavefronts per
      * workgroup: where small boxes (8 by their own rule) meet larger ones
      * (4), all take 4, in one launch. */
-    std::vector<int> own_waves(nruns);
+    std::vector<int> own_waves(nruns), own_push(nruns), own_gather(nruns);
     bool mixed = false;
+    double markers = 0, tiles = 0;
+    for (int q = 0; q < nruns; ++q) {
+        markers += (double)runs[q]->n;
+        tiles += runs[q]->tv.ntiles;
+    }
     for (int q = 0; q < nruns; ++q) {
         own_waves[q] = runs[q]->tile_waves;
+        own_push[q] = runs[q]->tile_blocks;
+        own_gather[q] = runs[q]->gather_blocks;
+        const int np = ensemble_share(runs[q]->fp32 ? ENS_PUSH32 : ENS_PUSH64, runs[q]->ncu,
+                                      (double)runs[q]->n, markers),
+                  ng = ensemble_share(ENS_GATHER, runs[q]->ncu, runs[q]->tv.ntiles, tiles);
+        if (np < own_push[q]) runs[q]->tile_blocks = np;
+        if (ng < own_gather[q]) runs[q]->gather_blocks = ng;
         mixed = mixed || own_waves[q] != runs[0]->tile_waves;
     }
     for (int q = 0; q < nruns && mixed; ++q)
@@ -2450,7 +2481,11 @@ static int ensemble_build(mpic_run *const *runs, int nruns, Ensemble **out)
         recs[0][q] = std::move(two[0]);
         recs[1][q] = std::move(two[1]);
     }
-    for (int q = 0; q < nruns; ++q) runs[q]->tile_waves = own_waves[q];
+    for (int q = 0; q < nruns; ++q) {
+        runs[q]->tile_waves = own_waves[q];
+        runs[q]->tile_blocks = own_push[q];
+        runs[q]->gather_blocks = own_gather[q];
+    }
     std::vector<std::vector<const LaunchRec *>> seq[2];
     std::vector<FusedLaunch> fl[2];
     size_t bytes = 0;

@@ -8,6 +8,7 @@ import pytest
 import mandor3_amd as ma
 from mandor3_amd import workloads
 from test_gpu_modes import _split_twenty_steps
+from test_gpu_parity import rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -76,3 +77,33 @@ def test_field_energy_sums(n, prec):
     # partial sums, all positive: (6 + 8 + 2048) 2^-53 < 3e-13
     np.testing.assert_allclose(r.energy(), want, rtol=3e-13)
     r.close()
+
+
+@pytest.mark.parametrize("prec,tol", [(ma.FP64, 1e-12), (ma.FP32_SPLIT, 2e-5)])
+def test_fused_runs_with_fewer_workgroups_than_tiles(prec, tol):
+    """Fused launches share workgroups out by markers: the 32^3 box with a
+    sixteenth of the markers beside the full one gets fewer than its 512 tiles
+    (241 FP32 in two runs, 128 FP64 in six, on 256 CUs): a workgroup takes
+    several; the results are those of the run alone, to the order of the J sums (the serving
+    loop's bar)."""
+    st = workloads.two_stream_box(32)
+
+    def make(M):
+        r = ma.Run(st["n"], st["h"], st["L"], st["tau"], st["bc"], 0.0, precision=prec,
+                   max_markers=M.size)
+        z = np.zeros(3 * r.nodes)
+        r.set_fields(z, z)
+        r.load_markers(M)
+        r.init()
+        return r
+
+    thin, full = st["markers"][::16], st["markers"]
+    alone = make(thin)
+    runs = [make(thin)] + [make(full) for _ in range(5 if prec == ma.FP64 else 1)]
+    alone.advance(6)
+    ma.batch_advance(runs, 6)
+    for a, b in zip(alone.fields(), runs[0].fields()):
+        assert np.linalg.norm(a) > 0 and rel_l2(b, a) <= tol
+    assert alone.marker_count() == runs[0].marker_count() == thin.size
+    for r in [alone] + runs:
+        r.close()
