@@ -697,25 +697,25 @@ int launch_keys32(hipStream_t s, const Markers32 &m, long n, const TileView &tv,
 }
 
 /* CIC charge density of the split-precision markers of the order, FP64. */
-__global__ void k_rho32(Markers32 m, long n, double *rho, Grid g, TileView tv, int parity)
+__global__ void __launch_bounds__(TPB) k_rho32(Markers32 m, long n, double *rho, Grid g,
+                                               TileView tv, int parity)
 {
     const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n || (tv.perm && q >= tv.nmark[parity])) return;
-    const long p = tv.perm ? tv.perm[q] : q;            /* no permutation: the loaded order */
-    const float4 a = m.pos[p];
-    const int word = __float_as_int(a.x);
-    if (word < 0) return;
-    int i, j, k;
-    key_to_ijk(tv, word & KEY_MASK, i, j, k);
-    const double sx = a.y, sy = a.z, sz = a.w, val = m.mom[p].w;
-    unsafeAtomicAdd(rho + gidx(g, i, j, k), (1 - sx) * ((1 - sy) * ((1 - sz) * val)));
-    unsafeAtomicAdd(rho + gidx(g, i + 1, j, k), sx * ((1 - sy) * ((1 - sz) * val)));
-    unsafeAtomicAdd(rho + gidx(g, i, j + 1, k), (1 - sx) * (sy * ((1 - sz) * val)));
-    unsafeAtomicAdd(rho + gidx(g, i + 1, j + 1, k), sx * (sy * ((1 - sz) * val)));
-    unsafeAtomicAdd(rho + gidx(g, i, j, k + 1), (1 - sx) * ((1 - sy) * (sz * val)));
-    unsafeAtomicAdd(rho + gidx(g, i + 1, j, k + 1), sx * ((1 - sy) * (sz * val)));
-    unsafeAtomicAdd(rho + gidx(g, i, j + 1, k + 1), (1 - sx) * (sy * (sz * val)));
-    unsafeAtomicAdd(rho + gidx(g, i + 1, j + 1, k + 1), sx * (sy * (sz * val)));
+    /* no permutation: the loaded order */
+    const long p = q < n && (!tv.perm || q < tv.nmark[parity]) ? (tv.perm ? tv.perm[q] : q) : -1;
+    double v[8] = {};
+    long cell = -1;
+    if (p >= 0) {
+        const float4 a = m.pos[p];
+        const int word = __float_as_int(a.x);
+        if (word >= 0) {
+            int i, j, k;
+            key_to_ijk(tv, word & KEY_MASK, i, j, k);
+            cell = gidx(g, i, j, k);
+            cic_weights(a.y, a.z, a.w, m.mom[p].w, v);
+        }
+    }
+    rho_run_add(rho, g, cell, v);
 }
 
 int launch_rho32(hipStream_t s, const Markers32 &m, long n, double *rho, const Grid &g,

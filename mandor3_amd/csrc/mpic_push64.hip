@@ -653,16 +653,6 @@ __device__ static inline int push64_marker(Marker64 &k, const F64View &v, const 
     return cell_key_of(tv, g, k.r);
 }
 
-/* Row shift of a double by D lanes inside rows of 16 (DPP row_shr on
- * both halves; 0 from outside the row).  Every lane must be active. */
-template <int D> __device__ static inline double row_shr(double x)
-{
-    const long long b = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x110 + D, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x110 + D, 0xf, 0xf, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
 /* The first segments of a batch (one marker per lane, lanes in cell
  * order): summed over each run of lanes in one cell within each row of 16
  * lanes, then added to LDS by the run's last lane in the row (at most 4
@@ -675,22 +665,8 @@ __device__ static inline void first_run_add(double *lj, First64 &fs)
     int start, len;
     bool head;
     wave_run(fs.cell, start, len, head);
-    const int lane = threadIdx.x & 63;
-    /* fma(y, 1, x) is x + y rounded once, fma(y, 0, x) is x: one
-     * instruction instead of a select of y and an add */
-    const double m1 = lane - 1 >= start ? 1.0 : 0.0, m2 = lane - 2 >= start ? 1.0 : 0.0,
-                 m4 = lane - 4 >= start ? 1.0 : 0.0, m8 = lane - 8 >= start ? 1.0 : 0.0;
-#pragma unroll
-    for (int q = 0; q < 12; ++q) {
-        double x = fs.v[q];
-        x = __builtin_fma(row_shr<1>(x), m1, x);
-        x = __builtin_fma(row_shr<2>(x), m2, x);
-        x = __builtin_fma(row_shr<4>(x), m4, x);
-        x = __builtin_fma(row_shr<8>(x), m8, x);
-        fs.v[q] = x;
-    }
-    const bool tail = lane == start + len - 1 || ((lane & 15) == 15 && lane < start + len - 1);
-    if (tail && fs.cell >= 0) seg_add(lj, fs.cell >> 8, fs.cell >> 4 & 15, fs.cell & 15, fs.v);
+    run_sums<12>(fs.v, start);
+    if (run_tail(start, len) && fs.cell >= 0) seg_add(lj, fs.cell >> 8, fs.cell >> 4 & 15, fs.cell & 15, fs.v);
 }
 
 /* Tiled push: a workgroup of W wavefronts takes work items (a tile's markers
@@ -922,27 +898,23 @@ int launch_push64_tiled(hipStream_t s, const Markers64 &m, const Markers64 &dst,
 /* CIC charge density of the live markers, source/core/plasma_rho.c:160-173:
  * the order's markers through its permutation (perm non-null: the first
  * nmark[parity] entries), else the first n records. */
-__global__ void k_rho64(Markers64 m, long n, double *rho, Grid g, const int *perm,
-                        const int *nmark, int parity)
+__global__ void __launch_bounds__(TPB) k_rho64(Markers64 m, long n, double *rho, Grid g,
+                                               const int *perm, const int *nmark, int parity)
 {
     const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n || (perm && q >= nmark[parity])) return;
-    const long p = perm ? perm[q] : q;
-    if (m.qm[p] == 0.0f) return;
-    int i, j, k;
-    double sx, sy, sz;
-    sx = m.x[p] / g.h[0]; i = DBL_TO_INT(sx); sx -= i;
-    sy = m.y[p] / g.h[1]; j = DBL_TO_INT(sy); sy -= j;
-    sz = m.z[p] / g.h[2]; k = DBL_TO_INT(sz); sz -= k;
-    const double val = m.w[p];
-    unsafeAtomicAdd(rho + gidx(g, i, j, k), (1 - sx) * ((1 - sy) * ((1 - sz) * val)));
-    unsafeAtomicAdd(rho + gidx(g, i + 1, j, k), sx * ((1 - sy) * ((1 - sz) * val)));
-    unsafeAtomicAdd(rho + gidx(g, i, j + 1, k), (1 - sx) * (sy * ((1 - sz) * val)));
-    unsafeAtomicAdd(rho + gidx(g, i + 1, j + 1, k), sx * (sy * ((1 - sz) * val)));
-    unsafeAtomicAdd(rho + gidx(g, i, j, k + 1), (1 - sx) * ((1 - sy) * (sz * val)));
-    unsafeAtomicAdd(rho + gidx(g, i + 1, j, k + 1), sx * ((1 - sy) * (sz * val)));
-    unsafeAtomicAdd(rho + gidx(g, i, j + 1, k + 1), (1 - sx) * (sy * (sz * val)));
-    unsafeAtomicAdd(rho + gidx(g, i + 1, j + 1, k + 1), sx * (sy * (sz * val)));
+    const long p = q < n && (!perm || q < nmark[parity]) ? (perm ? perm[q] : q) : -1;
+    double v[8] = {};
+    long cell = -1;
+    if (p >= 0 && m.qm[p] != 0.0f) {
+        int i, j, k;
+        double sx, sy, sz;
+        sx = m.x[p] / g.h[0]; i = DBL_TO_INT(sx); sx -= i;
+        sy = m.y[p] / g.h[1]; j = DBL_TO_INT(sy); sy -= j;
+        sz = m.z[p] / g.h[2]; k = DBL_TO_INT(sz); sz -= k;
+        cell = gidx(g, i, j, k);
+        cic_weights(sx, sy, sz, m.w[p], v);
+    }
+    rho_run_add(rho, g, cell, v);
 }
 
 int launch_rho64(hipStream_t s, const Markers64 &m, long n, double *rho, const Grid &g,

@@ -102,6 +102,74 @@ __device__ static inline void wave_run_count(int *count, int key)
     if (head && key >= 0) atomicAdd(count + key, len);
 }
 
+/* Row shift of a double by D lanes inside rows of 16 (DPP row_shr on
+ * both halves; 0 from outside the row).  Every lane must be active. */
+template <int D> __device__ static inline double row_shr(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x110 + D, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x110 + D, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+/* Sums of N values over the lanes' runs (first lane 'start') within each row
+ * of 16 lanes: the last lane of a run in a row (run_tail) ends up with that
+ * row's part.  fma(y, 1, x) is x + y rounded once, fma(y, 0, x) is x: one
+ * instruction instead of a select of y and an add.  All lanes must call. */
+template <int N> __device__ static inline void run_sums(double *v, int start)
+{
+    const int lane = threadIdx.x & 63;
+    const double m1 = lane - 1 >= start ? 1.0 : 0.0, m2 = lane - 2 >= start ? 1.0 : 0.0,
+                 m4 = lane - 4 >= start ? 1.0 : 0.0, m8 = lane - 8 >= start ? 1.0 : 0.0;
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        double x = v[q];
+        x = __builtin_fma(row_shr<1>(x), m1, x);
+        x = __builtin_fma(row_shr<2>(x), m2, x);
+        x = __builtin_fma(row_shr<4>(x), m4, x);
+        x = __builtin_fma(row_shr<8>(x), m8, x);
+        v[q] = x;
+    }
+}
+
+__device__ static inline bool run_tail(int start, int len)
+{
+    const int lane = threadIdx.x & 63, last = start + len - 1;
+    return lane == last || ((lane & 15) == 15 && lane < last);
+}
+
+/* A marker's charge at its cell's eight nodes, source/core/plasma_rho.c:160-173;
+ * node (a, b, c) of the cell is v[4 a + 2 b + c]. */
+__device__ static inline void cic_weights(double sx, double sy, double sz, double val, double *v)
+{
+    v[0] = (1 - sx) * ((1 - sy) * ((1 - sz) * val));
+    v[4] = sx * ((1 - sy) * ((1 - sz) * val));
+    v[2] = (1 - sx) * (sy * ((1 - sz) * val));
+    v[6] = sx * (sy * ((1 - sz) * val));
+    v[1] = (1 - sx) * ((1 - sy) * (sz * val));
+    v[5] = sx * ((1 - sy) * (sz * val));
+    v[3] = (1 - sx) * (sy * (sz * val));
+    v[7] = sx * (sy * (sz * val));
+}
+
+/* rho += the lanes' markers (cell: index of the cell's first node, -1 none):
+ * markers in cell order are summed over each run of one cell first, so that
+ * HBM sees at most four atomics per node and run of a wavefront.  With one per
+ * marker and node the atomics were all the time: 96 x 48 x 48 foil (0.3 M
+ * markers) 372 us, laser-foil 4.34 ms; now 20 and 248 us. */
+__device__ static inline void rho_run_add(double *rho, const Grid &g, long cell, double *v)
+{
+    int start, len;
+    bool head;
+    wave_run((int)cell, start, len, head);
+    run_sums<8>(v, start);
+    if (!run_tail(start, len) || cell < 0) return;
+    const long si = (long)g.GY * g.GZ, sj = g.GZ;
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+        unsafeAtomicAdd(rho + cell + (q >> 2) * si + ((q >> 1) & 1) * sj + (q & 1), v[q]);
+}
+
 int launch_keys64(hipStream_t s, const Markers64 &m, long n, const Grid &g, const TileView &tv,
                   int parity);
 /* The tile scan's word buffer (zeroed once at allocation) and launcher;

@@ -107,3 +107,44 @@ def test_fused_runs_with_fewer_workgroups_than_tiles(prec, tol):
     assert alone.marker_count() == runs[0].marker_count() == thin.size
     for r in [alone] + runs:
         r.close()
+
+
+@pytest.mark.parametrize("prec", [ma.FP64, ma.FP32_SPLIT])
+@pytest.mark.parametrize("count", [1, 63, 64, 65, 700])
+def test_charge_density_by_runs(count, prec):
+    """A wavefront's markers are summed by runs of one cell: runs that end at,
+    before and past a row of 16 lanes, a wavefront and a workgroup (markers in
+    three cells), against the CIC sum in numpy."""
+    n, h = (9, 10, 11), (0.1, 0.2, 0.05)
+    rng = np.random.default_rng(count)
+    M = np.zeros(count, dtype=ma.MARKER_DTYPE)
+    c0 = np.array([(3, 4, 5), (3, 4, 6), (6, 3, 2)])[np.arange(count) * 3 // count]
+    for a, c in enumerate("xyz"):
+        M[c] = (c0[:, a] + rng.uniform(0.01, 0.99, count)) * h[a]
+    M["rho"] = rng.uniform(-1, 1, count).astype(np.float32)
+    M["qDivM"], M["id"] = -1.0, np.arange(1, count + 1)
+    r = ma.Run(n, h, tuple(a * b for a, b in zip(n, h)), 0.01, [ma.BC_OPEN] * 6, 0.0,
+               precision=prec, max_markers=count)
+    z = np.zeros(3 * r.nodes)
+    r.set_fields(z, z)
+    r.load_markers(M)
+    r.init()
+    # nodes [0, n]: the fold at the walls mirrors inner nodes onto the ghosts (plasma_rho.c:23-96)
+    own = (slice(2, -2),) * 3
+    got = r.rho().reshape([v + 5 for v in n])[own]
+    P = r.markers()
+    assert P.size == count
+    want = np.zeros([v + 5 for v in n])
+    s = [P[c].astype(float) / h[a] for a, c in enumerate("xyz")]
+    i = [np.floor(v).astype(int) for v in s]
+    f = [v - k for v, k in zip(s, i)]
+    for d in np.ndindex(2, 2, 2):
+        w = P["rho"].astype(float)
+        for a in range(3):
+            w = w * (f[a] if d[a] else 1 - f[a])
+        np.add.at(want, tuple(i[a] + 2 + d[a] for a in range(3)), w)
+    want = want[own]
+    # a sum of `count` terms, and positions to a few units in the last place of s < 12
+    bar = (count + 200) * 2.0 ** -53 * np.abs(P["rho"]).sum()
+    assert np.abs(want).max() > 0 and np.abs(got - want).max() <= bar
+    r.close()
