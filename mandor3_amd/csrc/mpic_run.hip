@@ -143,10 +143,11 @@ struct mpic_run {
     std::vector<Laser> lasers;
     PushConsts    pc;
     double       *dacc;       /* device scratch: [5..6] gauss */
-    double       *henergy;    /* pinned: em_energy partial sums, 2 per workgroup */
-    double       *hacc;       /* pinned host mirror */
+    double       *hpin;       /* one pinned allocation: hkin, hacc, dring, henergy */
+    double       *henergy;    /* em_energy partial sums, 2 per workgroup */
+    double       *hacc;       /* host mirror of dacc */
     double       *dkin;       /* the push's kinetic sums: KIN_SLOTS partial sums */
-    double       *hkin;       /* pinned: mpic_temperature's copy of the sums */
+    double       *hkin;       /* mpic_temperature's copy of the sums */
     unsigned     *derr;       /* device error flags (bit 0: marker off the grid, bit 1: a
                                  tile scan's wait for an earlier workgroup ran out) */
     int           stage;
@@ -593,12 +594,18 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     }
     r->n = 0;
     MPIC_CHECK(hipMalloc(&r->dacc, sizeof(double) * 8));
-    MPIC_CHECK(hipHostMalloc(&r->hacc, sizeof(double) * 8, hipHostMallocDefault));
-    MPIC_CHECK(hipHostMalloc(&r->henergy, sizeof(double) * 2 * energy_blocks(r->g),
-                             hipHostMallocDefault));
+    {
+        /* what kernels store for the host, in one allocation (each costs mpic_create
+         * as much as several device ones) */
+        const long nk = KIN_SLOTS * KIN_STRIDE, nr = 5 * DIAG_RING;
+        MPIC_CHECK(hipHostMalloc(&r->hpin, sizeof(double) * (nk + 8 + nr + 2 * energy_blocks(r->g)),
+                                 hipHostMallocDefault));
+        r->hkin = r->hpin;
+        r->hacc = r->hkin + nk;
+        r->dring = r->hacc + 8;
+        r->henergy = r->dring + nr;
+    }
     MPIC_CHECK(hipMalloc(&r->dkin, sizeof(double) * KIN_SLOTS * KIN_STRIDE));
-    MPIC_CHECK(hipHostMalloc(&r->hkin, sizeof(double) * KIN_SLOTS * KIN_STRIDE,
-                             hipHostMallocDefault));
     MPIC_CHECK(hipMemsetAsync(r->dkin, 0, sizeof(double) * KIN_SLOTS * KIN_STRIDE, r->stream));
     MPIC_CHECK(hipMalloc(&r->derr, sizeof(unsigned)));
     MPIC_CHECK(hipMemsetAsync(r->derr, 0, sizeof(unsigned), r->stream));
@@ -614,7 +621,6 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     }
     r->nparts = h_full_blocks(g, cfg->precision == MPIC_FP32_SPLIT);
     MPIC_CHECK(hipMalloc(&r->dpart, sizeof(double) * 2 * r->nparts));
-    MPIC_CHECK(hipHostMalloc(&r->dring, sizeof(double) * 5 * DIAG_RING, hipHostMallocDefault));
     r->ring_step.assign(DIAG_RING, -1);
     r->ring_time.assign(DIAG_RING, 0.0);
     cap_geometry(cfg->n, cfg->bc, kUpdH, kFlH, r->cH);
@@ -674,10 +680,8 @@ extern "C" int mpic_destroy(mpic_run_t *r)
     hipFree(r->tj);
     hipFree(r->dacc);
     hipFree(r->dkin);
-    if (r->hkin) hipHostFree(r->hkin);
+    if (r->hpin) hipHostFree(r->hpin);
     hipFree(r->derr);
-    if (r->hacc) hipHostFree(r->hacc);
-    if (r->henergy) hipHostFree(r->henergy);
     for (double *b : r->murbuf) hipFree(b);
     for (Laser &l : r->lasers) hipFree(l.dmap);
     for (hipEvent_t e : r->evpool) hipEventDestroy(e);
@@ -688,7 +692,6 @@ extern "C" int mpic_destroy(mpic_run_t *r)
     hipFree(r->dstep);
     hipFree(r->djr);
     hipFree(r->dpart);
-    if (r->dring) hipHostFree(r->dring);
     hipFree(r->dprobe);
     if (r->hsample) hipHostFree(r->hsample);
     hipFree(r->spot.dprof);
