@@ -50,7 +50,7 @@ def parse():
     p.add_argument("--no-cpu", action="store_true")
     p.add_argument("--autotune", action="store_true",
                    help="pick the FP32 push's launch shape with mpic_autotune before the timed "
-                        "steps (the default shape is one wavefront per tile, 16 workgroups per "
+                        "steps (the default shape is four wavefronts per tile, 4 to 16 workgroups per "
                         "CU)")
     p.add_argument("--cpu-seconds", type=float, default=10.0,
                    help="CPU baseline: seconds of oracle steps per core")
@@ -127,7 +127,13 @@ def measured_traffic(kernel, workload):
 
 
 PUSH32_KERNEL = "k_one_w<Push32ArgsW<%d> >"     # the FP32 push as the kernel trace names it
-PUSH64_KERNEL = "k_one_w<Push64TArgs>"
+PUSH64_KERNEL = "k_one_w<Push64TArgsW<4> >"
+
+
+def default_wavefronts(n):
+    """The FP32 push's wavefronts per workgroup by mpic_create's rule: 8 on a
+    box of at most two 4^3-cell tiles per CU (256 CUs), else 4."""
+    return 8 if int(np.prod([(v + 3) // 4 for v in n])) <= 512 else 4
 
 
 def run_gpu(ma, wl, precision, steps, warmup, autotune=False):
@@ -172,7 +178,8 @@ def run_gpu(ma, wl, precision, steps, warmup, autotune=False):
             "launch_shape": ({"workgroups": tuned[0], "wavefronts_per_workgroup": tuned[1],
                               "markers_per_item": tuned[2], "picked_by": "mpic_autotune"}
                              if tuned is not None else
-                             {"workgroups": "16 per CU", "wavefronts_per_workgroup": 1,
+                             {"workgroups": "one per 512 markers, 4 to 16 per CU",
+                              "wavefronts_per_workgroup": default_wavefronts(wl["n"]),
                               "markers_per_item": 0, "picked_by": "default"}
                              if precision == "fp32" else None),
             "last_diag": [float(v) for v in hist[-1]]}
@@ -414,9 +421,9 @@ def main_large(a):
                    "cell_updates_per_s": int(np.prod(wl["n"])) * a.steps / wall,
                    "push_kernel_ms": avg_push, "deposit_gather_ms": dep_ms / a.steps,
                    "rest_of_step_ms": rest_ms / a.steps, "setup_s": t1 - t0},
-        "roofline": {"bound": "hbm", "kernel": PUSH32_KERNEL % 1, "achieved": gbs,
+        "roofline": {"bound": "hbm", "kernel": PUSH32_KERNEL % 4, "achieved": gbs,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS,
-                     "traffic": measured_traffic(PUSH32_KERNEL % 1, wl["name"])},
+                     "traffic": measured_traffic(PUSH32_KERNEL % 4, wl["name"])},
         "checks": {"sort_counts_sum_to_live": counts_ok,
                    "markers_only_removed": bool(live_end <= live)}}))
 

@@ -606,10 +606,10 @@ int launch_h_update(hipStream_t s, const FieldsT<T> &f, const Grid &g, const Box
  * place, a boundary node that a wall copies from another one is computed
  * from that one's inputs, so the walls on H need no launch of their own.
  *
- * Laser-foil (256 x 128 x 128), J clear included: 47 us FP32, 87 us FP64,
+ * Laser-foil (256 x 128 x 128), J clear included: 50 us FP32, 87 us FP64,
  * against 105 and 167 us for cap update, two wall launches and two H passes
  * (36 B moved per node in FP32 instead of 60, four dependent launches fewer);
- * HBM-bound, 165 MB at 4.0 TB/s in FP32.  32^3 box: 6.7 us against 29. */
+ * HBM-bound, 251 MB moved at 5.0 TB/s in FP32.  32^3 box: 6.7 us against 29. */
 template <class T> struct HFullArgs {
     FieldsT<T>    f;           /* H: H^{n-1/2}, Hc: H^{n+1/2}, Ec: H^n */
     Grid          g;

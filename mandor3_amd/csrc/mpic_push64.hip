@@ -676,9 +676,9 @@ __device__ static inline void first_run_add(double *lj, First64 &fs)
  * cell key, to the output buffer at its position in the order, and the
  * per-cell counts of the new positions are kept for the next sort.
  *
- * Laser-foil (8.57 M markers) 600 -> 336 us, 3.3 TB/s of the 128 B per marker
- * against 4.8 TB/s of a plain copy; 64^3 full box 469 -> 251 us, 64^3 foil
- * 98 -> 43, 32^3 box 59 -> 45.  The 600 us were gathers from L2 with one batch
+ * Laser-foil (8.57 M markers) 600 -> 327 us, 3.4 TB/s of the 128 B per marker
+ * against 4.8 TB/s of a plain copy; 64^3 full box 469 -> 246 us, 64^3 foil
+ * 98 -> 39, 32^3 box 59 -> 39.  The 600 us were gathers from L2 with one batch
  * in flight, 31 IEEE divisions per marker of which 27 had a divisor known
  * before (h, 12, tau h h) and a branch per number of face crossings, each
  * with its own segment code.  Two wavefronts per SIMD (231 VGPRs) measured
