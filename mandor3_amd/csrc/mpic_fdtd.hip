@@ -606,10 +606,11 @@ int launch_h_update(hipStream_t s, const FieldsT<T> &f, const Grid &g, const Box
  * place, a boundary node that a wall copies from another one is computed
  * from that one's inputs, so the walls on H need no launch of their own.
  *
- * Laser-foil (256 x 128 x 128), J clear included: 50 us FP32, 87 us FP64,
+ * Laser-foil (256 x 128 x 128), J clear included: 40 us FP32, 76 us FP64,
  * against 105 and 167 us for cap update, two wall launches and two H passes
  * (36 B moved per node in FP32 instead of 60, four dependent launches fewer);
- * HBM-bound, 251 MB moved at 5.0 TB/s in FP32.  32^3 box: 6.7 us against 29. */
+ * HBM-bound.  The z walls' nodes are done by the rows' own threads (50 and 87
+ * us with edge workgroups reading those rows again, 251 MB moved in FP32).  32^3 box: 6.7 us against 29. */
 template <class T> struct HFullArgs {
     FieldsT<T>    f;           /* H: H^{n-1/2}, Hc: H^{n+1/2}, Ec: H^n */
     Grid          g;
@@ -619,6 +620,8 @@ template <class T> struct HFullArgs {
     LaserPlane    lp;          /* a laser's H plane added to H^{n+1/2} (on = 0: none) */
     const int    *xr;          /* planes where H^n is wanted */
     int           mir[3];      /* the max wall of the axis is a mirror: its normal H is zero */
+    int           z0, z1;      /* the z walls whose nodes (k = 0, k = n+1) are the rows' own:
+                                * 1 mirror, 2 Mur; 0 periodic, left to the edge workgroups */
 };
 
 /* Sum over the workgroup of (we, wb), stored as part[0..1]; every thread of
@@ -667,7 +670,7 @@ __device__ static inline void energy_terms(const Grid &g, int i, int j, int k, T
     if (i1 && j1 && k0) wb = __builtin_fma((double)hz, (double)hz, wb);
 }
 
-/* Nodes [1, n]^3. */
+/* Nodes [1, n]^3, and the rows' own nodes at k = 0 and n+1 (z0, z1). */
 template <class T>
 __device__ static inline void h_full(const HFullArgs<T> &A, const VBlock &b, const VBlock &gd,
                                      double &we, double &wb)
@@ -719,6 +722,41 @@ __device__ static inline void h_full(const HFullArgs<T> &A, const VBlock &b, con
         if (k >= 1 && k <= g.n[2])
             energy_terms<T>(g, i, j, k, ex[e], ey[e], ez[e], ax[e], ay[e], az[e], we, wb);
     }
+    /* a z wall that is not periodic copies from the row's own first or last
+     * node, so that node is done here, where its cache line is (see h_edge for
+     * what a wall leaves) */
+    const int kn = g.n[2] - k0;               /* node n's place in the group */
+    if (A.z1 && kn < V) {
+        T fx = bx[0], fy = by[0];
+#pragma unroll
+        for (int e = 1; e < V; ++e) {
+            fx = e == kn ? bx[e] : fx;
+            fy = e == kn ? by[e] : fy;
+        }
+        const long q = o + kn + 1;
+        const T ox = f.H[0][q], oy = f.H[1][q];
+        f.Hc[0][q] = fx;
+        f.Hc[1][q] = fy;
+        if (want) {
+            f.Ec[0][q] = (T)0.5 * (ox + fx);
+            f.Ec[1][q] = (T)0.5 * (oy + fy);
+        }
+    }
+    int klo = 1;
+    if (A.z0 && k0 <= 0) {
+        klo = 0;
+#pragma unroll
+        for (int e = 0; e + 1 < V; ++e)
+            if (k0 + e == 0) {
+                bx[e] = bx[e + 1];
+                by[e] = by[e + 1];
+                if (A.z0 == 1) bz[e] = 0;
+                ax[e] = (T)0.5 * (hx[e] + bx[e]);
+                ay[e] = (T)0.5 * (hy[e] + by[e]);
+                az[e] = (T)0.5 * (hz[e] + bz[e]);
+                energy_terms<T>(g, i, j, 0, ex[e], ey[e], ez[e], ax[e], ay[e], az[e], we, wb);
+            }
+    }
     laser_group<T>(A.lp, i, j, k0, V, by, bz);
     if (k0 >= 1 && k0 + V - 1 <= g.n[2]) {
         *(VT *)(f.Hc[0] + o) = bx;
@@ -733,7 +771,7 @@ __device__ static inline void h_full(const HFullArgs<T> &A, const VBlock &b, con
     }
 #pragma unroll
     for (int e = 0; e < V; ++e) {            /* a row's end: its other nodes are h_edge's */
-        if (k0 + e < 1 || k0 + e > g.n[2]) continue;
+        if (k0 + e < klo || k0 + e > g.n[2]) continue;
         f.Hc[0][o + e] = bx[e];
         f.Hc[1][o + e] = by[e];
         f.Hc[2][o + e] = bz[e];
@@ -745,7 +783,8 @@ __device__ static inline void h_full(const HFullArgs<T> &A, const VBlock &b, con
     }
 }
 
-/* The nodes of [0, n+1]^3 with a coordinate 0 or n+1.  Component c of such
+/* The nodes of [0, n+1]^3 with a coordinate 0 or n+1, but those of a z wall
+ * that is not periodic in rows (i, j) of [1, n] (h_full's).  Component c of such
  * a node is, per axis, the one the axis' walls leave there (in their order
  * x, y, z the copies compose axis by axis): the node's own update, a copy of
  * the update of node n, 1 (periodic) or of the neighbour inside (mirror, Mur;
@@ -839,15 +878,17 @@ static Span h_full_span(const Grid &g, int V)
     return V == 4 ? span_of<4>(1, 1, g.n[1], 1, g.n[2]) : span_of<2>(1, 1, g.n[1], 1, g.n[2]);
 }
 
-static BoxSet h_edge_set(const Grid &g)
+static BoxSet h_edge_set(const Grid &g, const int bc[6])
 {
     const int N[3] = {g.n[0], g.n[1], g.n[2]};
     BoxSet s;
-    s.n = 6;
+    s.n = 0;
     s.shell = -1;
     s.off[0] = 0;
-    for (int q = 0; q < 6; ++q) {
-        const int a = q >> 1, at = (q & 1) ? N[a] + 1 : 0;
+    for (int w = 0; w < 6; ++w) {
+        /* z walls that are not periodic: h_full's */
+        if ((w == 4 && bc[2] != MPIC_BC_PERIODIC) || (w == 5 && bc[5] != MPIC_BC_PERIODIC)) continue;
+        const int q = s.n++, a = w >> 1, at = (w & 1) ? N[a] + 1 : 0;
         long v = 1;
         for (int x = 0; x < 3; ++x) {
             s.b[q].lo[x] = x == a ? at : (x < a ? 1 : 0);
@@ -865,9 +906,9 @@ static unsigned h_edge_blocks(const BoxSet &s)
 }
 
 /* Workgroups of the one-pass H update: the energy partial sums it writes. */
-int h_full_blocks(const Grid &g, int fp32)
+int h_full_blocks(const Grid &g, const int bc[6], int fp32)
 {
-    const BoxSet s = h_edge_set(g);
+    const BoxSet s = h_edge_set(g, bc);
     return (int)(grid_span(h_full_span(g, fp32 ? Vec<float>::N : Vec<double>::N), g.n[0]) +
                  h_edge_blocks(s));
 }
@@ -1960,7 +2001,9 @@ int launch_h_full_jclear(hipStream_t s, const FieldsT<T> &f, const Grid &g, cons
     }
     a.lp = lp;
     a.xr = xr;
-    e.bs = h_edge_set(g);
+    a.z0 = bc[2] == MPIC_BC_PERIODIC ? 0 : bc[2] == MPIC_BC_MIRROR ? 1 : 2;
+    a.z1 = bc[5] == MPIC_BC_PERIODIC ? 0 : bc[5] == MPIC_BC_MIRROR ? 1 : 2;
+    e.bs = h_edge_set(g, bc);
     for (int q = 0; q < 6; ++q) e.bc[q] = bc[q];
     const unsigned na = grid_span(a.sp, g.n[0]), ne = h_edge_blocks(e.bs);
     HFullArgs<T> inner = a;

@@ -222,10 +222,10 @@ template <class T> int launch_energy(hipStream_t s, const FieldsT<T> &f, const G
 /* The kinetic sums' slots to pinned host memory. */
 int launch_kin_out(hipStream_t s, const double *kin, double *out);
 /* Loop-body diagnostics: the one-pass H update writes em_energy partial sums
- * (two doubles per workgroup, h_full_blocks(g, fp32) workgroups); the ring
+ * (two doubles per workgroup, h_full_blocks workgroups); the ring
  * row {W_E sum, W_M sum, WTx, WTy, WTz} of the device step counter's step
  * sums them. */
-int h_full_blocks(const Grid &g, int fp32);
+int h_full_blocks(const Grid &g, const int bc[6], int fp32);
 int launch_zero(hipStream_t s, double *p, long n);
 int launch_jclear(hipStream_t s, double *J, const Grid &g, double *kin, int *range,
                   const int *step, const int *xr, int full);

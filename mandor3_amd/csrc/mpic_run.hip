@@ -619,7 +619,7 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
         MPIC_CHECK(hipMalloc(&r->djr, sizeof(full)));
         MPIC_CHECK(hipMemcpy(r->djr, full, sizeof(full), hipMemcpyHostToDevice));
     }
-    r->nparts = h_full_blocks(g, cfg->precision == MPIC_FP32_SPLIT);
+    r->nparts = h_full_blocks(g, cfg->bc, cfg->precision == MPIC_FP32_SPLIT);
     MPIC_CHECK(hipMalloc(&r->dpart, sizeof(double) * 2 * r->nparts));
     r->ring_step.assign(DIAG_RING, -1);
     r->ring_time.assign(DIAG_RING, 0.0);
