@@ -610,7 +610,7 @@ int launch_h_update(hipStream_t s, const FieldsT<T> &f, const Grid &g, const Box
  * against 105 and 167 us for cap update, two wall launches and two H passes
  * (36 B moved per node in FP32 instead of 60, four dependent launches fewer);
  * HBM-bound.  The z walls' nodes are done by the rows' own threads (50 and 87
- * us with edge workgroups reading those rows again, 251 MB moved in FP32).  32^3 box: 6.7 us against 29. */
+ * us with edge workgroups reading those rows again; 251 -> 185 MB in FP32).  32^3 box: 6.7 us against 29. */
 template <class T> struct HFullArgs {
     FieldsT<T>    f;           /* H: H^{n-1/2}, Hc: H^{n+1/2}, Ec: H^n */
     Grid          g;
