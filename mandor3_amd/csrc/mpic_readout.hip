@@ -168,9 +168,12 @@ int Readout::launch(hipStream_t s, long first, long count, void *out) const
 }
 
 /* ---------------- pinned slots and helper threads ----------------
- * One set per process, shared by all runs (calls that overlap take turns):
- * two slots for each of at most HELPERS + 1 threads, allocated and started
- * when first needed, given back with the last run.  The threads wait between
+ * One set per process, shared by all runs: two slots for each of at most
+ * HELPERS + 1 threads, allocated and started when first needed, given back with
+ * the last run.  Calls that overlap take turns at packing and copying only: a
+ * call waits for the work on its run's stream before it takes its turn, so a
+ * read-out behind steps in flight holds up no other run's, and runs are counted
+ * under a lock of their own, so it holds up no mpic_create or mpic_destroy.  The threads wait between
  * calls and claim chunks one by one, so that one that wakes late (the
  * caller's process may keep every core busy) only finds less left to do;
  * threads started for each call and dealt fixed chunks took 2.5 ms instead of
@@ -188,8 +191,9 @@ struct Job {
 };
 
 struct Pool {
-    std::mutex call;                   /* one read-out at a time */
+    std::mutex life;                   /* guards runs; taken before call */
     int        runs = 0;
+    std::mutex call;                   /* one read-out at a time packs and copies */
     long       words = 0;              /* pinned words allocated */
     void      *mem = nullptr;
     std::mutex mu;                     /* guards what follows */
@@ -267,14 +271,15 @@ static void helper(int w)
 
 void readout_ref(void)
 {
-    std::lock_guard<std::mutex> lk(g_pool.call);
+    std::lock_guard<std::mutex> lk(g_pool.life);
     ++g_pool.runs;
 }
 
 void readout_unref(void)
 {
-    std::lock_guard<std::mutex> lk(g_pool.call);
+    std::lock_guard<std::mutex> l0(g_pool.life);
     if (--g_pool.runs > 0) return;
+    std::lock_guard<std::mutex> lk(g_pool.call);
     {
         std::lock_guard<std::mutex> l2(g_pool.mu);
         g_pool.stop = true;
@@ -302,6 +307,8 @@ static int slots_reserve(long words)
 
 int readout(const Readout *r, int n, int dev, hipStream_t s)
 {
+    /* steps in flight are waited for before the turn, not during it */
+    MPIC_CHECK(hipStreamSynchronize(s));
     std::lock_guard<std::mutex> lk(g_pool.call);
     long all = 0;
     for (int q = 0; q < n; ++q) all += r[q].words;
@@ -309,11 +316,13 @@ int readout(const Readout *r, int n, int dev, hipStream_t s)
         /* everything through one slot, one wait */
         TRY_READOUT(slots_reserve(SLOT_WORDS));
         char *at = (char *)g_pool.mem;
-        for (int q = 0; q < n; ++q) {
-            if (r[q].words) TRY_READOUT(r[q].launch(s, 0, r[q].words, at));
+        int rc = MPIC_OK;
+        for (int q = 0; q < n && rc == MPIC_OK; ++q) {
+            if (r[q].words) rc = r[q].launch(s, 0, r[q].words, at);
             at += 8 * r[q].words;
         }
-        MPIC_CHECK(hipStreamSynchronize(s));
+        MPIC_CHECK(hipStreamSynchronize(s));         /* nothing writes the slot any more */
+        if (rc != MPIC_OK) return rc;
         at = (char *)g_pool.mem;
         for (int q = 0; q < n; ++q) {
             if (r[q].words) memcpy(r[q].dst, at, 8 * r[q].words);
