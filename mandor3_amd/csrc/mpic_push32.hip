@@ -247,9 +247,10 @@ struct TilePos {
     bool edge;
 };
 
-__device__ static inline int clamp1(float f)
+/* Cells crossed along an axis by a move to offset x, at most one. */
+__device__ static inline float crossed(float x)
 {
-    return (int)__builtin_amdgcn_fmed3f(f, -1.0f, 1.0f);
+    return __builtin_amdgcn_fmed3f(floorf(x), -1.0f, 1.0f);
 }
 
 /* Push of one marker of tile-local cell (li,lj,lk) (cell (ci,cj,ck)):
@@ -305,12 +306,15 @@ __device__ static inline int push32_marker(MarkerRegs &out, const MarkerRegs &r,
     const float ig = rsq(1.0f + ux * ux + uy * uy + uz * uz);
     /* move in cell units from (ox,oy,oz) of cell (ci,cj,ck) */
     const float x2 = ox + ux * c.dtn[0] * ig, y2 = oy + uy * c.dtn[1] * ig, z2 = oz + uz * c.dtn[2] * ig;
-    const float flx = floorf(x2), fly = floorf(y2), flz = floorf(z2);
-    /* -1, 0 or 1: a marker moves less than a cell per step, mpic_create's
-     * Courant condition.  The clamp only keeps one that is not a number inside
-     * the block, so a segment needs no range check: a tile's markers start in
-     * block cells 1 to 4 and cross at most one face per axis. */
-    const int fx = clamp1(flx), fy = clamp1(fly), fz = clamp1(flz);
+    /* -1, 0 or 1 for the deposit: a marker moves less than a cell per step,
+     * mpic_create's Courant condition, so a segment needs no range check: a
+     * tile's markers start in block cells 1 to 4 and cross at most one face
+     * per axis.  In FP32 tau / h may round to 1 and x2 to 2 (or just below -1):
+     * the last segment then ends on the far face of the cell it is in, and the
+     * marker beyond it, in the cell of the true floor below.  A marker that is
+     * not a number stays inside the block too. */
+    const float cfx = crossed(x2), cfy = crossed(y2), cfz = crossed(z2);
+    const int fx = (int)cfx, fy = (int)cfy, fz = (int)cfz;
     const float wx = w * c.cj[0], wy = w * c.cj[1], wz = w * c.cj[2];
     /* Segments: from the start to the first face crossing (or the end),
      * then one per crossed face.  Crossing fractions ascend; an axis that is
@@ -341,9 +345,9 @@ __device__ static inline int push32_marker(MarkerRegs &out, const MarkerRegs &r,
         for (int s = 1; s <= nc; ++s) {
             const bool cx = axs == 0, cy = axs == 1, cz = axs == 2;
             p += cx ? fx * LJO(1, 0, 0, 0) : cy ? fy * LJO(0, 1, 0, 0) : fz * LJO(0, 0, 1, 0);
-            sx += cx ? flx : 0.0f;
-            sy += cy ? fly : 0.0f;
-            sz += cz ? flz : 0.0f;
+            sx += cx ? cfx : 0.0f;
+            sy += cy ? cfy : 0.0f;
+            sz += cz ? cfz : 0.0f;
             a0 = a1;
             x0 = x1;
             a1 = a2;
@@ -360,7 +364,8 @@ __device__ static inline int push32_marker(MarkerRegs &out, const MarkerRegs &r,
         }
     }
     /* new cell and offset, then the walls */
-    int ni = ci + fx, nj = cj + fy, nk = ck + fz;
+    const float flx = floorf(x2), fly = floorf(y2), flz = floorf(z2);
+    int ni = ci + (int)flx, nj = cj + (int)fly, nk = ck + (int)flz;
     float nx = x2 - flx, ny = y2 - fly, nz = z2 - flz;
     if (nx >= 1.0f) { nx = 0.0f; ++ni; }
     if (ny >= 1.0f) { ny = 0.0f; ++nj; }
