@@ -152,17 +152,36 @@ __device__ static inline void cic_weights(double sx, double sy, double sz, doubl
     v[7] = sx * (sy * (sz * val));
 }
 
+/* run_sums for values that need not be finite: a lane outside the run is not
+ * added at all (0 times infinity would reach the neighbouring runs). */
+template <int D> __device__ static inline double run_step(double x, bool in)
+{
+    const double y = row_shr<D>(x);
+    return in ? x + y : x;
+}
+
+template <int N> __device__ static inline void run_sums_any(double *v, int start)
+{
+    const int lane = threadIdx.x & 63;
+    const bool m1 = lane - 1 >= start, m2 = lane - 2 >= start, m4 = lane - 4 >= start,
+               m8 = lane - 8 >= start;
+#pragma unroll
+    for (int q = 0; q < N; ++q)
+        v[q] = run_step<8>(run_step<4>(run_step<2>(run_step<1>(v[q], m1), m2), m4), m8);
+}
+
 /* rho += the lanes' markers (cell: index of the cell's first node, -1 none):
  * markers in cell order are summed over each run of one cell first, so that
  * HBM sees at most four atomics per node and run of a wavefront.  With one per
  * marker and node the atomics were all the time: 96 x 48 x 48 foil (0.3 M
- * markers) 372 us, laser-foil 4.34 ms; now 20 and 248 us. */
+ * markers) 372 us, laser-foil 4.34 ms; now 20 and 248 us.  A marker whose
+ * charge is not finite leaves the other cells' sums alone. */
 __device__ static inline void rho_run_add(double *rho, const Grid &g, long cell, double *v)
 {
     int start, len;
     bool head;
     wave_run((int)cell, start, len, head);
-    run_sums<8>(v, start);
+    run_sums_any<8>(v, start);
     if (!run_tail(start, len) || cell < 0) return;
     const long si = (long)g.GY * g.GZ, sj = g.GZ;
 #pragma unroll
