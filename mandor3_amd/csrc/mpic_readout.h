@@ -13,9 +13,13 @@ struct NodeBlock {
     int  lo, d[3], nc;
 };
 
-/* Markers of an order, as records of 'words' 8-byte words (8 or 7). */
+/* Markers of an order, as records of 'words' 8-byte words (8 or 7).  An entry
+ * of the order that names none of the buffer's first *extent records is not
+ * followed: its position goes to *bad (host memory, set to -1 by the caller). */
 struct MarkerBlock {
     const int *perm;
+    const int *extent;
+    long      *bad;
     int        words;
     int        nt[3];              /* FP32: tiles per axis, mesh steps, q/m per species */
     double     h[3];

@@ -88,6 +88,15 @@ __device__ static inline unsigned long long two_words(float lo, float hi)
     return (unsigned long long)__float_as_uint(hi) << 32 | __float_as_uint(lo);
 }
 
+/* The record at position u of the order, -1 (reported) if there is none. */
+__device__ static inline long order_entry(const MarkerBlock &b, long u)
+{
+    const int q = b.perm[u];
+    if (q >= 0 && q < *b.extent) return q;
+    *b.bad = u;
+    return -1;
+}
+
 __global__ void k_pack_markers32(MarkerBlock b, Markers32 m, long first, long count,
                                  unsigned long long *out)
 {
@@ -95,7 +104,11 @@ __global__ void k_pack_markers32(MarkerBlock b, Markers32 m, long first, long co
     if (t >= count) return;
     const long e = first + t, u = e / b.words;
     const int w = (int)(e - u * b.words);
-    const long q = b.perm[u];
+    const long q = order_entry(b, u);
+    if (q < 0) {
+        out[t] = 0;
+        return;
+    }
     if (w == 7) {
         out[t] = (unsigned)m.id[q];
         return;
@@ -124,7 +137,11 @@ __global__ void k_pack_markers64(MarkerBlock b, Markers64 m, long first, long co
     if (t >= count) return;
     const long e = first + t, u = e / b.words;
     const int w = (int)(e - u * b.words);
-    const long q = b.perm[u];
+    const long q = order_entry(b, u);
+    if (q < 0) {
+        out[t] = 0;
+        return;
+    }
     if (w == 7) {
         out[t] = (unsigned)m.id[q];
     } else if (w == 6) {

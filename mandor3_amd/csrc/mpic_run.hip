@@ -143,11 +143,12 @@ struct mpic_run {
     std::vector<Laser> lasers;
     PushConsts    pc;
     double       *dacc;       /* device scratch: [5..6] gauss */
-    double       *hpin;       /* one pinned allocation: hkin, hacc, dring, henergy */
+    double       *hpin;       /* one pinned allocation: hkin, hacc, hbad, dring, henergy */
     double       *henergy;    /* em_energy partial sums, 2 per workgroup */
     double       *hacc;       /* host mirror of dacc */
     double       *dkin;       /* the push's kinetic sums: KIN_SLOTS partial sums */
     double       *hkin;       /* mpic_temperature's copy of the sums */
+    long         *hbad;       /* position of an order entry that names no record, from a save */
     unsigned     *derr;       /* device error flags (bit 0: marker off the grid, bit 1: a
                                  tile scan's wait for an earlier workgroup ran out) */
     int           stage;
@@ -598,11 +599,12 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
         /* what kernels store for the host, in one allocation (each costs mpic_create
          * as much as several device ones) */
         const long nk = KIN_SLOTS * KIN_STRIDE, nr = 5 * DIAG_RING;
-        MPIC_CHECK(hipHostMalloc(&r->hpin, sizeof(double) * (nk + 8 + nr + 2 * energy_blocks(r->g)),
+        MPIC_CHECK(hipHostMalloc(&r->hpin, sizeof(double) * (nk + 10 + nr + 2 * energy_blocks(r->g)),
                                  hipHostMallocDefault));
         r->hkin = r->hpin;
         r->hacc = r->hkin + nk;
-        r->dring = r->hacc + 8;
+        r->hbad = (long *)(r->hacc + 8);
+        r->dring = r->hacc + 10;
         r->henergy = r->dring + nr;
     }
     MPIC_CHECK(hipMalloc(&r->dkin, sizeof(double) * KIN_SLOTS * KIN_STRIDE));
@@ -1040,6 +1042,8 @@ static int save_order(mpic_run *r, void *rec, long *n, int recsize, long N)
     q.words = N * (recsize / 8);
     q.dst = rec;
     q.markers.perm = r->tv.perm;
+    q.markers.extent = r->tv.nmark + (r->parity ^ 1);   /* records written to the buffer */
+    q.markers.bad = r->hbad;
     q.markers.words = recsize / 8;
     for (int a = 0; a < 3; ++a) {
         q.markers.nt[a] = r->tv.nt[a];
@@ -1048,7 +1052,13 @@ static int save_order(mpic_run *r, void *rec, long *n, int recsize, long N)
     for (int s = 0; s < 8; ++s) q.markers.qm[s] = r->qm[s];
     q.m32 = r->m32;
     q.m64 = r->m;
+    *r->hbad = -1;
     TRY(readout(&q, 1, r->dev, r->stream));
+    if (*(volatile long *)r->hbad >= 0) {
+        mpic_set_error("mpic_markers_save: entry %ld of the order of %ld markers names no record",
+                       *r->hbad, N);
+        return MPIC_ERR_STATE;
+    }
     *n = N;
     return MPIC_OK;
 }
