@@ -1622,8 +1622,9 @@ __global__ void __launch_bounds__(KIN_SLOTS) k_kin_out(const double4 *kin, doubl
 int launch_kin_out(hipStream_t s, const double *kin, double *out)
 {
     static_assert(KIN_STRIDE == 4, "one double4 per slot");
-    k_kin_out<<<1, KIN_SLOTS, 0, s>>>((const double4 *)kin, (double4 *)out);
-    MPIC_CHECK(hipGetLastError());
+    /* (its own status: an earlier call's error is not this one's) */
+    void *args[] = {(void *)&kin, (void *)&out};
+    MPIC_CHECK(hipLaunchKernel((const void *)k_kin_out, dim3(1), dim3(KIN_SLOTS), args, 0, s));
     return MPIC_OK;
 }
 

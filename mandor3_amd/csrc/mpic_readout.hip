@@ -23,6 +23,7 @@
 #include <memory>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "mpic_readout.h"
@@ -152,36 +153,32 @@ __global__ void k_pack_markers64(MarkerBlock b, Markers64 m, long first, long co
     }
 }
 
+/* A launch that returns its own status: hipGetLastError would also return (and
+ * take away) what a call of the caller's thread has left there. */
+template <class... A>
+static int start(hipStream_t s, unsigned blocks, void (*kernel)(A...), std::common_type_t<A>... a)
+{
+    void *args[] = {(void *)&a...};
+    MPIC_CHECK(hipLaunchKernel((const void *)kernel, dim3(blocks), dim3(TPB), args, 0, s));
+    return MPIC_OK;
+}
+
 int Readout::launch(hipStream_t s, long first, long count, void *out) const
 {
     const unsigned nb = nblk(count);
+    double *d = (double *)out;
+    unsigned long long *w = (unsigned long long *)out;
+    const float *f0 = (const float *)F[0], *f1 = (const float *)F[1], *f2 = (const float *)F[2];
+    const double *d0 = (const double *)F[0], *d1 = (const double *)F[1], *d2 = (const double *)F[2];
     switch (kind) {
-    case BLOCK32:
-        k_pack_block<float><<<nb, TPB, 0, s>>>(block, (const float *)F[0], (const float *)F[1],
-                                              (const float *)F[2], first, count, (double *)out);
-        break;
-    case BLOCK64:
-        k_pack_block<double><<<nb, TPB, 0, s>>>(block, (const double *)F[0], (const double *)F[1],
-                                               (const double *)F[2], first, count, (double *)out);
-        break;
-    case NODES32:
-        k_pack_nodes<float><<<nb, TPB, 0, s>>>(block.g, mean, (const float *)F[0], (const float *)F[1],
-                                              (const float *)F[2], first, count, (double *)out);
-        break;
-    case NODES64:
-        k_pack_nodes<double><<<nb, TPB, 0, s>>>(block.g, mean, (const double *)F[0],
-                                               (const double *)F[1], (const double *)F[2], first,
-                                               count, (double *)out);
-        break;
-    case MARKERS32:
-        k_pack_markers32<<<nb, TPB, 0, s>>>(markers, m32, first, count, (unsigned long long *)out);
-        break;
-    case MARKERS64:
-        k_pack_markers64<<<nb, TPB, 0, s>>>(markers, m64, first, count, (unsigned long long *)out);
-        break;
+    case BLOCK32: return start(s, nb, k_pack_block<float>, block, f0, f1, f2, first, count, d);
+    case BLOCK64: return start(s, nb, k_pack_block<double>, block, d0, d1, d2, first, count, d);
+    case NODES32: return start(s, nb, k_pack_nodes<float>, block.g, mean, f0, f1, f2, first, count, d);
+    case NODES64: return start(s, nb, k_pack_nodes<double>, block.g, mean, d0, d1, d2, first, count, d);
+    case MARKERS32: return start(s, nb, k_pack_markers32, markers, m32, first, count, w);
+    case MARKERS64: return start(s, nb, k_pack_markers64, markers, m64, first, count, w);
     }
-    MPIC_CHECK(hipGetLastError());
-    return MPIC_OK;
+    return MPIC_ERR_ARG;
 }
 
 /* ---------------- pinned slots and helper threads ----------------
