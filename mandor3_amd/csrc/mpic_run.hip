@@ -183,6 +183,7 @@ struct mpic_run {
                                  memory: a step's kernel writes its row, the host reads it */
     std::vector<long>   ring_step;  /* step whose row a slot holds (-1: none) */
     std::vector<double> ring_time;  /* Time at the start of that step */
+    int           created;    /* mpic_create has handed the run out */
     int           capturing;  /* step_body is being recorded into graphs, not run */
     double        vsp;        /* VSP convolution weight alpha (1: off) */
     long          topo;       /* bumped whenever the launch sequence of a step changes */
@@ -450,7 +451,6 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     MPIC_CHECK(hipSetDevice(cfg->device));
     TRY(scratch_setup(cfg->device));
     mpic_run *r = new mpic_run();
-    readout_ref();
     r->cfg = *cfg;
     r->dev = cfg->device;
     MPIC_CHECK(hipSetDevice(r->dev));
@@ -652,6 +652,8 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     r->stage = 0;
     r->vsp = 1.0;
     MPIC_CHECK(hipStreamSynchronize(r->stream));
+    readout_ref();               /* mpic_destroy's counterpart: only of runs handed out */
+    r->created = 1;
     *out = r;
     return MPIC_OK;
 }
@@ -707,7 +709,7 @@ extern "C" int mpic_destroy(mpic_run_t *r)
     for (int k = 0; k < 2; ++k)
         if (r->exec[k]) hipGraphExecDestroy(r->exec[k]);
     if (r->stream) hipStreamDestroy(r->stream);
-    readout_unref();
+    if (r->created) readout_unref();
     delete r;
     return MPIC_OK;
 }
