@@ -388,6 +388,16 @@ static int push32_item_markers(void)
     return v >= 64 ? v : 0;
 }
 
+/* Markers per work item of the FP64 push (0: one item per tile).  It adds its
+ * blocks to J by atomics, so a tile may also be cut there: on boxes of at most
+ * 64 tiles, where a wavefront's serial batches are the time (push in us without
+ * and with 512 markers per item: 12^3 box 21 / 14, 16^3 box, 64 tiles, 21 / 15;
+ * 20^3 box, 125 tiles, 22 / 26). */
+static int push64_item_markers(long ntiles)
+{
+    return ntiles <= 64 ? 512 : 0;
+}
+
 /* Work items of a run: at most one per tile plus one per chm markers. */
 static long items_capacity(int ntiles, long cap, int chm)
 {
@@ -404,10 +414,12 @@ extern "C" int mpic_footprint(const mpic_config_t *cfg, size_t *bytes)
     const size_t mk = (cfg->precision == MPIC_FP32_SPLIT) ? (4 + 7 * 4 + 4 + 4) : (6 * 8 + 2 * 4 + 4 + 4);
     const int fp32 = cfg->precision == MPIC_FP32_SPLIT;
     const long cap = cfg->max_markers > 0 ? cfg->max_markers : 1;
-    const size_t items = (size_t)items_capacity((int)tiles, cap, fp32 ? push32_item_markers() : 0);
+    const int chm = fp32 ? push32_item_markers() : push64_item_markers((long)tiles);
+    const size_t items = (size_t)items_capacity((int)tiles, cap, chm);
     *bytes = field_bytes(cfg->n, fp32) + 2 * sizeof(double) * cells +
              2 * (size_t)cap * mk + tiles * 64 * 3 * sizeof(int) + tiles * 9 * sizeof(int) +
-             items * sizeof(int4) + (fp32 ? items * TJB * sizeof(float) : 0);
+             items * sizeof(int4) + (fp32 ? items * TJB * sizeof(float) : 0) +
+             sizeof(double) * KIN_SLOTS * KIN_STRIDE;
     return MPIC_OK;
 }
 
@@ -536,12 +548,7 @@ extern "C" int mpic_create(const mpic_config_t *cfg, mpic_run_t **out)
     tv.perm = nullptr;
     if (r->tiled) MPIC_CHECK(hipMalloc(&tv.perm, sizeof(int) * r->cap));
     MPIC_CHECK(hipMalloc(&tv.active, sizeof(int) * 2 * tv.ntiles));
-    /* The FP64 push adds its blocks to J by atomics, so a tile may also be cut
-     * there: with fewer tiles than a quarter of the CUs, where a wavefront's
-     * serial batches are the time (push in us without and with 512 markers
-     * per item: 12^3 box 21 / 14, 16^3 box, 64 tiles, 21 / 15; 20^3 box,
-     * 125 tiles, 22 / 26). */
-    tv.chm = r->fp32 ? push32_item_markers() : (tv.ntiles <= 64 ? 512 : 0);
+    tv.chm = r->fp32 ? push32_item_markers() : push64_item_markers(tv.ntiles);
     r->items_cap = items_capacity(tv.ntiles, r->cap, tv.chm);
     MPIC_CHECK(hipMalloc(&tv.item, sizeof(int4) * r->items_cap));
     MPIC_CHECK(hipMalloc(&tv.titem, sizeof(int2) * 2 * tv.ntiles));
