@@ -2732,8 +2732,8 @@ extern "C" int mpic_autotune(mpic_run_t *r, int steps, int *chosen)
     if (!r->fp32 || !r->tiled) {
         if (chosen) {
             chosen[0] = r->tile_blocks;
-            chosen[1] = 1;
-            chosen[2] = 0;
+            chosen[1] = r->tiled ? (r->tile_waves == 8 ? 8 : 4) : 1;
+            chosen[2] = r->tiled ? r->tv.chm : 0;
         }
         return MPIC_OK;
     }
