@@ -255,9 +255,10 @@ int  mpic_marker_cells(mpic_run_t *run, int32_t *cells, long *n);
 /* Kernel timing of the last mpic_advance, from HIP events on the run's
  * stream (three per step: before the push, after it, after the deposit;
  * waits for those steps to finish): milliseconds, summed over the steps, in
- * the push kernel, in the rest of the deposit (the FP32 form's J gather; 0
- * for FP64) and in everything else of the step (from the deposit's end to
- * the next push, scaled to all the steps). */
+ * the push kernel, in the rest of the deposit (the FP32 form's J gather,
+ * timed in the last step, where it has a launch of its own, and scaled to all
+ * of them; 0 for FP64) and in everything else of the step (from the deposit's
+ * end to the next push, scaled to all the steps). */
 int  mpic_last_timing(mpic_run_t *run, double *push_ms, double *deposit_ms, double *rest_ms);
 
 #ifdef __cplusplus

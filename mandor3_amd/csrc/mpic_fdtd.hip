@@ -2098,7 +2098,8 @@ template <> struct KernelDef<DiagRingArgs> {
  *         [y, z walls]
  * in place of ten launches.  The two walls of an axis (7 cells or more)
  * touch disjoint node layers, and so do its two J folds, so each pair runs in
- * one launch whatever its kinds. */
+ * one launch whatever its kinds.  A step that times the J gather (after_gather)
+ * runs it by itself. */
 template <class T>
 int launch_after_push(hipStream_t s, const FieldsT<T> &f, const Grid &g, const AfterPush &p)
 {
@@ -2129,8 +2130,13 @@ int launch_after_push(hipStream_t s, const FieldsT<T> &f, const Grid &g, const A
     const unsigned nfx = gfx.x * gfx.y;
     if (sizeof(T) == 4) {
         const JGatherArgs jg = {p.jp, g, *p.tv, p.tj, p.parity};
-        TRY_LAUNCH(launch_three(s, ScanLeanArgs{sc}, gsc, cap, gcap, jg, dim3(p.gather_blocks)));
-        if (p.after_gather) MPIC_CHECK(hipEventRecord(p.after_gather, s));
+        if (p.after_gather) {
+            TRY_LAUNCH(launch_def(s, jg, (unsigned)p.gather_blocks));
+            MPIC_CHECK(hipEventRecord(p.after_gather, s));
+            TRY_LAUNCH(launch_pair(s, ScanLeanArgs{sc}, gsc, cap, gcap));
+        } else {
+            TRY_LAUNCH(launch_three(s, ScanLeanArgs{sc}, gsc, cap, gcap, jg, dim3(p.gather_blocks)));
+        }
         TRY_LAUNCH(launch_three(s, pair_of(ring, 1, fx, gfx), dim3(1 + nfx), jx, gjx, rk, grk));
         return launch_pair(s, fp, dim3(planes), jp, gjp);
     }

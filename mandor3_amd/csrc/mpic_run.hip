@@ -172,6 +172,8 @@ struct mpic_run {
     hipGraphExec_t exec[2];   /* one step from each of the two marker-buffer parities */
     int           exec_phase;      /* the run's phase when exec[0] was captured */
     int           ev_steps;   /* timed steps of the last mpic_advance */
+    int           ev_alone;   /* FP32: the last ev_alone of them ran the J gather in a launch of its own */
+    int           alone;      /* the step being launched is one of those */
     int          *dprobe;     /* probe nodes, 3 ints each */
     double       *hsample;    /* pinned: probe samples, 6 doubles each */
     int           nprobes;
@@ -2085,7 +2087,8 @@ static void mark_ring(mpic_run *r)
 }
 
 /* One step; with r->timed >= 0 its events (before the push, after it,
- * after the deposit: slots 1, 2, 3 of the step's five) are recorded. */
+ * after the deposit: slots 1, 2, 3 of the step's five) are recorded; FP32: the
+ * last only where the J gather has a launch of its own (r->alone). */
 static int step_body(mpic_run *r)
 {
     TRY(check_stage(r, 0));
@@ -2127,7 +2130,7 @@ static int step_body(mpic_run *r)
     ap.nbound = r->n;
     ap.tj = r->tj;
     ap.gather_blocks = r->gather_blocks;
-    ap.after_gather = r->timed >= 0 && r->fp32 ? r->evpool[5 * r->timed + 3] : nullptr;
+    ap.after_gather = r->alone ? r->evpool[5 * r->timed + 3] : nullptr;
     ap.part = r->dpart;
     ap.nparts = r->nparts;
     ap.kin = r->dkin;
@@ -2199,8 +2202,11 @@ extern "C" int mpic_step(mpic_run_t *r, double *diag)
     return MPIC_OK;
 }
 
-/* n steps with a timed event record per step (kernel timing). */
-static int advance_timed(mpic_run *r, int nsteps)
+/* n steps with a timed event record per step (kernel timing).  The J gather
+ * shares its launch with the next order's scan and the E caps, so it is timed
+ * in a launch of its own in the last 'alone' steps (FP32 form; about 4 us more
+ * than the shared launch each). */
+static int advance_timed(mpic_run *r, int nsteps, int alone)
 {
     while ((int)r->evpool.size() < 5 * nsteps) {
         hipEvent_t e;
@@ -2209,8 +2215,14 @@ static int advance_timed(mpic_run *r, int nsteps)
         MPIC_CHECK(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
         r->evpool.push_back(e);
     }
-    for (int s = 0; s < nsteps; ++s) TRY(step_async(r, s));
+    for (int s = 0; s < nsteps; ++s) {
+        r->alone = r->fp32 && s >= nsteps - alone;
+        const int rc = step_async(r, s);
+        r->alone = 0;
+        TRY(rc);
+    }
     r->ev_steps = nsteps;
+    r->ev_alone = alone < nsteps ? alone : nsteps;
     return MPIC_OK;
 }
 
@@ -2305,7 +2317,7 @@ extern "C" int mpic_advance(mpic_run_t *r, int nsteps)
 {
     if (!r || nsteps < 0) return MPIC_ERR_ARG;
     MPIC_CHECK(hipSetDevice(r->dev));
-    if (!r->use_graphs) return advance_timed(r, nsteps);
+    if (!r->use_graphs) return advance_timed(r, nsteps, 1);
     if (!r->inited || r->stage != 0) {
         mpic_set_error("stage order violated: run is at stage %d, a replayed step starts at "
                        "stage 0", r->stage);
@@ -2749,7 +2761,7 @@ extern "C" int mpic_autotune(mpic_run_t *r, int steps, int *chosen)
         /* the item list of the current order follows the item size */
         r->tv.chm = chm;
         TRY(sort_pass(r, 1));
-        TRY(advance_timed(r, 1));          /* untimed: first launches of the new lists */
+        TRY(advance_timed(r, 1, 1));       /* untimed: first launches of the new lists */
         for (int wi = 0; wi < 3; ++wi) {
             const int w = wavess[wi];
             for (int per_cu = 4; per_cu <= 64; per_cu *= 2) {
@@ -2757,7 +2769,7 @@ extern "C" int mpic_autotune(mpic_run_t *r, int steps, int *chosen)
                 if (nb > r->items_cap) nb = (int)r->items_cap;
                 r->tile_blocks = nb;
                 r->tile_waves = w;
-                TRY(advance_timed(r, steps));
+                TRY(advance_timed(r, steps, steps));
                 double p, d, rest;
                 TRY(mpic_last_timing(r, &p, &d, &rest));
                 if (verbose && verbose[0] == '1')
@@ -2823,17 +2835,24 @@ extern "C" int mpic_last_timing(mpic_run_t *r, double *push_ms, double *deposit_
     if (n > 0) {
         MPIC_CHECK(hipSetDevice(r->dev));
         MPIC_CHECK(hipEventSynchronize(r->evpool[5 * (n - 1) + 3]));
+        const int first = r->fp32 ? n - r->ev_alone : 0;    /* steps with the deposit's end marked */
+        double gather = 0;
+        for (int s = first; s < n; ++s) {
+            float c;
+            MPIC_CHECK(hipEventElapsedTime(&c, r->evpool[5 * s + 2], r->evpool[5 * s + 3]));
+            gather += c;
+        }
+        gather /= n - first;
+        t[1] = n * gather;
         for (int s = 0; s < n; ++s) {
             const hipEvent_t *e = &r->evpool[5 * s];
-            float b, c;
+            float b;
             MPIC_CHECK(hipEventElapsedTime(&b, e[1], e[2]));
-            MPIC_CHECK(hipEventElapsedTime(&c, e[2], e[3]));
             t[0] += b;
-            t[1] += c;
             if (s + 1 < n) {              /* from this step's deposit end to the next push */
                 float a;
-                MPIC_CHECK(hipEventElapsedTime(&a, e[3], r->evpool[5 * (s + 1) + 1]));
-                t[2] += a;
+                MPIC_CHECK(hipEventElapsedTime(&a, s < first ? e[2] : e[3], r->evpool[5 * (s + 1) + 1]));
+                t[2] += s < first ? a - gather : a;
             }
         }
         if (n > 1) t[2] *= (double)n / (n - 1);

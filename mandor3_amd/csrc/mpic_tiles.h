@@ -230,7 +230,7 @@ struct AfterPush {
     long                nbound;
     const float        *tj;            /* FP32: the J blocks */
     int                 gather_blocks;
-    hipEvent_t          after_gather;  /* recorded after the J gather (null: not timed) */
+    hipEvent_t          after_gather;  /* FP32: the J gather alone, then this (null: not timed) */
     /* the diagnostics ring's row of this step */
     const double       *part, *kin;
     int                 nparts;
