@@ -182,16 +182,22 @@ int Readout::launch(hipStream_t s, long first, long count, void *out) const
 }
 
 /* ---------------- pinned slots and helper threads ----------------
- * One set per process, shared by all runs: two slots for each of at most
- * HELPERS + 1 threads, allocated and started when first needed, given back with
- * the last run.  Calls that overlap take turns at packing and copying only: a
- * call waits for the work on its run's stream before it takes its turn, so a
- * read-out behind steps in flight holds up no other run's, and runs are counted
- * under a lock of their own, so it holds up no mpic_create or mpic_destroy.  The threads wait between
- * calls and claim chunks one by one, so that one that wakes late (the
- * caller's process may keep every core busy) only finds less left to do;
- * threads started for each call and dealt fixed chunks took 2.5 ms instead of
- * 0.5 for 13 MB beside spinning OpenMP threads. */
+ * Two sets per process, shared by all runs: two slots for each of at most
+ * HELPERS + 1 threads, and two for a caller without helpers, allocated and
+ * started when first needed, given back with the last run.  A call takes the
+ * first set if it is free and packs behind whatever is in flight on its run's
+ * stream.  One that finds it taken, perhaps by a call that waits for a thousand
+ * steps, waits for its own stream, then takes the first set if it is free by
+ * now and the second if not: that one is never held while steps run.  So a
+ * read-out behind queued steps holds up no other run's, and since runs are
+ * counted under a lock of their own, no mpic_create or mpic_destroy.  (With
+ * every call waiting for its stream first, a read-out behind steps took 20 to
+ * 45 us more: its launches were no longer queued while the steps ran.)
+ *
+ * The threads wait between calls and claim chunks one by one, so that one that
+ * wakes late (the caller's process may keep every core busy) only finds less
+ * left to do; threads started for each call and dealt fixed chunks took 2.5 ms
+ * instead of 0.5 for 13 MB beside spinning OpenMP threads. */
 #define SLOT_WORDS (1L << 17)          /* 1 MiB */
 #define HELPERS 7
 
@@ -204,13 +210,17 @@ struct Job {
     std::atomic<int>  rc{MPIC_OK};
 };
 
-struct Pool {
-    std::mutex life;                   /* guards runs; taken before call */
-    int        runs = 0;
-    std::mutex call;                   /* one read-out at a time packs and copies */
+struct Slots {
+    std::mutex use;                    /* held by the call that packs through them */
     long       words = 0;              /* pinned words allocated */
     void      *mem = nullptr;
-    std::mutex mu;                     /* guards what follows */
+};
+
+struct Pool {
+    std::mutex life;                   /* guards runs; taken before the sets */
+    int        runs = 0;
+    Slots      set[2];                 /* with the helpers; for the caller alone */
+    std::mutex mu;                     /* guards what follows, the helpers' */
     std::condition_variable wake, finished;
     std::vector<std::thread> threads;
     std::shared_ptr<Job> job;
@@ -279,7 +289,7 @@ static void helper(int w)
             seen = g_pool.serial;
             job = g_pool.job;
         }
-        work(*job, (char *)g_pool.mem + 8 * SLOT_WORDS * 2 * w);
+        work(*job, (char *)g_pool.set[0].mem + 8 * SLOT_WORDS * 2 * w);
     }
 }
 
@@ -293,7 +303,6 @@ void readout_unref(void)
 {
     std::lock_guard<std::mutex> l0(g_pool.life);
     if (--g_pool.runs > 0) return;
-    std::lock_guard<std::mutex> lk(g_pool.call);
     {
         std::lock_guard<std::mutex> l2(g_pool.mu);
         g_pool.stop = true;
@@ -302,34 +311,43 @@ void readout_unref(void)
     for (std::thread &t : g_pool.threads) t.join();
     g_pool.threads.clear();
     g_pool.stop = false;
-    if (g_pool.mem) hipHostFree(g_pool.mem);
-    g_pool.mem = nullptr;
-    g_pool.words = 0;
+    for (Slots &S : g_pool.set) {
+        if (S.mem) hipHostFree(S.mem);
+        S.mem = nullptr;
+        S.words = 0;
+    }
 }
 
 /* At least 'words' pinned words; only grows while no helper runs. */
-static int slots_reserve(long words)
+static int slots_reserve(Slots &S, long words)
 {
-    if (words <= g_pool.words) return MPIC_OK;
-    if (g_pool.mem) hipHostFree(g_pool.mem);
-    g_pool.mem = nullptr;
-    g_pool.words = 0;
-    MPIC_CHECK(hipHostMalloc(&g_pool.mem, 8 * words, hipHostMallocPortable));
-    g_pool.words = words;
+    if (words <= S.words) return MPIC_OK;
+    if (S.mem) hipHostFree(S.mem);
+    S.mem = nullptr;
+    S.words = 0;
+    MPIC_CHECK(hipHostMalloc(&S.mem, 8 * words, hipHostMallocPortable));
+    S.words = words;
     return MPIC_OK;
 }
 
 int readout(const Readout *r, int n, int dev, hipStream_t s)
 {
-    /* steps in flight are waited for before the turn, not during it */
-    MPIC_CHECK(hipStreamSynchronize(s));
-    std::lock_guard<std::mutex> lk(g_pool.call);
+    int k = 0;
+    std::unique_lock<std::mutex> lk(g_pool.set[0].use, std::try_to_lock);
+    if (!lk) {
+        MPIC_CHECK(hipStreamSynchronize(s));
+        if (!lk.try_lock()) {
+            k = 1;
+            lk = std::unique_lock<std::mutex>(g_pool.set[1].use);
+        }
+    }
+    Slots &S = g_pool.set[k];
     long all = 0;
     for (int q = 0; q < n; ++q) all += r[q].words;
     if (all <= SLOT_WORDS) {
         /* everything through one slot, one wait */
-        TRY_READOUT(slots_reserve(SLOT_WORDS));
-        char *at = (char *)g_pool.mem;
+        TRY_READOUT(slots_reserve(S, SLOT_WORDS));
+        char *at = (char *)S.mem;
         int rc = MPIC_OK;
         for (int q = 0; q < n && rc == MPIC_OK; ++q) {
             if (r[q].words) rc = r[q].launch(s, 0, r[q].words, at);
@@ -337,14 +355,15 @@ int readout(const Readout *r, int n, int dev, hipStream_t s)
         }
         MPIC_CHECK(hipStreamSynchronize(s));         /* nothing writes the slot any more */
         if (rc != MPIC_OK) return rc;
-        at = (char *)g_pool.mem;
+        at = (char *)S.mem;
         for (int q = 0; q < n; ++q) {
             if (r[q].words) memcpy(r[q].dst, at, 8 * r[q].words);
             at += 8 * r[q].words;
         }
         return MPIC_OK;
     }
-    TRY_READOUT(slots_reserve(SLOT_WORDS * 2 * (HELPERS + 1)));
+    const int helpers = k == 0 ? HELPERS : 0;
+    TRY_READOUT(slots_reserve(S, SLOT_WORDS * 2 * (helpers + 1)));
     for (int q = 0; q < n; ++q) {
         const auto job = std::make_shared<Job>();
         job->r = r + q;
@@ -352,7 +371,7 @@ int readout(const Readout *r, int n, int dev, hipStream_t s)
         job->dev = dev;
         job->stream = s;
         if (!job->nchunks) continue;
-        while (g_pool.threads.size() < (size_t)std::min<long>(HELPERS, job->nchunks - 1)) {
+        while (g_pool.threads.size() < (size_t)std::min<long>(helpers, job->nchunks - 1)) {
             try {
                 const int w = (int)g_pool.threads.size() + 1;
                 g_pool.threads.emplace_back(helper, w);
@@ -360,14 +379,14 @@ int readout(const Readout *r, int n, int dev, hipStream_t s)
                 break;                              /* no more threads: fewer do */
             }
         }
-        {
+        if (helpers) {
             std::lock_guard<std::mutex> l2(g_pool.mu);
             g_pool.job = job;
             ++g_pool.serial;
         }
-        if (job->nchunks > 1) g_pool.wake.notify_all();
-        work(*job, (char *)g_pool.mem);
-        {
+        if (helpers && job->nchunks > 1) g_pool.wake.notify_all();
+        work(*job, (char *)S.mem);
+        if (helpers) {
             std::unique_lock<std::mutex> l2(g_pool.mu);
             g_pool.finished.wait(l2, [&] { return job->done == job->nchunks; });
             g_pool.job.reset();
