@@ -1047,10 +1047,11 @@ int launch_e_tauJ(hipStream_t s, const FieldsT<T> &f, const Grid &g, int *tick, 
 /* The E step of the loop body in one pass: the interior update of
  * em_EStep_start, the cap flush E = Ec and E -= tau J of em_EStep_finish,
  * node by node in that order, over nodes [-1, n+1]^3 (the J fold has run
- * before).  Per node the arithmetic is that of e_update then e_tauJ; the
- * loop body uses it where no source adds to E between the two (no laser, no
- * TFSF interface) in the FP64 form, and always in the FP32 split form,
- * whose sources then add after E -= tau J (a different rounding order). */
+ * before).  Per node the arithmetic is that of e_update then e_tauJ, with one
+ * laser's plane added between the two; the loop body uses it in the FP64 form
+ * where nothing else adds to E there (no TFSF interface, at most one laser),
+ * and always in the FP32 split form, whose other sources then add after
+ * E -= tau J (a different rounding order). */
 template <class T> struct EFusedArgs {
     FieldsT<T> f;
     Grid       g;
