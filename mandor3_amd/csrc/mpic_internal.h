@@ -9,7 +9,8 @@
  *            single index formula for every kernel.
  *   caps     Hc/Ec: H^{n+1/2} and E^{n+1} of the boundary layer, computed
  *            ahead of the interior exactly as the reference's boundary caps
- *            (source/core/em_caps.c:405-725), stored on the same padded grid.
+ *            (source/core/em_caps.c:405-725), stored on the same padded grid;
+ *            in the loop body H^{n+1/2} whole, and H^n before the E caps.
  *   markers  structure-of-arrays (FP64 plain form): x y z ux uy uz (double),
  *            w qm (float), id (int32).  A deleted marker has qm == 0.
  */
