@@ -39,10 +39,12 @@ def test_finished_run_beside_a_busy_one(n, monkeypatch):
     busy.node_fields(0)                   # (first uses: pinned slots, helper threads)
     want = done.fields()[0]
     assert np.abs(want).max() > 0
-    busy.advance(1)
-    t0 = time.time()
+    busy.advance(2)
     busy.sync()
-    step = time.time() - t0
+    t0 = time.time()
+    busy.advance(5)
+    busy.sync()
+    step = (time.time() - t0) / 5
     busy.advance(1 + int(1.5 / max(step, 1e-3)))      # 1.5 s of steps, or 1500 steps
     reader = threading.Thread(target=busy.node_fields, args=(0,))
     reader.start()
