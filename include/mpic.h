@@ -186,14 +186,15 @@ int  mpic_batch_advance(mpic_run_t *const *runs, int nruns, int nsteps);
 /* Picks the launch shape of the FP32 push -- markers per work item (a
  * tile's markers split into even items of at most 2048 or 1024, or one item
  * per tile), wavefronts per workgroup (1, 2 or 4 sharing one tile's staged
- * fields and J block; not the 8 that mpic_create gives a box of at most two
- * tiles per CU, which such a box is better left with) and workgroup count --
- * by timing 'steps' real steps per candidate (the steps advance the run; the
- * choice changes results only by the summation order of J).  chosen (may be
- * NULL) receives {workgroups, wavefronts per workgroup, markers per item (0:
- * one item per tile)}.  The work-item buffers may grow by up to an eighth of the marker buffers'
- * size.  Between steps only.  FP64 runs keep their shape, which chosen
- * receives (wavefronts per workgroup 4 or 8; untiled runs 1). */
+ * fields and J block; also 8, which mpic_create gives a box of at most two
+ * tiles per CU, if such a box holds 512 markers per tile) and workgroup count
+ * -- by timing 'steps' real steps per candidate (the steps advance the run;
+ * the choice changes results only by the summation order of J).  chosen (may
+ * be NULL) receives {workgroups, wavefronts per workgroup, markers per item
+ * (0: one item per tile)}.  The work-item buffers may grow by up to an eighth
+ * of the marker buffers' size.  Between steps only.  FP64 runs keep their
+ * shape, which chosen receives (wavefronts per workgroup 4 or 8; untiled runs
+ * 1). */
 int  mpic_autotune(mpic_run_t *run, int steps, int *chosen);
 int  mpic_sync(mpic_run_t *run);
 double mpic_time(mpic_run_t *run);

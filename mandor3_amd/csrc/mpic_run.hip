@@ -2750,7 +2750,12 @@ extern "C" int mpic_autotune(mpic_run_t *r, int steps, int *chosen)
         return MPIC_OK;
     }
     const int chms[3] = {0, 2048, 1024};
-    const int wavess[3] = {1, 2, 4};
+    const int wavess[4] = {1, 2, 4, 8};
+    /* eight wavefronts are the rule's choice on such boxes (see mpic_create) and
+     * faster there where each has a batch of its own: push in us with the best
+     * shape of 4 / 8 and 1024 markers per tile, 12^3 box 16.4 / 14.1; on larger
+     * boxes slower (64^3 full 127 / 138) */
+    const int nw = r->tv.ntiles <= 2 * r->ncu && r->n >= 8 * 64L * r->tv.ntiles ? 4 : 3;
     const char *verbose = getenv("MPIC_AUTOTUNE_VERBOSE");
     int best_nb = r->tile_blocks, best_w = r->tile_waves, best_chm = r->tv.chm;
     double best_ms = 1e300;
@@ -2762,7 +2767,7 @@ extern "C" int mpic_autotune(mpic_run_t *r, int steps, int *chosen)
         r->tv.chm = chm;
         TRY(sort_pass(r, 1));
         TRY(advance_timed(r, 1, 1));       /* untimed: first launches of the new lists */
-        for (int wi = 0; wi < 3; ++wi) {
+        for (int wi = 0; wi < nw; ++wi) {
             const int w = wavess[wi];
             for (int per_cu = 4; per_cu <= 64; per_cu *= 2) {
                 int nb = per_cu * r->ncu / w;
